@@ -227,6 +227,115 @@ std::array<int, 3> choose_blocks(const Strength &s, double theta, const std::vec
     return b;
 }
 
+// Index blocks and offsets of the one-workgroup tail (see TailLayout), from the
+// coarsest level up to the finest that still fits: 16-bit local indices, at
+// most 4096 rows of an instance and index and FP64 value prefixes of at most
+// kTailBytes.  Level prefixes are padded to 16 bytes for the vector copies.
+void build_tail(AmgHierarchy &H) {
+    TailLayout &T = H.tail;
+    const int L = int(H.lev.size()), ninst = int(H.lev.back().inst_ptr.size()) - 1;
+    T = TailLayout();
+    T.tab.assign((size_t)ninst * L * TL_K, 0);
+    T.iend.assign(L, 0);
+    T.vend.assign(L, 0);
+    T.vec.assign(L, 0);
+    // sizes first: the finest level every instance can hold
+    T.first = L - 1;
+    for (int l = L - 1; l >= 1; --l) {
+        const AmgLevel &F = H.lev[l];
+        bool fits = true;
+        for (int s = 0; s < ninst; ++s) {
+            int *t = &T.tab[((size_t)s * L + l) * TL_K];
+            const int *up = l + 1 < L ? t + TL_K : nullptr;
+            t[TL_R0] = F.inst_ptr[s];
+            const long long n = t[TL_N] = F.inst_ptr[s + 1] - F.inst_ptr[s];
+            long long ni = up ? up[TL_IEND] : 0, nv = up ? up[TL_VEND] : 0;
+            t[TL_VEC] = up ? up[TL_VEC] + (l + 2 < L ? 3 : 2) * up[TL_N] : 0;
+            auto take = [](long long &at, long long k) { const long long o = at; at += k; return (int)o; };
+            if (!up) {
+                t[TL_VAL] = take(nv, n * n);
+            } else {
+                const long long nC = up[TL_N];
+                t[TL_E0] = F.row_ptr[t[TL_R0]];
+                t[TL_NNZ] = F.row_ptr[t[TL_R0] + n] - t[TL_E0];
+                t[TL_RP] = take(ni, n + 1);
+                t[TL_COL] = take(ni, t[TL_NNZ]);
+                t[TL_VAL] = take(nv, t[TL_NNZ]);
+                t[TL_WD] = take(nv, n);
+                if (F.sa_out) {
+                    t[TL_PT0] = F.pt_ptr[up[TL_R0]];
+                    t[TL_NPT] = F.pt_ptr[up[TL_R0] + nC] - t[TL_PT0];
+                    t[TL_T0] = F.t_ptr[t[TL_R0]];
+                    t[TL_NT] = F.t_ptr[t[TL_R0] + n] - t[TL_T0];
+                    t[TL_PTP] = take(ni, nC + 1);
+                    t[TL_PTC] = take(ni, t[TL_NPT]);
+                    t[TL_TP] = take(ni, n + 1);
+                    t[TL_TC] = take(ni, t[TL_NT]);
+                    t[TL_PTV] = take(nv, t[TL_NPT]);
+                    t[TL_MV] = take(nv, t[TL_NT]);
+                } else {
+                    t[TL_CP] = take(ni, nC + 1);
+                    t[TL_CH] = take(ni, n);
+                    t[TL_AGG] = take(ni, n);
+                }
+            }
+            ni = (ni + 7) / 8 * 8;
+            nv = (nv + 3) / 4 * 4;
+            // (the coarsest level always fits: at most kMaxCoarsest rows)
+            if (up && (n > 4096 || t[TL_NNZ] > 65535 || t[TL_NPT] > 65535 || t[TL_NT] > 65535 ||
+                       2 * ni + 8 * nv > kTailBytes))
+                fits = false;
+            t[TL_IEND] = (int)std::min<long long>(ni, 1 << 30);
+            t[TL_VEND] = (int)std::min<long long>(nv, 1 << 30);
+            T.iend[l] = std::max(T.iend[l], t[TL_IEND]);
+            T.vend[l] = std::max(T.vend[l], t[TL_VEND]);
+            T.vec[l] = std::max(T.vec[l], t[TL_VEC] + (up ? 3 : 2) * (int)n);
+        }
+        if (!fits) break;
+        T.first = l;
+    }
+    long long ni = 0, nv = 0;
+    for (int s = 0; s < ninst; ++s) {
+        int *t0 = &T.tab[(size_t)s * L * TL_K];
+        t0[0] = int(ni);
+        t0[1] = int(nv);
+        ni += t0[T.first * TL_K + TL_IEND];
+        nv += t0[T.first * TL_K + TL_VEND];
+    }
+    if (ni > 0x7fffffffLL || nv > 0x7fffffffLL) {   // 32-bit offsets: the coarsest level alone
+        T.first = L - 1;
+        ni = nv = 0;
+        for (int s = 0; s < ninst; ++s) {
+            int *t0 = &T.tab[(size_t)s * L * TL_K];
+            t0[0] = 0;
+            t0[1] = int(nv);
+            nv += t0[(L - 1) * TL_K + TL_VEND];
+        }
+    }
+    T.nval = nv;
+    T.idx.assign(std::max<long long>(ni, 8), 0);
+    for (int s = 0; s < ninst; ++s)
+        for (int l = T.first; l + 1 < L; ++l) {
+            const AmgLevel &F = H.lev[l], &C = H.lev[l + 1];
+            const int *t = &T.tab[((size_t)s * L + l) * TL_K], *up = t + TL_K;
+            uint16_t *o = &T.idx[T.tab[(size_t)s * L * TL_K]];
+            const int r0 = t[TL_R0], n = t[TL_N], c0 = up[TL_R0], nC = up[TL_N];
+            for (int i = 0; i <= n; ++i) o[t[TL_RP] + i] = uint16_t(F.row_ptr[r0 + i] - t[TL_E0]);
+            for (int e = 0; e < t[TL_NNZ]; ++e) o[t[TL_COL] + e] = uint16_t(F.col[t[TL_E0] + e] - r0);
+            if (F.sa_out) {
+                for (int i = 0; i <= nC; ++i) o[t[TL_PTP] + i] = uint16_t(F.pt_ptr[c0 + i] - t[TL_PT0]);
+                for (int e = 0; e < t[TL_NPT]; ++e) o[t[TL_PTC] + e] = uint16_t(F.pt_col[t[TL_PT0] + e] - r0);
+                for (int i = 0; i <= n; ++i) o[t[TL_TP] + i] = uint16_t(F.t_ptr[r0 + i] - t[TL_T0]);
+                for (int e = 0; e < t[TL_NT]; ++e) o[t[TL_TC] + e] = uint16_t(F.t_col[t[TL_T0] + e] - c0);
+            } else {
+                const int k0 = C.child_ptr[c0];
+                for (int i = 0; i <= nC; ++i) o[t[TL_CP] + i] = uint16_t(C.child_ptr[c0 + i] - k0);
+                for (int k = k0; k < C.child_ptr[c0 + nC]; ++k) o[t[TL_CH] + k - k0] = uint16_t(C.child[k] - r0);
+                for (int i = 0; i < n; ++i) o[t[TL_AGG] + i] = uint16_t(C.agg[r0 + i] - c0);
+            }
+        }
+}
+
 }  // namespace
 
 std::string instance_dims(const Topology &T, const std::vector<int> &ijk, std::vector<int> &dims) {
@@ -385,6 +494,7 @@ std::string build_amg(AmgHierarchy &H, const Topology &T, const std::vector<int>
     for (size_t l = 1; l < H.lev.size(); ++l)
         for (int I = 0; I < H.lev[l].n; ++I)
             if (H.lev[l].diag[I] < 0) return "coarse row without a diagonal entry";
+    build_tail(H);
     return "";
 }
 

@@ -62,11 +62,38 @@ struct ApPattern {
     std::vector<int> src;              // face-matrix SELL positions
 };
 
+// The small levels of one V-cycle as the one-workgroup tail kernel reads them
+// (k_vcycle_tail): per instance one block of 16-bit indices and one block of
+// values, each ordered from the coarsest level to finer ones, so that a tail
+// starting at level lt copies a prefix of both into LDS.  The index block is
+// static; the values are gathered into theirs once per solve.
+enum {
+    TL_R0 = 0, TL_N,                   // first row, rows of the instance on this level
+    TL_E0, TL_NNZ,                     // entries of those rows in the level's matrix
+    TL_RP, TL_COL,                     // index block: local row pointers and columns
+    TL_CP, TL_CH, TL_AGG,              // tentative transfer to the next level: children, aggregates
+    TL_PTP, TL_PTC, TL_TP, TL_TC,      // smoothed transfer: rows of P' and of M
+    TL_PT0, TL_NPT, TL_T0, TL_NT,      // their entries in the level's arrays
+    TL_VAL, TL_WD, TL_PTV, TL_MV,      // value block: matrix, w D^-1, P', M (coarsest: the dense inverse)
+    TL_VEC,                            // vectors: b, x, res (coarsest: b, x), in rows
+    TL_IEND, TL_VEND,                  // lengths of the prefixes that include this level
+    TL_K
+};                                     // (row 0 of an instance: offsets of its blocks in TL_R0, TL_N)
+struct TailLayout {
+    int first = 0;                     // finest level the blocks hold
+    std::vector<int> tab;              // [ninst][nlev][TL_K]
+    std::vector<uint16_t> idx;
+    long long nval = 0;                // values over all instances
+    std::vector<int> iend, vend, vec;  // per level: longest prefixes and most vector rows of an instance
+};
+constexpr int kTailBytes = 152 * 1024; // LDS the tail may take
+
 struct AmgHierarchy {
     std::vector<AmgLevel> lev;      // lev[0] unused placeholder, lev[1..] coarse levels
     std::vector<std::array<int, 3>> blocks;  // logical block factors of each transfer (l -> l+1)
     std::vector<int> coarse_off;    // [ninst+1] offsets of the dense coarsest inverses
     ApPattern ap;
+    TailLayout tail;
     int nlev() const { return int(lev.size()); }
 };
 

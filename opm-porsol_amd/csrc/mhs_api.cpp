@@ -74,7 +74,6 @@ struct mhs_solver {
     hipStream_t user_stream = nullptr;  // caller's stream, ordered against ours
     hipEvent_t ev_in = nullptr, ev_out = nullptr;
     hipEvent_t ev_ph[4] = {};       // phase boundaries of a solve on its stream (report times)
-    std::vector<unsigned char> dA_copied;   // the multigrid descriptor last copied to the device
     std::string err;
     // this device's scratch array (mhs_sum_outflux_noalloc); null when the
     // address lookup at creation failed, with the reason in scratch_err
@@ -227,7 +226,6 @@ void mhs_solver::free_amg() {
     amg_bufs.clear();
     amg_planned = false;
     dA = DevAmg{};
-    dA_copied.clear();      // a new hierarchy has a new device descriptor
     setup_gen = -1;
     has_amg = false;
     H = AmgHierarchy();
@@ -501,7 +499,16 @@ int build_amg_device(mhs_solver *s, const Strength &strength) {
         if (he == hipSuccess) A.ap64 = dalloc<double>(s, L, (size_t)A.ap_slots, &he);
         if (he == hipSuccess) A.ap32 = dalloc<float>(s, L, (size_t)A.ap_slots, &he);
         if (he == hipSuccess) A.coarse_off = dupload(s, L, s->H.coarse_off, &he);
-        if (he == hipSuccess) A.dev = dalloc<DevAmg>(s, L, 1, &he);
+        if (he == hipSuccess) A.tail_tab = dupload(s, L, s->H.tail.tab, &he);
+        if (he == hipSuccess) A.tail_idx = dupload(s, L, s->H.tail.idx, &he);
+        if (he == hipSuccess) A.tail_val64 = dalloc<double>(s, L, (size_t)s->H.tail.nval, &he);
+        if (he == hipSuccess) A.tail_val32 = dalloc<float>(s, L, (size_t)s->H.tail.nval, &he);
+        A.tail_first = s->H.tail.first;
+        for (int l = 0; l < A.nlev; ++l) {
+            A.tail_iend[l] = s->H.tail.iend[l];
+            A.tail_vend[l] = s->H.tail.vend[l];
+            A.tail_vec[l] = s->H.tail.vec[l];
+        }
         A.alpha_sa = 1.0;
         A.omega_p = 2.0 / 3.0;
         if (he == hipSuccess) A.cinv64 = dalloc<double>(s, L, (size_t)s->H.coarse_off.back(), &he);
@@ -1597,17 +1604,9 @@ int solve_impl(mhs_solver *s, const double *totmob, const double *rhomob, const 
                     s->dA.omega_l[l] = r > 0.0 ? std::min(1.0, std::max(0.2, 4.0 / (3.0 * r))) : 0.7;
                 }
             }
-            // the kernels that walk the whole hierarchy read this copy (nothing of
-            // the previous solve is still running: it ended with a synchronise;
-            // the set-up kernels above do not read it)
-            // (copied only when it changed: a blocking copy stalls the stream)
-            const unsigned char *da = reinterpret_cast<const unsigned char *>(&s->dA);
-            if (s->dA_copied.size() != sizeof(DevAmg) ||
-                std::memcmp(s->dA_copied.data(), da, sizeof(DevAmg)) != 0) {
-                HIPCHECK(hipMemcpy(const_cast<DevAmg *>(s->dA.dev), &s->dA, sizeof(DevAmg), hipMemcpyHostToDevice));
-                s->dA_copied.assign(da, da + sizeof(DevAmg));
-            }
             if (!mg_reused) HIPCHECK(launch_amg_combine(s->stream, s->dA, mixed));
+            // (also for kept levels: their last solve may have had the other precision)
+            HIPCHECK(launch_amg_tail_pack(s->stream, s->dA, mixed));
         }
 
         // --- launch shapes -------------------------------------------------------

@@ -146,7 +146,15 @@ struct DevAmg {
     double alpha;                   // coarse-correction (prolongation) factor
     double alpha_sa;                // coarse-correction factor across smoothed transfers
     double omega_p;                 // prolongation-smoothing weight of those transfers
-    const DevAmg *dev;              // this structure's copy in device memory (refreshed by the host)
+    // one-workgroup tail: its offsets, index blocks and value blocks (see
+    // TailLayout), the finest level they hold, and per level the longest index
+    // and value prefixes and the most vector rows of an instance
+    const int *tail_tab;
+    const uint16_t *tail_idx;
+    double *tail_val64;
+    float *tail_val32;
+    int tail_first;
+    int tail_iend[kMaxLevels], tail_vend[kMaxLevels], tail_vec[kMaxLevels];
     int nu;                         // smoothing sweeps before and after the coarse correction
     int max_rows[kMaxLevels];       // rows of the largest instance on each level
     int max_children[kMaxLevels];   // most finer rows aggregated into one row of each level
@@ -163,8 +171,6 @@ struct DevAmg {
     const int *ap_esrc_ptr, *ap_esrc;
     long long ap_ensrc;
 };
-// DevAmg is larger than the kernel-argument limit: kernels that need the
-// whole hierarchy read a copy in device memory.
 
 hipError_t launch_static_ip(hipStream_t st, const DevTopo &T, const DevGeom &G, int maxn,
                             const double *perm, const double *grav, double *binv_pk,
@@ -241,9 +247,11 @@ hipError_t launch_resnorm(hipStream_t st, const DevTopo &T, int nrhs, const doub
 
 // Multigrid: per-solve set-up (Galerkin products, diagonals, coarsest inverses)
 // and the preconditioned iteration pieces.
-// The up-sweep operator M = P - w D^-1 T of each smoothed transfer, once the
-// smoother weights are known (after launch_amg_setup).
+// Once the smoother weights are known (after launch_amg_setup): the up-sweep
+// operator M = P - w D^-1 T of each smoothed transfer, and (after it) the value
+// blocks of the one-workgroup tail in the PCG's precision.
 hipError_t launch_amg_combine(hipStream_t st, const DevAmg &A, bool mixed);
+hipError_t launch_amg_tail_pack(hipStream_t st, const DevAmg &A, bool mixed);
 hipError_t launch_amg_setup(hipStream_t st, const DevTopo &T, const DevAmg &A, const double *val64,
                             bool mixed, const double *elem64 = nullptr, bool ap_only = false);
 // Lanczos on D^-1/2 A_l D^-1/2 (FP64) for the Jacobi weight of level l:

@@ -1236,8 +1236,7 @@ __global__ __launch_bounds__(256) void k_resnorm(DevTopo T, const double *__rest
 // are loaded together, then everything that depends on them, so a row costs a
 // few memory round trips instead of one dependent chain per entry (the small
 // levels are latency-bound).  Padding lanes either read the row's own entries
-// or issue no load at all: never a row of another instance, which the
-// one-workgroup-per-instance tail may not have written yet (0 * NaN != 0).
+// or issue no load at all (0 * NaN != 0).
 constexpr int kChunk = 8;
 
 // Rows can be shared by a group of G lanes (G divides 64, so a group lies in
@@ -1411,11 +1410,11 @@ __global__ __launch_bounds__(1024) void k_coarse_inverse(DevAmgLevel L, const in
 }
 
 template <typename VT>
-__device__ __forceinline__ const VT *lvl_val(const DevAmgLevel &L) {
+__host__ __device__ __forceinline__ const VT *lvl_val(const DevAmgLevel &L) {
     if constexpr (std::is_same<VT, float>::value) return L.val32; else return L.val64;
 }
 template <typename VT>
-__device__ __forceinline__ const VT *lvl_dinv(const DevAmgLevel &L) {
+__host__ __device__ __forceinline__ const VT *lvl_dinv(const DevAmgLevel &L) {
     if constexpr (std::is_same<VT, float>::value) return L.dinv32; else return L.dinv64;
 }
 
@@ -1521,15 +1520,15 @@ __device__ __forceinline__ void row_restrict(const int *__restrict__ child_ptr, 
 }
 
 template <typename VT>
-__device__ __forceinline__ const VT *lvl_p(const DevAmgLevel &L) {
+__host__ __device__ __forceinline__ const VT *lvl_p(const DevAmgLevel &L) {
     if constexpr (std::is_same<VT, float>::value) return L.p_val32; else return L.p_val64;
 }
 template <typename VT>
-__device__ __forceinline__ const VT *lvl_pt(const DevAmgLevel &L) {
+__host__ __device__ __forceinline__ const VT *lvl_pt(const DevAmgLevel &L) {
     if constexpr (std::is_same<VT, float>::value) return L.pt_val32; else return L.pt_val64;
 }
 template <typename VT>
-__device__ __forceinline__ const VT *lvl_m(const DevAmgLevel &L) {
+__host__ __device__ __forceinline__ const VT *lvl_m(const DevAmgLevel &L) {
     if constexpr (std::is_same<VT, float>::value) return L.m_val32; else return L.m_val64;
 }
 
@@ -2084,120 +2083,225 @@ __global__ __launch_bounds__(256) void k_vcc_up_plain(DevAmgLevel F, const VT *_
     }
 }
 
-// The small levels lt..L-1 of one V(1,1) cycle (one sweep each way), one
-// workgroup per instance: the same arithmetic as k_vcc_down + k_restrict,
-// k_coarse_solve and k_vcc_up1, with workgroup barriers between the steps
-// instead of kernel launches.  Reads lev[lt].b, writes lev[l].x for l >= lt.
-template <typename VT, int NRHS>
-__global__ __launch_bounds__(1024) void k_vcycle_tail(Gate gt, const DevAmg *__restrict__ Ap, int lt, VT al,
-                                                      VT als,
-                                                      VT *__restrict__ xf) {
-    const DevAmg &A = *Ap;
-    const int s = blockIdx.x;
-    if (gate_off<NRHS>(gt, s)) return;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int L = A.nlev;
-    for (int l = lt; l < L - 1; ++l) {
-        const DevAmgLevel &F = A.lev[l];
-        const DevAmgLevel &C = A.lev[l + 1];
-        const VT w = (VT)A.omega_l[l];
-        const VT *val = lvl_val<VT>(F);
-        const VT *dinv = lvl_dinv<VT>(F);
-        const VT *b = (const VT *)F.b;
-        VT *res = (VT *)F.res;
-        const int r0 = F.inst_ptr[s], r1 = F.inst_ptr[s + 1];
-        for (int i = r0 + tid; i < r1; i += nt) {
-            VT acc[NRHS];
-            row_down<VT, NRHS>(F, val, dinv, b, w, i, acc);
+// Copies n 16-byte words to LDS, four loads in flight per thread.
+__device__ __forceinline__ void copy_lds(uint4 *__restrict__ dst, const uint4 *__restrict__ src, int n) {
+    for (int base = threadIdx.x; base < n; base += 4 * 1024) {
+        uint4 v[4];
 #pragma unroll
-            for (int k = 0; k < NRHS; ++k) res[(size_t)i * NRHS + k] = b[(size_t)i * NRHS + k] - acc[k];
+        for (int u = 0; u < 4; ++u)
+            if (base + 1024 * u < n) v[u] = src[base + 1024 * u];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (base + 1024 * u < n) dst[base + 1024 * u] = v[u];
+    }
+}
+
+// acc = sum over entries [p[i], p[i+1]) of val * x[col], G lanes (a power of
+// two, at most a wavefront) sharing the row; all lanes get the sum.
+template <typename VT, int NRHS>
+__device__ __forceinline__ void lds_row(const uint16_t *p, const uint16_t *col, const VT *val, const VT *x, int i,
+                                        int sub, int G, VT (&acc)[NRHS]) {
+#pragma unroll
+    for (int k = 0; k < NRHS; ++k) acc[k] = VT(0);
+    const int e1 = p[i + 1];
+    for (int e = p[i] + sub; e < e1; e += G) {
+        const VT a = val[e];
+        const int c = col[e];
+#pragma unroll
+        for (int k = 0; k < NRHS; ++k) acc[k] += a * x[c * NRHS + k];
+    }
+    for (int m = G >> 1; m >= 1; m >>= 1)
+#pragma unroll
+        for (int k = 0; k < NRHS; ++k) acc[k] += __shfl_xor(acc[k], m, 64);
+}
+
+// log2 of the lanes per row that keep 1024 threads busy on n rows (at most 16).
+__device__ __forceinline__ int tail_lanes(int n) {
+    int g = 0;
+    while (g < 4 && (n << (g + 1)) <= 1024) ++g;
+    return g;
+}
+
+// The small levels lt..L-1 of one V(1,1) cycle (one sweep each way), one
+// workgroup per instance, everything in LDS: the workgroup copies the
+// instance's index and value prefixes and b of level lt in one round trip,
+// then every step is LDS reads, a few lanes per row and a workgroup barrier.
+// Bound by that first round trip and the LDS latency of the steps.  With the
+// matrices read from global memory, a dependent chain of loads per row and
+// step, it took (rocprofv3) 20.4 us for levels of 125 and 27 rows in FP64, 24.9
+// us for the same behind a smoothed transfer with three right-hand sides and
+// 24.0 us for 384 and 48 rows in FP32; now 8.3, 11.8 and 13.4 us.
+// Reads lev[lt].b, writes lev[lt].x and, when the transfer from the finer level
+// is tentative and covers it, prolongs that into the finer level's iterate in
+// place: x~_f = w D^-1 b + al x_lt[agg_f] (the down-sweep wrote w D^-1 b).
+template <typename VT, int NRHS>
+__global__ __launch_bounds__(1024) void k_vcycle_tail(Gate gt, const int *__restrict__ tabs,
+                                                      const uint16_t *__restrict__ idx,
+                                                      const VT *__restrict__ vals, int L, int lt, int vbase,
+                                                      int xbase, const VT *__restrict__ gb, VT *__restrict__ gx,
+                                                      VT al, VT als, const int *__restrict__ fagg,
+                                                      VT *__restrict__ xf) {
+    extern __shared__ __align__(16) unsigned char tail_lds[];
+    uint16_t *ix = reinterpret_cast<uint16_t *>(tail_lds);
+    VT *vl = reinterpret_cast<VT *>(tail_lds + vbase);
+    VT *vec = reinterpret_cast<VT *>(tail_lds + xbase);
+    const int s = blockIdx.x, tid = threadIdx.x;
+    const int *tab = tabs + (size_t)s * L * TL_K;
+    if (gate_off<NRHS>(gt, s)) return;
+    auto rows = [&](int l) { return tab + l * TL_K; };
+    auto vb = [&](int l) { return vec + (size_t)rows(l)[TL_VEC] * NRHS; };   // b, then x, then res
+    constexpr int PF = 4;
+    const int *T0 = rows(lt);
+    const int n0 = T0[TL_N], nf = xf ? rows(lt - 1)[TL_N] : 0, f0 = xf ? rows(lt - 1)[TL_R0] : 0;
+    // the finer level's aggregates and iterate, needed last, are loaded first
+    int ag[PF];
+    VT xv[PF][NRHS];
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+        const int f = tid + 1024 * u;
+        ag[u] = f < nf ? fagg[f0 + f] - T0[TL_R0] : 0;
+#pragma unroll
+        for (int k = 0; k < NRHS; ++k) xv[u][k] = f < nf ? xf[(size_t)(f0 + f) * NRHS + k] : VT(0);
+    }
+    {
+        VT *b = vb(lt);
+        for (int i = tid; i < n0 * NRHS; i += 1024) b[i] = gb[(size_t)T0[TL_R0] * NRHS + i];
+        copy_lds(reinterpret_cast<uint4 *>(ix), reinterpret_cast<const uint4 *>(idx + tab[0]), T0[TL_IEND] / 8);
+        copy_lds(reinterpret_cast<uint4 *>(vl), reinterpret_cast<const uint4 *>(vals + tab[1]),
+                 T0[TL_VEND] / (int)(16 / sizeof(VT)));
+    }
+    __syncthreads();
+    for (int l = lt; l < L - 1; ++l) {
+        const int *t = rows(l), n = t[TL_N], nC = t[TL_K + TL_N];
+        VT *b = vb(l), *x = b + n * NRHS, *res = x + n * NRHS, *bc = vb(l + 1);
+        const VT *wd = vl + t[TL_WD];
+        for (int i = tid; i < n * NRHS; i += 1024) x[i] = wd[i / NRHS] * b[i];
+        __syncthreads();
+        const int g = tail_lanes(n);
+        for (int q = tid; q < n << g; q += 1024) {
+            const int i = q >> g, sub = q & ((1 << g) - 1);
+            VT acc[NRHS];
+            lds_row<VT, NRHS>(ix + t[TL_RP], ix + t[TL_COL], vl + t[TL_VAL], x, i, sub, 1 << g, acc);
+            if (sub == 0)
+#pragma unroll
+                for (int k = 0; k < NRHS; ++k) res[i * NRHS + k] = b[i * NRHS + k] - acc[k];
         }
         __syncthreads();
-        VT *bc = (VT *)C.b;
-        for (int I = C.inst_ptr[s] + tid; I < C.inst_ptr[s + 1]; I += nt) {
-            VT acc[NRHS];
-            if (F.sa_out) row_restrict_sa<VT, NRHS>(F, res, I, acc);
-            else row_restrict<VT, NRHS>(C.child_ptr, C.child, res, I, acc);
+        if (t[TL_NPT]) {
+            const int gc = tail_lanes(nC);
+            for (int q = tid; q < nC << gc; q += 1024) {
+                const int I = q >> gc, sub = q & ((1 << gc) - 1);
+                VT acc[NRHS];
+                lds_row<VT, NRHS>(ix + t[TL_PTP], ix + t[TL_PTC], vl + t[TL_PTV], res, I, sub, 1 << gc, acc);
+                if (sub == 0)
 #pragma unroll
-            for (int k = 0; k < NRHS; ++k) bc[(size_t)I * NRHS + k] = acc[k];
+                    for (int k = 0; k < NRHS; ++k) bc[I * NRHS + k] = acc[k];
+            }
+        } else {
+            const uint16_t *cp = ix + t[TL_CP], *ch = ix + t[TL_CH];
+            for (int q = tid; q < nC * NRHS; q += 1024) {
+                const int I = q / NRHS, k = q % NRHS;
+                VT a = VT(0);
+                for (int c = cp[I]; c < cp[I + 1]; ++c) a += res[ch[c] * NRHS + k];
+                bc[q] = a;
+            }
         }
         __syncthreads();
     }
+    const VT *xc;
     {
-        // coarsest level: x = A^-1 b with the dense inverse, one wavefront per
-        // (row, rhs) and four of them per pass: lane j takes column j (the
-        // row-major inverse is read coalesced), a shuffle sum finishes the row
-        const DevAmgLevel &C = A.lev[L - 1];
-        const int r0 = C.inst_ptr[s], m = C.inst_ptr[s + 1] - r0;
-        const VT *inv;
-        if constexpr (std::is_same<VT, float>::value) inv = A.cinv32 + A.coarse_off[s];
-        else inv = A.cinv64 + A.coarse_off[s];
-        const VT *b = (const VT *)C.b;
-        VT *x = (VT *)C.x;
-        const int lane = tid & 63, wid = tid >> 6, nw = nt >> 6;
-        const int rows = m * NRHS;
-        for (int e0 = wid; e0 < rows; e0 += 4 * nw) {
-            VT acc[4];
+        // coarsest level: x = A^-1 b with the dense inverse, 16 lanes per row
+        const int *t = rows(L - 1), m = t[TL_N];
+        const VT *b = vb(L - 1), *inv = vl + t[TL_VAL];
+        VT *x = vb(L - 1) + m * NRHS;
+        for (int q = tid; q < m * NRHS * 16; q += 1024) {
+            const int e = q >> 4, i = e / NRHS, k = e % NRHS;
+            VT a = VT(0);
+            for (int j = q & 15; j < m; j += 16) a += inv[i * m + j] * b[j * NRHS + k];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                acc[u] = VT(0);
-                const int e = e0 + u * nw;
-                if (e >= rows) continue;
-                const int i = e / NRHS, k = e % NRHS;
-                for (int j = lane; j < m; j += 64) acc[u] += inv[i * m + j] * b[(size_t)(r0 + j) * NRHS + k];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) acc[u] += __shfl_xor(acc[u], off, 64);
-                const int e = e0 + u * nw;
-                if (lane == 0 && e < rows) x[(size_t)(r0 + e / NRHS) * NRHS + e % NRHS] = acc[u];
-            }
+            for (int o = 8; o >= 1; o >>= 1) a += __shfl_xor(a, o, 64);
+            if ((q & 15) == 0) x[e] = a;
         }
+        xc = x;
         __syncthreads();
     }
     for (int l = L - 2; l >= lt; --l) {
-        const DevAmgLevel &F = A.lev[l];
-        const VT w = (VT)A.omega_l[l];
-        const int *agg = A.lev[l + 1].agg;
-        const VT *xc = (const VT *)A.lev[l + 1].x;
-        if (F.sa_out) {
-            for (int i = F.inst_ptr[s] + tid; i < F.inst_ptr[s + 1]; i += nt) up_sa_row<VT, NRHS>(F, xc, w, als, i);
+        const int *t = rows(l), n = t[TL_N], g = tail_lanes(n);
+        VT *b = vb(l), *x = b + n * NRHS, *res = x + n * NRHS;
+        const VT *wd = vl + t[TL_WD];
+        const bool sa = t[TL_NPT] != 0;
+        if (!sa) {
+            const uint16_t *agg = ix + t[TL_AGG];
+            for (int q = tid; q < n * NRHS; q += 1024) x[q] += al * xc[agg[q / NRHS] * NRHS + q % NRHS];
             __syncthreads();
-            continue;
         }
-        const VT *val = lvl_val<VT>(F);
-        const VT *dinv = lvl_dinv<VT>(F);
-        const VT *b = (const VT *)F.b;
-        VT *xo = (VT *)F.x;
-        for (int i = F.inst_ptr[s] + tid; i < F.inst_ptr[s + 1]; i += nt) {
+        for (int q = tid; q < n << g; q += 1024) {
+            const int i = q >> g, sub = q & ((1 << g) - 1);
             VT acc[NRHS];
-            row_up1<VT, NRHS>(F, val, dinv, b, agg, xc, w, al, i, acc);
-            const VT d = w * dinv[i];
-            const int g = agg[i];
+            if (sa) lds_row<VT, NRHS>(ix + t[TL_TP], ix + t[TL_TC], vl + t[TL_MV], xc, i, sub, 1 << g, acc);
+            else lds_row<VT, NRHS>(ix + t[TL_RP], ix + t[TL_COL], vl + t[TL_VAL], x, i, sub, 1 << g, acc);
+            if (sub != 0) continue;
+            const VT d = wd[i];
 #pragma unroll
             for (int k = 0; k < NRHS; ++k) {
-                const size_t q = (size_t)i * NRHS + k;
-                const VT xv = d * b[q] + al * xc[(size_t)g * NRHS + k];
-                xo[q] = xv + d * (b[q] - acc[k]);
+                const int e = i * NRHS + k;
+                // (res is free once read: every row reads and writes its own)
+                res[e] = sa ? d * (b[e] + res[e]) + als * acc[k] : x[e] + d * (b[e] - acc[k]);
             }
         }
+        xc = res;
         __syncthreads();
     }
-    if (xf) {
-        // the transfer from level lt to the finer level is tentative and
-        // covers it: prolong lev[lt].x into that level's iterate in place,
-        // x~_f = w D^-1 b + al x_lt[agg_f] (the down-sweep wrote w D^-1 b)
-        // (one thread per finer row: every row has its aggregate)
-        const DevAmgLevel &C = A.lev[lt];
-        const DevAmgLevel &F = A.lev[lt - 1];
-        const VT *xc = (const VT *)C.x;
-        for (int f = F.inst_ptr[s] + tid; f < F.inst_ptr[s + 1]; f += nt) {
-            const int J = C.agg[f];
+    for (int i = tid; i < n0 * NRHS; i += 1024) gx[(size_t)T0[TL_R0] * NRHS + i] = xc[i];
 #pragma unroll
-            for (int k = 0; k < NRHS; ++k) xf[(size_t)f * NRHS + k] += al * xc[(size_t)J * NRHS + k];
-        }
+    for (int u = 0; u < PF; ++u) {
+        const int f = tid + 1024 * u;
+        if (f >= nf) break;
+#pragma unroll
+        for (int k = 0; k < NRHS; ++k) xf[(size_t)(f0 + f) * NRHS + k] = xv[u][k] + al * xc[ag[u] * NRHS + k];
     }
+    for (int f = tid + 1024 * PF; f < nf; f += 1024) {
+        const int J = fagg[f0 + f] - T0[TL_R0];
+#pragma unroll
+        for (int k = 0; k < NRHS; ++k) xf[(size_t)(f0 + f) * NRHS + k] += al * xc[J * NRHS + k];
+    }
+}
+
+// Value blocks of the tail: one workgroup per instance, array (blockIdx.y:
+// matrix, w D^-1, P', M; on the coarsest level its inverse) and level.
+template <typename VT>
+struct TailSrc {
+    const VT *val, *dinv, *ptv, *mv;
+    VT w;
+};
+template <typename VT>
+struct TailPack {
+    const int *tab, *coff;
+    const VT *cinv;
+    VT *out;
+    int L, first;
+    TailSrc<VT> lev[kMaxLevels];
+};
+template <typename VT>
+__global__ __launch_bounds__(256) void k_tail_pack(TailPack<VT> P) {
+    const int s = blockIdx.x, what = blockIdx.y, l = P.first + blockIdx.z;
+    const int *tab = P.tab + (size_t)s * P.L * TL_K, *t = tab + l * TL_K;
+    VT *o = P.out + tab[1];
+    const TailSrc<VT> &F = P.lev[l];
+    const int n = t[TL_N];
+    if (l == P.L - 1) {
+        if (what == 0)
+            for (int e = threadIdx.x; e < n * n; e += 256) o[t[TL_VAL] + e] = P.cinv[P.coff[s] + e];
+        return;
+    }
+    if (what == 0)
+        for (int e = threadIdx.x; e < t[TL_NNZ]; e += 256) o[t[TL_VAL] + e] = F.val[t[TL_E0] + e];
+    else if (what == 1)
+        for (int e = threadIdx.x; e < n; e += 256) o[t[TL_WD] + e] = F.w * F.dinv[t[TL_R0] + e];
+    else if (what == 2)
+        for (int e = threadIdx.x; e < t[TL_NPT]; e += 256) o[t[TL_PTV] + e] = F.ptv[t[TL_PT0] + e];
+    else
+        for (int e = threadIdx.x; e < t[TL_NT]; e += 256) o[t[TL_MV] + e] = F.mv[t[TL_T0] + e];
 }
 
 // p = z + beta p (beta = 0 on a restart); in FP32 also fold x32 into x64 for
@@ -3224,6 +3328,21 @@ hipError_t launch_amg_combine(hipStream_t st, const DevAmg &A, bool mixed) {
     return hipGetLastError();
 }
 
+template <typename VT>
+static void tail_pack(hipStream_t st, const DevAmg &A, VT *out, const VT *cinv) {
+    TailPack<VT> P{A.tail_tab, A.coarse_off, cinv, out, A.nlev, A.tail_first, {}};
+    for (int l = A.tail_first; l < A.nlev; ++l) {
+        const DevAmgLevel &F = A.lev[l];
+        P.lev[l] = TailSrc<VT>{lvl_val<VT>(F), lvl_dinv<VT>(F), lvl_pt<VT>(F), lvl_m<VT>(F), (VT)A.omega_l[l]};
+    }
+    k_tail_pack<VT><<<dim3(A.ninst, 4, A.nlev - A.tail_first), 256, 0, st>>>(P);
+}
+hipError_t launch_amg_tail_pack(hipStream_t st, const DevAmg &A, bool mixed) {
+    if (mixed) tail_pack<float>(st, A, A.tail_val32, A.cinv32);
+    else tail_pack<double>(st, A, A.tail_val64, A.cinv64);
+    return hipGetLastError();
+}
+
 static inline unsigned lz_blocks(int n) { return (unsigned)((n + 255) / 256); }
 
 hipError_t launch_lanczos_init(hipStream_t st, int n, double *w, double *part) {
@@ -3290,6 +3409,21 @@ static void sweep0(hipStream_t st, const DevTopo &T, const VT *val0, const VT *d
     });
 }
 
+// LDS of a tail that starts at level lt: indices, then values, then vectors.
+static inline int tail_vbase(const DevAmg &A, int lt) { return 2 * A.tail_iend[lt]; }
+template <typename VT>
+static inline int tail_xbase(const DevAmg &A, int lt) {
+    return tail_vbase(A, lt) + A.tail_vend[lt] * (int)sizeof(VT);
+}
+template <typename VT, int NR>
+static inline long long tail_bytes(const DevAmg &A, int lt) {
+    return tail_xbase<VT>(A, lt) + (long long)A.tail_vec[lt] * NR * (int)sizeof(VT);
+}
+template <typename VT, int NR>
+static inline bool tail_fits(const DevAmg &A, int lt) {
+    return lt >= A.tail_first && tail_bytes<VT, NR>(A, lt) <= kTailBytes;
+}
+
 // gt: inside the PCG loop the V-cycle skips the level-0 blocks and the tail
 // workgroups of finished instances.  The other coarse-level kernels are too
 // short for a gate to pay for its extra memory round trip: they run on, on
@@ -3341,7 +3475,7 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
     if (nu == 1) {
         // first level handled by the workgroup-per-instance tail kernel
         int lt = L - 1;
-        while (lt > 1 && A.max_rows[lt - 1] <= T.tail_rows) --lt;
+        while (lt > 1 && A.max_rows[lt - 1] <= T.tail_rows && tail_fits<VT, NR>(A, lt - 1)) --lt;
         const VT als = (VT)A.alpha_sa;
         for (int l = 1; l < lt; ++l) {
             const DevAmgLevel &F = A.lev[l];
@@ -3386,8 +3520,16 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
             const bool can = l == lt || A.lev[l].sa_out || fuse[l + 1];
             fuse[l] = can && !A.lev[l - 1].sa_out && A.covers[l];
         }
-        k_vcycle_tail<VT, NR><<<A.ninst, 1024, 0, st>>>(gt, A.dev, lt, al, als,
-                                                        fuse[lt] ? (VT *)A.lev[lt - 1].x : nullptr);
+        const VT *tv;
+        if constexpr (std::is_same<VT, float>::value) tv = A.tail_val32; else tv = A.tail_val64;
+        static const hipError_t lds_ok = hipFuncSetAttribute(
+            reinterpret_cast<const void *>(&k_vcycle_tail<VT, NR>), hipFuncAttributeMaxDynamicSharedMemorySize,
+            kTailBytes);
+        (void)lds_ok;   // where it is refused, a launch that needs it reports its own error
+        const int vbase = tail_vbase(A, lt), xbase = tail_xbase<VT>(A, lt);
+        k_vcycle_tail<VT, NR><<<A.ninst, 1024, (unsigned)tail_bytes<VT, NR>(A, lt), st>>>(
+            gt, A.tail_tab, A.tail_idx, tv, L, lt, vbase, xbase, (const VT *)A.lev[lt].b, (VT *)A.lev[lt].x, al, als,
+            A.lev[lt].agg, fuse[lt] ? (VT *)A.lev[lt - 1].x : nullptr);
         VT *xres[kMaxLevels];   // each level's result after its up-sweep
         xres[lt] = (VT *)A.lev[lt].x;
         for (int l = lt - 1; l >= 1; --l) {
