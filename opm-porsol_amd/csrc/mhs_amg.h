@@ -1,12 +1,11 @@
 // Aggregation multigrid hierarchy for the face system (host-side set-up).
 //
-// Aggregates are geometric: a face belongs to its owner cell (the cell of its
-// first half-face), and cells are grouped in blocks of their logical (i, j, k)
-// indices, 2 or 1 cells along each direction depending on the coupling
+// Aggregates are geometric: a face takes the mean of its two cells, and cells are
+// grouped in blocks of their logical (i, j, k) indices, 2 or 1 cells along each direction depending on the coupling
 // strength along it (semi-coarsening of anisotropic problems); every coarser
 // level groups the blocks again.  The coarse operators are algebraic,
-// A_{l+1} = P' A_l P with the piecewise-constant P of the aggregates (smoothed
-// on one transfer).  Their sparsity and, for every coarse entry,
+// A_{l+1} = P' A_l P with that averaging P from the faces and the
+// piecewise-constant P of the aggregates below (smoothed on one transfer).  Their sparsity and, for every coarse entry,
 // the list of finer entries that sum into it are built here once per
 // structure, so that each solve forms the Galerkin products with a pure gather.
 #pragma once
@@ -28,10 +27,13 @@ struct AmgLevel {
     std::vector<int> row_ptr, col;  // CSR pattern (columns sorted)
     std::vector<int> diag;          // position of the diagonal in each row
     std::vector<int> src_ptr;       // [nnz+1] gather list ranges
-    std::vector<int> src;           // positions in the finer level's value array
+    std::vector<int> src;           // positions in the finer level's value array (level 1, ~pos: half of it)
     std::vector<int> agg;           // [n_finer] row of this level each finer row feeds (-1: none)
+    // level 1: second aggregate of a face between two blocks (-1: the face lies
+    // inside one block); the transfer gives such a face the mean of both
+    std::vector<int> agg2;
     std::vector<int> child_ptr;     // [n+1]
-    std::vector<int> child;         // finer rows of each row
+    std::vector<int> child;         // finer rows of each row (level 1: ~f for a face with two aggregates)
     // Levels built by smoothed aggregation take their values as sums of
     // products over pairs (P position, T position) of the finer level's
     // transfer: src holds the P positions, src2 the T positions.
@@ -51,15 +53,16 @@ struct AmgLevel {
 };
 
 // A P with the level-1 aggregates: the fine-row by aggregate matrix of the
-// post-smoothing sweep, (A P)_{iJ} = sum of a_ij over the columns j in
-// aggregate J.  Stored in the SELL-64 layout of the face matrix (lane-major
+// post-smoothing sweep, (A P)_{iJ} = sum of a_ij P_jJ over the columns j that
+// touch aggregate J (P_jJ 1, or 1/2 for a face between two).  Stored in the SELL-64 layout of the face matrix (lane-major
 // slices; padding slots have column 0 and value 0), with, for every slot, the
 // list of face-matrix positions that sum into it.
 struct ApPattern {
     std::vector<long long> slice_ptr;  // [nslices+1]
     std::vector<int> col;              // level-1 row of each slot
     std::vector<int> src_ptr;          // [slots+1]
-    std::vector<int> src;              // face-matrix SELL positions
+    std::vector<int> src;              // face-matrix SELL positions (~pos: half the entry)
+    std::vector<int> slice;            // [slots/64] slice of each group of 64 slots
 };
 
 // The small levels of one V-cycle as the one-workgroup tail kernel reads them

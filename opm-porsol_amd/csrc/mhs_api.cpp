@@ -456,6 +456,7 @@ int build_amg_device(mhs_solver *s, const Strength &strength) {
             if (he == hipSuccess) D.child = dupload(s, L, H.child, &he);
             D.sa_in = H.sa_in ? 1 : 0;
             D.sa_out = H.sa_out ? 1 : 0;
+            D.nchild = H.child.size();
             if (H.sa_in && he == hipSuccess) D.src2 = dupload(s, L, H.src2, &he);
             if (H.sa_out) {
                 D.p_nnz = int(H.p_col.size());
@@ -492,6 +493,8 @@ int build_amg_device(mhs_solver *s, const Strength &strength) {
         }
         if (he == hipSuccess) A.ap_slice_ptr = dupload(s, L, s->H.ap.slice_ptr, &he);
         if (he == hipSuccess) A.ap_col = dupload(s, L, s->H.ap.col, &he);
+        if (he == hipSuccess) A.agg2 = dupload(s, L, s->H.lev[1].agg2, &he);
+        if (he == hipSuccess) A.ap_slice = dupload(s, L, s->H.ap.slice, &he);
         if (he == hipSuccess) A.ap_src_ptr = dupload(s, L, s->H.ap.src_ptr, &he);
         if (he == hipSuccess) A.ap_src = dupload(s, L, s->H.ap.src, &he);
         A.ap_slots = (long long)s->H.ap.col.size();
@@ -914,7 +917,7 @@ hipError_t one_iteration(mhs_solver *s, int nrhs, bool amg, const MT *val, const
                          VT *p, VT *q, VT *z, double tol2) {
     const DevEbe *E = std::is_same<VT, float>::value ? cur_ebe(s) : nullptr;
     if (amg)
-        return launch_pcg_iteration_amg<MT, VT>(s->stream, s->dT, s->dA, nrhs, val, dinv, x, r, p, q, z, s->R,
+        return launch_pcg_iteration_amg<MT, VT>(s->stream, s->dT, s->dA, s->ftype, nrhs, val, dinv, x, r, p, q, z, s->R,
                                                 s->S, s->val64, s->b, s->x64, tol2, E, s->r64);
     return launch_pcg_iteration<MT, VT>(s->stream, s->dT, nrhs, val, dinv, x, r, p, q, s->R, s->S, s->val64,
                                         s->b, s->x64, tol2, E, s->r64);
@@ -991,7 +994,7 @@ int ensure_ap_elements(mhs_solver *s) {
     if (A.ap_esrc_ptr) return MHS_OK;
     if (!s->ebe_ok || A.nlev < 2) return fail(s, MHS_ERR_STATE, "element A P: no element layout or hierarchy");
     std::vector<int> ptr, src;
-    const std::string e = ebe_ap_lists(s->EL, s->T, s->H.ap, s->H.lev[1].agg, ptr, src);
+    const std::string e = ebe_ap_lists(s->EL, s->T, s->H.ap, s->H.lev[1].agg, s->H.lev[1].agg2, ptr, src);
     if (!e.empty()) return fail(s, MHS_ERR_INVALID, "element A P: " + e);
     hipError_t he = hipSuccess;
     const int *dp = dupload(s, s->amg_bufs, ptr, &he);
@@ -1209,9 +1212,9 @@ int autotune(mhs_solver *s, int nrhs, bool mixed, bool amg, bool choose_ebe, dou
             for (int rows : {0, 128, 512, 2048, 8192, 32768}) {
                 s->dT.tail_rows = rows;
                 const float ms = time_it([&]() {
-                    return mixed ? launch_vcycle<float>(s->stream, s->dT, s->dA, nrhs, s->val32, s->dinv32, s->r32,
+                    return mixed ? launch_vcycle<float>(s->stream, s->dT, s->dA, s->ftype, nrhs, s->val32, s->dinv32, s->r32,
                                                         s->z32, s->R, E)
-                                 : launch_vcycle<double>(s->stream, s->dT, s->dA, nrhs, s->val64, s->dinv64,
+                                 : launch_vcycle<double>(s->stream, s->dT, s->dA, s->ftype, nrhs, s->val64, s->dinv64,
                                                          s->r64, s->z64, s->R);
                 });
                 if (ms < bt) { bt = ms; best.tail_rows = rows; }
@@ -1285,10 +1288,10 @@ int linear_solve(mhs_solver *s, const mhs_solve_options &opt, int nrhs, bool mix
     }
     if (amg) {
         if (!mixed)
-            HIPCHECK(launch_amg_start<double>(s->stream, s->dT, s->dA, nrhs, s->val64, s->dinv64, s->r64,
+            HIPCHECK(launch_amg_start<double>(s->stream, s->dT, s->dA, s->ftype, nrhs, s->val64, s->dinv64, s->r64,
                                               s->z64, s->p64, s->R, s->S, nullptr, s->x64));
         else
-            HIPCHECK(launch_amg_start<float>(s->stream, s->dT, s->dA, nrhs, s->val32, s->dinv32, s->r32,
+            HIPCHECK(launch_amg_start<float>(s->stream, s->dT, s->dA, s->ftype, nrhs, s->val32, s->dinv32, s->r32,
                                              s->z32, s->p32, s->R, s->S, nullptr, s->x32, cur_ebe(s)));
     }
     // The first chunk follows the start without a host round trip (its
@@ -1483,7 +1486,9 @@ int solve_impl(mhs_solver *s, const double *totmob, const double *rhomob, const 
     s->solved = false;
     s->last_aniso = binv_use != nullptr;
     const double *binv = binv_use ? binv_use : s->binv, *gflux = gflux_use ? gflux_use : s->gflux;
-    const int dguess = opt.linsolver_type != 0;  // AMG types start from the Dirichlet guess (:1521-1532)
+    // AMG types start from the Dirichlet guess (:1521-1532); the multigrid cycle
+    // leaves Dirichlet rows out, so with it their residual must be zero
+    const int dguess = opt.linsolver_type != 0 || (opt.precond == 1 && s->has_amg);
     float *fill32 = nullptr;
     bool filled_matrix = true;
     auto assemble = [&]() -> int {
@@ -1571,7 +1576,15 @@ int solve_impl(mhs_solver *s, const double *totmob, const double *rhomob, const 
             s->mat_valid = filled_matrix = true;
         }
         if (amg) {
-            s->dA.alpha = opt.prolongate_factor;
+            // Over-correction of the tentative transfers, from the option (default
+            // 1.6): 1.5 below the smoothed transfer and 1.3 between it and the
+            // faces.  Behind the averaging transfer from the faces the full factor
+            // over-shoots the smoothest modes, which in FP32 then alternate from
+            // one iteration to the next (200x200x50 faulted grid, 1e-10 residual:
+            // injection and production 2.4e-9 apart after 52 iterations with
+            // 1.6 and 1.6, 1.7e-10 after 51 now; 128x128x64: 34 and 35).
+            s->dA.alpha = 1.0 + (opt.prolongate_factor - 1.0) * (5.0 / 6.0);
+            s->dA.alpha_f = 1.0 + (opt.prolongate_factor - 1.0) * 0.5;
             s->dA.nu = std::max(1, opt.smooth_steps);
             // same_matrix (the caller's promise, :1491): the coarse levels,
             // the smoothed transfer and the coarsest inverses of the previous
@@ -1580,8 +1593,8 @@ int solve_impl(mhs_solver *s, const double *totmob, const double *rhomob, const 
             mg_reused = opt.same_matrix && attempt == 0 && s->setup_gen == s->perm_gen &&
                         (s->setup_mixed || !mixed) && s->setup_aniso == (binv_use != nullptr);
             // A P from the element values when no face matrix was filled
-            HIPCHECK(launch_amg_setup(s->stream, s->dT, s->dA, s->val64, mixed, s->mat_valid ? nullptr : s->dE.val64,
-                                      mg_reused));
+            HIPCHECK(launch_amg_setup(s->stream, s->dT, s->dA, s->ftype, s->val64, mixed,
+                                      s->mat_valid ? nullptr : s->dE.val64, mg_reused));
             if (!mg_reused) {
                 s->setup_gen = s->perm_gen;
                 s->setup_mixed = mixed;
@@ -1605,8 +1618,9 @@ int solve_impl(mhs_solver *s, const double *totmob, const double *rhomob, const 
                 }
             }
             if (!mg_reused) HIPCHECK(launch_amg_combine(s->stream, s->dA, mixed));
-            // (also for kept levels: their last solve may have had the other precision)
-            HIPCHECK(launch_amg_tail_pack(s->stream, s->dA, mixed));
+            // (also for kept levels: A P is new, and their last solve may have had the
+            // other precision)
+            HIPCHECK(launch_amg_ready(s->stream, s->dT, s->dA, s->ftype, s->dinv64, mixed));
         }
 
         // --- launch shapes -------------------------------------------------------

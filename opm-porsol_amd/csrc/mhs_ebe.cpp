@@ -48,10 +48,10 @@ int greedy_colours(int nc, const int *facepos, const int *nb, std::vector<int> &
 }
 
 std::string ebe_ap_lists(const EbeLayout &E, const Topology &T, const ApPattern &ap, const std::vector<int> &agg,
-                         std::vector<int> &ptr, std::vector<int> &src) {
+                         const std::vector<int> &agg2, std::vector<int> &ptr, std::vector<int> &src) {
     const long long slots = (long long)ap.col.size();
     if (slots >= 0x7fffffffLL || E.nval >= 0x7fffffffLL) return "too many values for 32-bit lists";
-    // slot of (row f, aggregate J): the row's slots are few (about 4)
+    // slot of (row f, aggregate J): the row's slots are few (about 7)
     auto slot_of = [&](int f, int J) -> long long {
         const int sl = f / kSlice;
         const long long base = ap.slice_ptr[sl] + f % kSlice;
@@ -78,15 +78,19 @@ std::string ebe_ap_lists(const EbeLayout &E, const Topology &T, const ApPattern 
                 const int f = T.hf_dof[f0 + i];
                 if (agg[f] < 0) continue;
                 for (int j = 0; j < n; ++j) {
-                    const int J = agg[T.hf_dof[f0 + j]];
-                    if (J < 0) continue;
-                    const long long q = slot_of(f, J);
-                    if (q < 0) return "a cell entry outside the A P pattern";
-                    if (pass == 0) {
-                        ++ptr[q + 1];
-                    } else {
-                        const int pq = i <= j ? pidx(i, j, n) : pidx(j, i, n);
-                        src[fill[q]++] = int(E.seg_val[s] + ebe_slot(l, pq, np));
+                    const int rj = T.hf_dof[f0 + j];
+                    const bool half = agg2[rj] >= 0;
+                    for (int J : {agg[rj], agg2[rj]}) {
+                        if (J < 0) continue;
+                        const long long q = slot_of(f, J);
+                        if (q < 0) return "a cell entry outside the A P pattern";
+                        if (pass == 0) {
+                            ++ptr[q + 1];
+                        } else {
+                            const int pq = i <= j ? pidx(i, j, n) : pidx(j, i, n);
+                            const int v = int(E.seg_val[s] + ebe_slot(l, pq, np));
+                            src[fill[q]++] = half ? ~v : v;
+                        }
                     }
                 }
             }

@@ -110,7 +110,8 @@ struct DevAmgLevel {
     const int *inst_ptr;            // [ninst+1] first row of each instance
     const int *row_ptr, *col, *diag, *src_ptr, *src;
     const int *agg;                 // rows of the finer level -> rows of this level
-    const int *child_ptr, *child;   // rows of this level -> rows of the finer level
+    const int *child_ptr, *child;   // rows of this level -> rows of the finer level (level 1: ~f with half weight)
+    size_t nchild;
     double *val64, *dinv64;
     float *val32, *dinv32;
     void *b, *x, *res, *xt;         // work vectors (PCG precision, n * nrhs)
@@ -143,7 +144,9 @@ struct DevAmg {
     double *cinv64;
     float *cinv32;
     double omega_l[kMaxLevels];     // Jacobi weight of each level's smoother
-    double alpha;                   // coarse-correction (prolongation) factor
+    // coarse-correction (prolongation) factor of the tentative transfers below
+    // the smoothed one, and of those between it and the faces
+    double alpha, alpha_f;
     double alpha_sa;                // coarse-correction factor across smoothed transfers
     double omega_p;                 // prolongation-smoothing weight of those transfers
     // one-workgroup tail: its offsets, index blocks and value blocks (see
@@ -159,8 +162,13 @@ struct DevAmg {
     int max_rows[kMaxLevels];       // rows of the largest instance on each level
     int max_children[kMaxLevels];   // most finer rows aggregated into one row of each level
     int covers[kMaxLevels];         // 1: every row of the finer level is a child of exactly one row
-    // A P with the level-1 aggregates (SELL-64 like the face matrix), refilled
-    // every solve from the face matrix through the gather lists
+    // A P with the level-1 aggregates lev[1].agg and agg2 (see AmgLevel; SELL-64
+    // like the face matrix), refilled every solve from the face matrix through
+    // the gather lists (~pos: half the entry).  Once the smoother weight is
+    // known the PCG-precision copy (FP64: ap64 itself) becomes the
+    // post-smoothing operator M0 = P - w D^-1 A P
+    const int *agg2;
+    const int *ap_slice;            // slice of each group of 64 slots
     const long long *ap_slice_ptr;
     const int *ap_col, *ap_src_ptr, *ap_src;
     long long ap_slots, ap_nsrc;
@@ -248,12 +256,14 @@ hipError_t launch_resnorm(hipStream_t st, const DevTopo &T, int nrhs, const doub
 // Multigrid: per-solve set-up (Galerkin products, diagonals, coarsest inverses)
 // and the preconditioned iteration pieces.
 // Once the smoother weights are known (after launch_amg_setup): the up-sweep
-// operator M = P - w D^-1 T of each smoothed transfer, and (after it) the value
-// blocks of the one-workgroup tail in the PCG's precision.
+// operator M = P - w D^-1 T of each smoothed transfer, and (after it, on every
+// solve) the level-0 operator M0 and the value blocks of the one-workgroup tail
+// in the PCG's precision.
 hipError_t launch_amg_combine(hipStream_t st, const DevAmg &A, bool mixed);
-hipError_t launch_amg_tail_pack(hipStream_t st, const DevAmg &A, bool mixed);
-hipError_t launch_amg_setup(hipStream_t st, const DevTopo &T, const DevAmg &A, const double *val64,
-                            bool mixed, const double *elem64 = nullptr, bool ap_only = false);
+hipError_t launch_amg_ready(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype,
+                            const double *dinv0, bool mixed);
+hipError_t launch_amg_setup(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype,
+                            const double *val64, bool mixed, const double *elem64 = nullptr, bool ap_only = false);
 // Lanczos on D^-1/2 A_l D^-1/2 (FP64) for the Jacobi weight of level l:
 // start vector w with |w|^2 partials; one step v = scale w, y = D^-1/2 A
 // D^-1/2 v with <v, y> partials; w = y - a v - b vp with |w|^2 partials.
@@ -269,7 +279,7 @@ hipError_t launch_lanczos_update(hipStream_t st, int n, const double *y, const d
 template <typename VT>
 hipError_t launch_sweep0(hipStream_t st, const DevTopo &T, int nrhs, const VT *val0, const VT *dinv0, const VT *b,
                          const VT *x, VT *xo, double w, DevRed R);
-// The fused post-smoothing sweep alone (z from x0, res0 and the level-1
+// The fused post-smoothing sweep alone (z from r, res0 and the level-1
 // correction of the last V-cycle; the autotuner times it).
 template <typename VT>
 hipError_t launch_post0(hipStream_t st, const DevTopo &T, const DevAmg &A, int nrhs, const VT *dinv0,
@@ -278,10 +288,10 @@ hipError_t launch_post0(hipStream_t st, const DevTopo &T, const DevAmg &A, int n
 // level-0 pre-smoothing residual run element by element; r64 is the FP64
 // accumulator of the fused residual replacement (FP32 iteration).
 template <typename VT>
-hipError_t launch_vcycle(hipStream_t st, const DevTopo &T, const DevAmg &A, int nrhs, const VT *val0,
-                         const VT *dinv0, const VT *r, VT *z, DevRed R, const DevEbe *E = nullptr);
+hipError_t launch_vcycle(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype, int nrhs,
+                         const VT *val0, const VT *dinv0, const VT *r, VT *z, DevRed R, const DevEbe *E = nullptr);
 template <typename MT, typename VT>
-hipError_t launch_pcg_iteration_amg(hipStream_t st, const DevTopo &T, const DevAmg &A, int nrhs,
+hipError_t launch_pcg_iteration_amg(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype, int nrhs,
                                     const MT *val, const VT *dinv, VT *x, VT *r, VT *p, VT *q, VT *z,
                                     DevRed R, DevScal S, const double *val64, const double *b,
                                     double *x64, double tol2, const DevEbe *E = nullptr,
@@ -289,7 +299,8 @@ hipError_t launch_pcg_iteration_amg(hipStream_t st, const DevTopo &T, const DevA
 // z = M^-1 r, rz, p = z (start of the preconditioned iteration after
 // launch_pcg_start64 / launch_reliable(init)).
 template <typename VT>
-hipError_t launch_amg_start(hipStream_t st, const DevTopo &T, const DevAmg &A, int nrhs, const VT *val0,
+hipError_t launch_amg_start(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype, int nrhs,
+                            const VT *val0,
                             const VT *dinv0, const VT *r, VT *z, VT *p, DevRed R, DevScal S,
                             double *x64, VT *x, const DevEbe *E = nullptr);
 

@@ -1254,7 +1254,15 @@ __device__ __forceinline__ void group_sum(VT (&acc)[NRHS]) {
         for (int k = 0; k < NRHS; ++k) acc[k] += __shfl_xor(acc[k], m, G);
 }
 
-// Galerkin product A_c = P' A P with piecewise-constant P: every coarse entry
+// Value of a list entry: position p, or half the value at ~p (a face between
+// two aggregates counts half in each).
+template <typename VT>
+__device__ __forceinline__ VT listed(const VT *__restrict__ v, int p) {
+    const VT x = v[p < 0 ? ~p : p];
+    return p < 0 ? VT(0.5) * x : x;
+}
+
+// Galerkin product A_c = P' A P with piecewise-constant or averaging P: every coarse entry
 // is the sum of the finer entries listed for it (no atomics),
 // out[e] = sum of fine[src[k]] over the gather list of entry e, G lanes per
 // entry (coalesced list reads, several gathers in flight per lane).
@@ -1273,14 +1281,57 @@ __global__ __launch_bounds__(256) void k_galerkin(int nnz, const int *__restrict
     for (int k = src_ptr[e] + sub; k < k1; k += G * KC) {
         int q[KC];
 #pragma unroll
-        for (int u = 0; u < KC; ++u) q[u] = k + G * u < k1 ? src[k + G * u] : -1;
+        for (int u = 0; u < KC; ++u) q[u] = k + G * u < k1 ? src[k + G * u] : 0;
 #pragma unroll
-        for (int u = 0; u < KC; ++u) s[0] += q[u] >= 0 ? fine[q[u]] : 0.0;
+        for (int u = 0; u < KC; ++u)
+            if (k + G * u < k1) s[0] += listed(fine, q[u]);
     }
     group_sum<G>(s);
     if (sub != 0) return;
     out64[e] = s[0];
     if (out32) out32[e] = (float)s[0];
+}
+
+// A P, one lane per slot: the slot's list of face-matrix (or element) values,
+// zero on Dirichlet rows (the cycle leaves them out: their residual is zero).
+// ~2.7 list entries per slot, so one lane each keeps the loads coalesced.
+__global__ __launch_bounds__(256) void k_ap_fill(long long slots, const int *__restrict__ slot_slice,
+                                                 const int *__restrict__ dof_hf, const uint8_t *__restrict__ ftype,
+                                                 const int *__restrict__ src_ptr, const int *__restrict__ src,
+                                                 const double *__restrict__ fine, double *__restrict__ out) {
+    const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (q >= slots) return;
+    const int f = slot_slice[q >> 6] * 64 + (int)(q & 63), h = dof_hf[f];
+    const int k0 = src_ptr[q], k1 = src_ptr[q + 1];
+    double s = 0.0;
+    for (int k = k0; k < k1; k += 4) {
+        int p[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) p[u] = k + u < k1 ? src[k + u] : 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (k + u < k1) s += listed(fine, p[u]);
+    }
+    out[q] = h >= 0 && ftype[h] == FT_DIRICHLET ? 0.0 : s;
+}
+
+// The post-smoothing operator M0 = P - w D^-1 A P on A P's pattern (which
+// holds P's: every row holds its diagonal; empty slots are padding), zero on
+// Dirichlet rows.  ap and out may be the same array (FP64).
+template <typename VT>
+__global__ __launch_bounds__(256) void k_ap_m0(long long slots, const int *__restrict__ slot_slice,
+                                               const int *__restrict__ dof_hf, const uint8_t *__restrict__ ftype,
+                                               const int *__restrict__ src_ptr, const int *__restrict__ col,
+                                               const int *__restrict__ agg, const int *__restrict__ agg2,
+                                               const double *__restrict__ dinv, double w, const double *ap, VT *out) {
+    const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (q >= slots) return;
+    const int f = slot_slice[q >> 6] * 64 + (int)(q & 63), h = dof_hf[f];
+    const int J = col[q], g = agg[f], g2 = agg2[f];
+    double v = 0.0;
+    if (src_ptr[q + 1] > src_ptr[q] && h >= 0 && ftype[h] != FT_DIRICHLET)
+        v = (J == g || J == g2 ? (g2 >= 0 ? 0.5 : 1.0) : 0.0) - w * dinv[f] * ap[q];
+    out[q] = (VT)v;
 }
 
 __global__ __launch_bounds__(256) void k_coarse_diag(int n, const int *__restrict__ diag,
@@ -1494,7 +1545,7 @@ __device__ __forceinline__ void row_up1(const DevAmgLevel &F, const VT *__restri
     group_sum<G>(acc);
 }
 
-// acc = sum over the children of coarse row I of res.
+// acc = sum over the children of coarse row I of res (half of it for children ~f).
 template <typename VT, int NRHS, int G = 1>
 __device__ __forceinline__ void row_restrict(const int *__restrict__ child_ptr, const int *__restrict__ child,
                                              const VT *__restrict__ res, int I, VT (&acc)[NRHS], int sub = 0) {
@@ -1505,12 +1556,15 @@ __device__ __forceinline__ void row_restrict(const int *__restrict__ child_ptr, 
     for (int base = child_ptr[I] + sub; base < e1; base += G * KC) {
         int c[KC];
 #pragma unroll
-        for (int u = 0; u < KC; ++u) c[u] = base + G * u < e1 ? child[base + G * u] : -1;
+        for (int u = 0; u < KC; ++u) c[u] = base + G * u < e1 ? child[base + G * u] : 0;
         VT r[KC][NRHS];
 #pragma unroll
-        for (int u = 0; u < KC; ++u)
+        for (int u = 0; u < KC; ++u) {
+            const VT wgt = base + G * u < e1 ? (c[u] < 0 ? VT(0.5) : VT(1)) : VT(0);
 #pragma unroll
-            for (int k = 0; k < NRHS; ++k) r[u][k] = c[u] >= 0 ? res[(size_t)c[u] * NRHS + k] : VT(0);
+            for (int k = 0; k < NRHS; ++k)
+                r[u][k] = base + G * u < e1 ? wgt * res[(size_t)(c[u] < 0 ? ~c[u] : c[u]) * NRHS + k] : VT(0);
+        }
 #pragma unroll
         for (int u = 0; u < KC; ++u)
 #pragma unroll
@@ -1726,15 +1780,16 @@ __device__ __forceinline__ void ap_row(const int *__restrict__ col, const VT *__
 }
 
 // Post-smoothing sweep after the coarse correction without reading A: with
-// x~ = x0 + alpha P xc and A x0 = r - res0 (from the pre-smoothing pass),
-//   z = x~ + w D^-1 (r - A x~) = x~ + w D^-1 (res0 - alpha (A P) xc),
-// where A P (fine rows x level-1 aggregates, a few entries per row) is
-// refilled every solve.  Also the <r, z> partials of the preconditioned CG.
+// x0 = w D^-1 r, x~ = x0 + P xc and A x0 = r - res0 (from the pre-smoothing pass),
+//   z = x~ + w D^-1 (r - A x~) = w D^-1 (r + res0) + (P - w D^-1 A P) xc,
+// one matrix M0 = P - w D^-1 A P (fine rows x level-1 aggregates, a few entries
+// per row), refilled every solve.  Also the <r, z> partials of the
+// preconditioned CG.  HBM bound: M0 once, r, res0 and D^-1 in, z out.
 template <typename VT, int NRHS, int TB>
 __global__ __launch_bounds__(TB) void k_vc0_post(Gate gt, DevTopo T, const long long *__restrict__ ap_ptr,
-                                                 const int *__restrict__ ap_col, const VT *__restrict__ ap,
-                                                 const int *__restrict__ agg, const VT *__restrict__ dinv,
-                                                 const VT *__restrict__ r, const VT *__restrict__ x0,
+                                                 const int *__restrict__ ap_col, const VT *__restrict__ m0,
+                                                 const VT *__restrict__ dinv,
+                                                 const VT *__restrict__ r,
                                                  const VT *__restrict__ res0, const VT *__restrict__ xc,
                                                  VT *__restrict__ z, VT w, VT al, DevRed R) {
     const int blk = T.sweep_xcd ? xcd_block(gridDim.x) : (int)blockIdx.x;
@@ -1753,15 +1808,13 @@ __global__ __launch_bounds__(TB) void k_vc0_post(Gate gt, DevTopo T, const long 
         // hexahedral grid) unroll to immediate load offsets
         with_ap_width(wd, [&](auto wc) {
             constexpr int W = decltype(wc)::value;
-            ap_row<VT, NRHS, W>(ap_col + s0 + lane, ap + s0 + lane, wd, xc, acc);
+            ap_row<VT, NRHS, W>(ap_col + s0 + lane, m0 + s0 + lane, wd, xc, acc);
         });
-        const int g = agg[f];
         const VT d = w * dinv[f];
 #pragma unroll
         for (int k = 0; k < NRHS; ++k) {
             const size_t i = (size_t)f * NRHS + k;
-            const VT xt = x0[i] + (g >= 0 ? al * xc[(size_t)g * NRHS + k] : VT(0));
-            const VT out = xt + d * (res0[i] - al * acc[k]);
+            const VT out = d * (r[i] + res0[i]) + al * acc[k];
             z[i] = out;
             part[k] += (double)r[i] * (double)out;
         }
@@ -1917,17 +1970,25 @@ __global__ __launch_bounds__(256) void k_scale0(Gate gt, const int *__restrict__
     for (int k = 0; k < NRHS; ++k) x0[(size_t)f * NRHS + k] = d * r[(size_t)f * NRHS + k];
 }
 
-// x~ = x + alpha P xc on level 0 (padding rows have no aggregate)
+// x~ = x + alpha P xc on level 0 (padding rows have no aggregate, Dirichlet
+// rows are left out)
 template <typename VT, int NRHS>
-__global__ __launch_bounds__(256) void k_prolong0(const int *__restrict__ agg, const VT *__restrict__ x,
-                                                  const VT *__restrict__ xc, VT *__restrict__ xo,
-                                                  VT alpha) {
+__global__ __launch_bounds__(256) void k_prolong0(const int *__restrict__ agg, const int *__restrict__ agg2,
+                                                  const int *__restrict__ dof_hf, const uint8_t *__restrict__ ftype,
+                                                  const VT *__restrict__ x, const VT *__restrict__ xc,
+                                                  VT *__restrict__ xo, VT alpha) {
     const int f = blockIdx.x * 256 + threadIdx.x;
-    const int g = agg[f];
+    const int g = agg[f], g2 = agg2[f], h = dof_hf[f];
+    const bool in = g >= 0 && h >= 0 && ftype[h] != FT_DIRICHLET;
 #pragma unroll
     for (int k = 0; k < NRHS; ++k) {
         const size_t i = (size_t)f * NRHS + k;
-        xo[i] = x[i] + (g >= 0 ? alpha * xc[(size_t)g * NRHS + k] : VT(0));
+        VT c = VT(0);
+        if (in) {
+            c = xc[(size_t)g * NRHS + k];
+            if (g2 >= 0) c = VT(0.5) * (c + xc[(size_t)g2 * NRHS + k]);
+        }
+        xo[i] = x[i] + alpha * c;
     }
 }
 
@@ -2139,7 +2200,7 @@ __global__ __launch_bounds__(1024) void k_vcycle_tail(Gate gt, const int *__rest
                                                       const uint16_t *__restrict__ idx,
                                                       const VT *__restrict__ vals, int L, int lt, int vbase,
                                                       int xbase, const VT *__restrict__ gb, VT *__restrict__ gx,
-                                                      VT al, VT als, const int *__restrict__ fagg,
+                                                      VT alf, VT ald, int lsa, VT als, const int *__restrict__ fagg,
                                                       VT *__restrict__ xf) {
     extern __shared__ __align__(16) unsigned char tail_lds[];
     uint16_t *ix = reinterpret_cast<uint16_t *>(tail_lds);
@@ -2232,6 +2293,7 @@ __global__ __launch_bounds__(1024) void k_vcycle_tail(Gate gt, const int *__rest
         const bool sa = t[TL_NPT] != 0;
         if (!sa) {
             const uint16_t *agg = ix + t[TL_AGG];
+            const VT al = l < lsa ? alf : ald;
             for (int q = tid; q < n * NRHS; q += 1024) x[q] += al * xc[agg[q / NRHS] * NRHS + q % NRHS];
             __syncthreads();
         }
@@ -2253,6 +2315,7 @@ __global__ __launch_bounds__(1024) void k_vcycle_tail(Gate gt, const int *__rest
         __syncthreads();
     }
     for (int i = tid; i < n0 * NRHS; i += 1024) gx[(size_t)T0[TL_R0] * NRHS + i] = xc[i];
+    const VT al = lt - 1 < lsa ? alf : ald;
 #pragma unroll
     for (int u = 0; u < PF; ++u) {
         const int f = tid + 1024 * u;
@@ -3258,18 +3321,15 @@ hipError_t launch_resnorm(hipStream_t st, const DevTopo &T, int nrhs, const doub
 }
 
 
-hipError_t launch_amg_setup(hipStream_t st, const DevTopo &T, const DevAmg &A, const double *val64,
-                            bool mixed, const double *elem64, bool ap_only) {
+hipError_t launch_amg_setup(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype,
+                            const double *val64, bool mixed, const double *elem64, bool ap_only) {
     // A P of the level-1 aggregates first: level 1's Galerkin sums its slots.
     // elem64: from the FP64 element values (no face matrix filled)
     if (A.ap_slots > 0) {
         const bool el = elem64 != nullptr;
-        const int *sp = el ? A.ap_esrc_ptr : A.ap_src_ptr, *sl = el ? A.ap_esrc : A.ap_src;
-        with_lanes(lanes_per_row(el ? A.ap_ensrc : A.ap_nsrc, (int)A.ap_slots), [&](auto g) {
-            constexpr int Gv = decltype(g)::value;
-            k_galerkin<Gv><<<row_blocks((int)A.ap_slots, Gv), 256, 0, st>>>(
-                (int)A.ap_slots, sp, sl, el ? elem64 : val64, A.ap64, mixed ? A.ap32 : nullptr);
-        });
+        k_ap_fill<<<(unsigned)((A.ap_slots + 255) / 256), 256, 0, st>>>(
+            A.ap_slots, A.ap_slice, T.dof_hf, ftype, el ? A.ap_esrc_ptr : A.ap_src_ptr, el ? A.ap_esrc : A.ap_src,
+            el ? elem64 : val64, A.ap64);
     }
     if (ap_only) return hipGetLastError();   // the coarse levels are kept
     for (int l = 1; l < A.nlev; ++l) {
@@ -3337,9 +3397,21 @@ static void tail_pack(hipStream_t st, const DevAmg &A, VT *out, const VT *cinv) 
     }
     k_tail_pack<VT><<<dim3(A.ninst, 4, A.nlev - A.tail_first), 256, 0, st>>>(P);
 }
-hipError_t launch_amg_tail_pack(hipStream_t st, const DevAmg &A, bool mixed) {
-    if (mixed) tail_pack<float>(st, A, A.tail_val32, A.cinv32);
-    else tail_pack<double>(st, A, A.tail_val64, A.cinv64);
+hipError_t launch_amg_ready(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype,
+                            const double *dinv0, bool mixed) {
+    const unsigned nb = (unsigned)((A.ap_slots + 255) / 256);
+    auto m0 = [&](auto *out) {
+        if (nb)
+            k_ap_m0<<<nb, 256, 0, st>>>(A.ap_slots, A.ap_slice, T.dof_hf, ftype, A.ap_src_ptr, A.ap_col, A.lev[1].agg,
+                                        A.agg2, dinv0, A.omega_l[0], A.ap64, out);
+    };
+    if (mixed) {
+        m0(A.ap32);
+        tail_pack<float>(st, A, A.tail_val32, A.cinv32);
+    } else {
+        m0(A.ap64);
+        tail_pack<double>(st, A, A.tail_val64, A.cinv64);
+    }
     return hipGetLastError();
 }
 
@@ -3372,14 +3444,13 @@ hipError_t launch_lanczos_update(hipStream_t st, int n, const double *y, const d
 // The fused post-smoothing sweep (k_vc0_post) in the tuned workgroup shape.
 template <typename VT, int NR>
 static void post0(hipStream_t st, const Gate &gt, const DevTopo &T, const DevAmg &A, const VT *dinv0, const VT *r,
-                  const VT *x0,
                   const VT *res0, const VT *xc, VT *z, VT w, VT al, DevRed R) {
     const VT *ap;
     if constexpr (std::is_same<VT, float>::value) ap = A.ap32; else ap = A.ap64;
     with_tb(T.sweep_tb, [&](auto tb) {
         constexpr int TBv = decltype(tb)::value;
-        k_vc0_post<VT, NR, TBv><<<T.nblk, TBv, 0, st>>>(gt, T, A.ap_slice_ptr, A.ap_col, ap, A.lev[1].agg, dinv0, r,
-                                                        x0, res0, xc, z, w, al, R);
+        k_vc0_post<VT, NR, TBv><<<T.nblk, TBv, 0, st>>>(gt, T, A.ap_slice_ptr, A.ap_col, ap, dinv0, r, res0, xc, z, w,
+                                                        al, R);
     });
 }
 
@@ -3388,8 +3459,8 @@ hipError_t launch_post0(hipStream_t st, const DevTopo &T, const DevAmg &A, int n
                         const VT *r, VT *z, DevRed R) {
     return with_nrhs(nrhs, [&](auto nr) {
         constexpr int NR = decltype(nr)::value;
-        post0<VT, NR>(st, Gate{}, T, A, dinv0, r, (const VT *)A.x0, (const VT *)A.res0, (const VT *)A.lev[1].x, z,
-                      (VT)A.omega_l[0], (VT)A.alpha, R);
+        post0<VT, NR>(st, Gate{}, T, A, dinv0, r, (const VT *)A.res0, (const VT *)A.lev[1].x, z, (VT)A.omega_l[0],
+                      (VT)A.alpha_sa, R);
     });
 }
 template hipError_t launch_post0<double>(hipStream_t, const DevTopo &, const DevAmg &, int, const double *,
@@ -3429,10 +3500,16 @@ static inline bool tail_fits(const DevAmg &A, int lt) {
 // short for a gate to pay for its extra memory round trip: they run on, on
 // values nothing reads.
 template <typename VT, int NR>
-static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const DevAmg &A, const VT *val0,
-                        const VT *dinv0, const VT *r, VT *z, DevRed R, bool x0_ready,
+static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const DevAmg &A, const uint8_t *ftype,
+                        const VT *val0, const VT *dinv0, const VT *r, VT *z, DevRed R, bool x0_ready,
                         const DevEbe *E = nullptr) {
-    const VT w = (VT)A.omega_l[0], al = (VT)A.alpha;   // w: level 0
+    const VT w = (VT)A.omega_l[0];   // level 0
+    // over-correction of the tentative transfer from level l + 1 to level l:
+    // weaker above the smoothed transfer (see DevAmg)
+    int lsa = 1;
+    while (lsa < A.nlev && !A.lev[lsa].sa_out) ++lsa;
+    if (lsa == A.nlev) lsa = 1;
+    auto alw = [&](int l) { return (VT)(l < lsa ? A.alpha_f : A.alpha); };
     auto wl = [&](int l) { return (VT)A.omega_l[l]; };
     const int nu = A.nu < 1 ? 1 : A.nu;
     const int rows_blocks = T.nfp / 256;
@@ -3461,7 +3538,7 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
     }
     {
         const DevAmgLevel &C = A.lev[1];
-        with_lanes(lanes_per_row(T.nfp, C.n), [&](auto g) {
+        with_lanes(lanes_per_row((long long)C.nchild, C.n), [&](auto g) {
             constexpr int Gv = decltype(g)::value;
             k_restrict<VT, NR, Gv><<<row_blocks(C.n, Gv), 256, 0, st>>>(C.n, C.child_ptr, C.child, res0,
                                                                        (VT *)C.b);
@@ -3528,7 +3605,8 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
         (void)lds_ok;   // where it is refused, a launch that needs it reports its own error
         const int vbase = tail_vbase(A, lt), xbase = tail_xbase<VT>(A, lt);
         k_vcycle_tail<VT, NR><<<A.ninst, 1024, (unsigned)tail_bytes<VT, NR>(A, lt), st>>>(
-            gt, A.tail_tab, A.tail_idx, tv, L, lt, vbase, xbase, (const VT *)A.lev[lt].b, (VT *)A.lev[lt].x, al, als,
+            gt, A.tail_tab, A.tail_idx, tv, L, lt, vbase, xbase, (const VT *)A.lev[lt].b, (VT *)A.lev[lt].x, alw(0),
+            (VT)A.alpha, lsa, als,
             A.lev[lt].agg, fuse[lt] ? (VT *)A.lev[lt - 1].x : nullptr);
         VT *xres[kMaxLevels];   // each level's result after its up-sweep
         xres[lt] = (VT *)A.lev[lt].x;
@@ -3541,7 +3619,7 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
                     constexpr int Gv = decltype(g)::value;
                     if (xf)
                         k_vcc_up_sa<VT, NR, Gv, true><<<row_blocks(F.n, Gv), 256, 0, st>>>(F, xc, wl(l), als, xf,
-                                                                                          al);
+                                                                                          alw(l - 1));
                     else
                         k_vcc_up_sa<VT, NR, Gv, false><<<row_blocks(F.n, Gv), 256, 0, st>>>(F, xc, wl(l), als,
                                                                                            nullptr, VT(0));
@@ -3553,17 +3631,17 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
                     constexpr int Gv = decltype(g)::value;
                     if (xf)
                         k_vcc_up_plain<VT, NR, Gv, true><<<row_blocks(F.n, Gv), 256, 0, st>>>(
-                            F, (const VT *)F.x, (VT *)F.xt, xf, wl(l), al);
+                            F, (const VT *)F.x, (VT *)F.xt, xf, wl(l), alw(l - 1));
                     else
                         k_vcc_up_plain<VT, NR, Gv, false><<<row_blocks(F.n, Gv), 256, 0, st>>>(
-                            F, (const VT *)F.x, (VT *)F.xt, nullptr, wl(l), al);
+                            F, (const VT *)F.x, (VT *)F.xt, nullptr, wl(l), VT(0));
                 });
                 xres[l] = (VT *)F.xt;
             } else {
                 with_lanes(lanes_per_row(F.nnz, F.n), [&](auto g) {
                     constexpr int Gv = decltype(g)::value;
                     k_vcc_up1<VT, NR, Gv><<<row_blocks(F.n, Gv), 256, 0, st>>>(F, A.lev[l + 1].agg, xc, (VT *)F.x,
-                                                                             wl(l), al);
+                                                                             wl(l), alw(l));
                 });
                 xres[l] = (VT *)F.x;
             }
@@ -3600,7 +3678,7 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
             const DevAmgLevel &F = A.lev[l];
             const unsigned nb = (F.n + 255) / 256;
             if (nu == 1) {
-                k_vcc_up1<VT, NR><<<nb, 256, 0, st>>>(F, A.lev[l + 1].agg, xcur[l + 1], xalt[l], wl(l), al);
+                k_vcc_up1<VT, NR><<<nb, 256, 0, st>>>(F, A.lev[l + 1].agg, xcur[l + 1], xalt[l], wl(l), alw(l));
                 std::swap(xcur[l], xalt[l]);
                 continue;
             }
@@ -3611,7 +3689,7 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
                                                      VT(0));
             } else {
                 k_vcc_up<VT, NR><<<nb, 256, 0, st>>>(F, A.lev[l + 1].agg, (const VT *)F.b, xcur[l],
-                                                     xcur[l + 1], xalt[l], wl(l), al);
+                                                     xcur[l + 1], xalt[l], wl(l), alw(l));
             }
             std::swap(xcur[l], xalt[l]);
             for (int it = 1; it < nu; ++it) {
@@ -3623,10 +3701,11 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
     }
     // ---- level 0 up: x~ = x0 + alpha P x1, then nu sweeps; the last writes z and <r, z>
     if (nu == 1) {
-        post0<VT, NR>(st, gt, T, A, dinv0, r, x0, res0, xcur[1], z, w, al, R);
+        post0<VT, NR>(st, gt, T, A, dinv0, r, res0, xcur[1], z, w, (VT)A.alpha_sa, R);
         return;
     }
-    k_prolong0<VT, NR><<<rows_blocks, 256, 0, st>>>(A.lev[1].agg, x0, xcur[1], xt0, al);
+    k_prolong0<VT, NR><<<rows_blocks, 256, 0, st>>>(A.lev[1].agg, A.agg2, T.dof_hf, ftype, x0, xcur[1], xt0,
+                                                   (VT)A.alpha_sa);
     std::swap(x0, xt0);
     for (int it = 1; it < nu; ++it) {
         sweep0<VT, NR, false>(st, T, val0, dinv0, r, x0, xt0, w, R);
@@ -3649,16 +3728,16 @@ template hipError_t launch_sweep0<float>(hipStream_t, const DevTopo &, int, cons
                                          const float *, const float *, float *, double, DevRed);
 
 template <typename VT>
-hipError_t launch_vcycle(hipStream_t st, const DevTopo &T, const DevAmg &A, int nrhs, const VT *val0,
-                         const VT *dinv0, const VT *r, VT *z, DevRed R, const DevEbe *E) {
+hipError_t launch_vcycle(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype, int nrhs,
+                         const VT *val0, const VT *dinv0, const VT *r, VT *z, DevRed R, const DevEbe *E) {
     return with_nrhs(nrhs, [&](auto nr) {
         constexpr int NR = decltype(nr)::value;
-        vcycle_impl<VT, NR>(st, Gate{}, T, A, val0, dinv0, r, z, R, false, E);
+        vcycle_impl<VT, NR>(st, Gate{}, T, A, ftype, val0, dinv0, r, z, R, false, E);
     });
 }
-template hipError_t launch_vcycle<double>(hipStream_t, const DevTopo &, const DevAmg &, int, const double *,
+template hipError_t launch_vcycle<double>(hipStream_t, const DevTopo &, const DevAmg &, const uint8_t *, int, const double *,
                                           const double *, const double *, double *, DevRed, const DevEbe *);
-template hipError_t launch_vcycle<float>(hipStream_t, const DevTopo &, const DevAmg &, int, const float *,
+template hipError_t launch_vcycle<float>(hipStream_t, const DevTopo &, const DevAmg &, const uint8_t *, int, const float *,
                                          const float *, const float *, float *, DevRed, const DevEbe *);
 
 hipError_t launch_ebe_spmv(hipStream_t st, int maxn, int nrhs, const DevEbe &E, const float *p, float *q,
@@ -3670,7 +3749,7 @@ hipError_t launch_ebe_spmv(hipStream_t st, int maxn, int nrhs, const DevEbe &E, 
 }
 
 template <typename MT, typename VT>
-hipError_t launch_pcg_iteration_amg(hipStream_t st, const DevTopo &T, const DevAmg &A, int nrhs,
+hipError_t launch_pcg_iteration_amg(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype, int nrhs,
                                     const MT *val, const VT *dinv, VT *x, VT *r, VT *p, VT *q, VT *z,
                                     DevRed R, DevScal S, const double *val64, const double *b,
                                     double *x64, double tol2, const DevEbe *E, double *r64) {
@@ -3701,37 +3780,38 @@ hipError_t launch_pcg_iteration_amg(hipStream_t st, const DevTopo &T, const DevA
         // the V-cycle's <r, z> partials after update_xr's: one finisher for both
         DevRed Rz = R;
         Rz.partials += (size_t)2 * NR * R.nblk;
-        vcycle_impl<VT, NR>(st, Gate{S.act}, T, A, val, dinv, r, z, Rz, true, E);
+        vcycle_impl<VT, NR>(st, Gate{S.act}, T, A, ftype, val, dinv, r, z, Rz, true, E);
         k_finish<3 * NR, FinXRZ<NR>><<<T.ninst, 256, 0, st>>>(R, S, Af);
         k_update_pz<VT, NR><<<T.nblk, 256, 0, st>>>(T, z, p, x, REL ? x64 : nullptr, S);
     });
 }
 template hipError_t launch_pcg_iteration_amg<double, double>(hipStream_t, const DevTopo &, const DevAmg &,
-                                                             int, const double *, const double *, double *,
+                                                             const uint8_t *, int, const double *, const double *, double *,
                                                              double *, double *, double *, double *, DevRed,
                                                              DevScal, const double *, const double *,
                                                              double *, double, const DevEbe *, double *);
-template hipError_t launch_pcg_iteration_amg<float, float>(hipStream_t, const DevTopo &, const DevAmg &, int,
+template hipError_t launch_pcg_iteration_amg<float, float>(hipStream_t, const DevTopo &, const DevAmg &, const uint8_t *, int,
                                                            const float *, const float *, float *, float *,
                                                            float *, float *, float *, DevRed, DevScal,
                                                            const double *, const double *, double *, double,
                                                            const DevEbe *, double *);
 
 template <typename VT>
-hipError_t launch_amg_start(hipStream_t st, const DevTopo &T, const DevAmg &A, int nrhs, const VT *val0,
+hipError_t launch_amg_start(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype, int nrhs,
+                            const VT *val0,
                             const VT *dinv0, const VT *r, VT *z, VT *p, DevRed R, DevScal S,
                             double *x64, VT *x, const DevEbe *E) {
     return with_nrhs(nrhs, [&](auto nr) {
         constexpr int NR = decltype(nr)::value;
-        vcycle_impl<VT, NR>(st, Gate{}, T, A, val0, dinv0, r, z, R, false, E);
+        vcycle_impl<VT, NR>(st, Gate{}, T, A, ftype, val0, dinv0, r, z, R, false, E);
         k_finish<NR, FinRZ<NR>><<<T.ninst, 256, 0, st>>>(R, S, FinArgs{0.0, 1});
         k_update_pz<VT, NR><<<T.nblk, 256, 0, st>>>(T, z, p, x, nullptr, S);
     });
 }
-template hipError_t launch_amg_start<double>(hipStream_t, const DevTopo &, const DevAmg &, int, const double *,
+template hipError_t launch_amg_start<double>(hipStream_t, const DevTopo &, const DevAmg &, const uint8_t *, int, const double *,
                                              const double *, const double *, double *, double *, DevRed,
                                              DevScal, double *, double *, const DevEbe *);
-template hipError_t launch_amg_start<float>(hipStream_t, const DevTopo &, const DevAmg &, int, const float *,
+template hipError_t launch_amg_start<float>(hipStream_t, const DevTopo &, const DevAmg &, const uint8_t *, int, const float *,
                                             const float *, const float *, float *, float *, DevRed, DevScal,
                                             double *, float *, const DevEbe *);
 

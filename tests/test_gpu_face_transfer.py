@@ -1,0 +1,67 @@
+"""The averaging transfer between the faces and the first coarse level against the
+oracle: Dirichlet rows left out of the cycle also where the solver type starts
+from zero, several sweeps, periodic pairs, and blocks one cell thick."""
+import numpy as np
+import pytest
+
+import cases
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("kw", [dict(linsolver_type=0, precond=1), dict(smooth_steps=2),
+                                dict(linsolver_type=0, precond=1, element_operator=2)])
+@pytest.mark.parametrize("dims", [(2, 2, 2), (7, 1, 5), (13, 10, 6)])
+def test_dirichlet_rows_and_sweeps(pkg, orc, dims, kw, precision):
+    g = pkg.grids.cartesian(*dims, 1.0, 1.0, 0.5)
+    nc = g.num_cells
+    perm = pkg.fields.perm_c1(nc, 8)
+    bt, bv = cases.xdrop_bc(g, 3.0, 1.0)
+    tm, rm = cases.unit_fluid(nc)
+    s = pkg.HybridSolver(0)
+    s.init(g, perm, (0, 0, 0), bt, None)
+    s.solve(tm, rm, np.zeros(nc), bt, bv, residual_tolerance=1e-12, precision=precision, **kw)
+    p, _, v = s.getSolution()
+    ref = orc.solve(g, perm, tm, rm, np.zeros(nc), bt, bv, tol=1e-14)
+    # solves to 1e-12 of systems with condition numbers below 1e4
+    assert cases.rel_err(p, ref.cell_pressure) < 1e-8
+    assert cases.rel_err(v, ref.outflux) < 1e-8
+
+
+@pytest.mark.parametrize("dims", [(4, 4, 4), (9, 6, 5)])
+def test_periodic_pairs(pkg, orc, dims):
+    g = pkg.grids.cartesian(*dims)
+    nc = g.num_cells
+    perm = pkg.fields.perm_c1(nc, 9)
+    bt, bv, partner = cases.periodic_bc(g)
+    tm, rm = cases.unit_fluid(nc)
+    s = pkg.HybridSolver(0)
+    s.init(g, perm, (0, 0, 0), bt, partner)
+    s.solve(tm, rm, np.zeros(nc), bt, bv, residual_tolerance=1e-12)
+    ref = orc.solve(g, perm, tm, rm, np.zeros(nc), bt, bv, partner=partner, tol=1e-14)
+    assert cases.rel_err(s.getSolution()[2], ref.outflux) < 1e-8
+
+
+def test_smoother_weights_of_a_batch(pkg, orc):
+    """Every level's weight of two unlike instances in one handle is the smaller
+    of theirs alone (the largest eigenvalue of a block-diagonal operator)."""
+    gs = [pkg.grids.cartesian(12, 9, 7), pkg.grids.cartesian(10, 10, 10, 1.0, 1.0, 0.4)]
+    perms = [pkg.fields.perm_c1(g.num_cells, 30 + t) for t, g in enumerate(gs)]
+    G, icp = pkg.grids.concat(gs)
+    bt, bv = cases.xdrop_bc(G)
+    s = pkg.HybridSolver(0)
+    s.init(G, np.concatenate(perms), (0, 0, 0), bt, None, inst_cellpos=icp)
+    tm, rm = cases.unit_fluid(G.num_cells)
+    s.solve(tm, rm, np.zeros(G.num_cells), bt, bv, residual_tolerance=1e-8)
+    w = s.report.as_dict()["smoother_weights"][0]
+    alone = []
+    for g, perm in zip(gs, perms):
+        b, v = cases.xdrop_bc(g)
+        q = pkg.HybridSolver(0)
+        q.init(g, perm, (0, 0, 0), b, None)
+        tm, rm = cases.unit_fluid(g.num_cells)
+        q.solve(tm, rm, np.zeros(g.num_cells), b, v, residual_tolerance=1e-8)
+        alone.append(q.report.as_dict()["smoother_weights"][0])
+    # 12 Lanczos steps come within a few percent of the eigenvalue from below
+    assert 0.97 * min(alone) <= w <= 1.05 * min(alone), (w, alone)
