@@ -136,6 +136,7 @@ struct mhs_solver {
     std::vector<double> rho;            // largest eigenvalue of D^-1 A per level (empty: not estimated)
     long long rho_gen = -1;             // permeability generation the estimate was made for
     bool rho_aniso = false;             // ... and whether that solve had tensor mobilities
+    double *lz[7] = {};                 // work arrays of that estimate (in amg_bufs, from the first one on)
     double *z64 = nullptr;
     float *z32 = nullptr;
 
@@ -224,6 +225,7 @@ T *dupload(mhs_solver *s, std::vector<DevBuf> &list, const std::vector<T> &v, hi
 void mhs_solver::free_amg() {
     for (auto &b : amg_bufs) (void)hipFree(b.p);
     amg_bufs.clear();
+    std::fill(lz, lz + 7, nullptr);
     amg_planned = false;
     dA = DevAmg{};
     setup_gen = -1;
@@ -1042,63 +1044,34 @@ double tridiag_max_eig(const std::vector<double> &a, const std::vector<double> &
 
 // rho(D^-1 A) of every smoothed level (0 .. nlev-2): the largest Ritz value
 // of 12 Lanczos steps on D^-1/2 A D^-1/2 (FP64, from a fixed pseudo-random
-// start), which approaches rho from below.  Done once per hierarchy.
+// start), which approaches rho from below.  Done once per permeability, with
+// work arrays kept with the hierarchy.
 int estimate_rho(mhs_solver *s) {
-    constexpr int kSteps = 12;
     if (const int rm = ensure_matrix(s)) return rm;
     const DevAmg &A = s->dA;
     const int nl = A.nlev - 1;
-    size_t nmax = (size_t)s->T.nfp;
-    for (int l = 1; l < nl; ++l) nmax = std::max(nmax, (size_t)A.lev[l].n);
-    std::vector<DevBuf> tmp;
-    struct Release {
-        std::vector<DevBuf> &t;
-        ~Release() { for (auto &b : t) (void)hipFree(b.p); }
-    } release{tmp};
-    hipError_t he = hipSuccess;
-    double *w = dalloc<double>(s, tmp, nmax, &he);
-    double *V[2] = {nullptr, nullptr}, *u = nullptr, *y = nullptr, *part = nullptr;
-    if (he == hipSuccess) V[0] = dalloc<double>(s, tmp, nmax, &he);
-    if (he == hipSuccess) V[1] = dalloc<double>(s, tmp, nmax, &he);
-    if (he == hipSuccess) u = dalloc<double>(s, tmp, nmax, &he);
-    if (he == hipSuccess) y = dalloc<double>(s, tmp, nmax, &he);
-    if (he == hipSuccess) part = dalloc<double>(s, tmp, nmax / 256 + 1, &he);
-    if (he != hipSuccess) return fail(s, MHS_ERR_ALLOC, std::string("smoother weights: ") + hipGetErrorString(he));
-    std::vector<double> hp(nmax / 256 + 1);
+    if (!s->lz[0]) {
+        const size_t n = lanczos_rows(s->dT, A), sizes[7] = {n, n, n, n, n, lanczos_parts(s->dT, A),
+                                                             (size_t)kLzState * kMaxLevels};
+        hipError_t he = hipSuccess;
+        for (int i = 6; i >= 0 && he == hipSuccess; --i) s->lz[i] = dalloc<double>(s, s->amg_bufs, sizes[i], &he);
+        if (he != hipSuccess) {
+            s->lz[0] = nullptr;
+            return fail(s, MHS_ERR_ALLOC, std::string("smoother weights: ") + hipGetErrorString(he));
+        }
+    }
+    HIPCHECK(launch_lanczos(s->stream, s->dT, A, s->val64, s->dinv64, s->lz[0], s->lz[1], s->lz[2], s->lz[3], s->lz[4],
+                            s->lz[5], s->lz[6]));
+    std::vector<double> st((size_t)kLzState * kMaxLevels);
+    HIPCHECK(hipMemcpyAsync(st.data(), s->lz[6], st.size() * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+    HIPCHECK(hipStreamSynchronize(s->stream));
     std::vector<double> rho(nl, 0.0);
     for (int l = 0; l < nl; ++l) {
-        const int n = l == 0 ? s->T.nfp : A.lev[l].n;
-        const size_t nb = ((size_t)n + 255) / 256;
-        if (n == 0) continue;
-        auto total = [&](double *out) -> int {
-            HIPCHECK(hipMemcpyAsync(hp.data(), part, nb * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-            HIPCHECK(hipStreamSynchronize(s->stream));
-            double t = 0.0;
-            for (size_t i = 0; i < nb; ++i) t += hp[i];
-            *out = t;
-            return MHS_OK;
-        };
-        double ww = 0.0;
-        HIPCHECK(launch_lanczos_init(s->stream, n, w, part));
-        if (int rc = total(&ww)) return rc;
-        double beta = std::sqrt(ww);
-        std::vector<double> al, be;
-        for (int j = 0; j < kSteps && beta > 0.0; ++j) {
-            HIPCHECK(launch_lanczos_step(s->stream, s->dT, A, l, s->val64, s->dinv64, w, 1.0 / beta, V[j & 1], u,
-                                         y, part));
-            double a = 0.0;
-            if (int rc = total(&a)) return rc;
-            al.push_back(a);
-            HIPCHECK(launch_lanczos_update(s->stream, n, y, V[j & 1], j ? V[(j + 1) & 1] : nullptr, a, beta, w,
-                                           part));
-            if (int rc = total(&ww)) return rc;
-            const double bn = std::sqrt(ww);
-            if (!(bn > 1e-12 * std::fabs(a))) break;   // invariant subspace found
-            if (j + 1 < kSteps) be.push_back(bn);
-            beta = bn;
-        }
-        be.resize(al.empty() ? 0 : al.size() - 1);
-        rho[l] = al.empty() ? 0.0 : tridiag_max_eig(al, be);
+        const double *S = &st[(size_t)l * kLzState];
+        const int n = l == 0 ? s->T.nfp : A.lev[l].n, k = n > 0 ? (int)S[LZ_COUNT] : 0;
+        if (k == 0) continue;
+        rho[l] = tridiag_max_eig(std::vector<double>(S + LZ_A, S + LZ_A + k),
+                                 std::vector<double>(S + LZ_B, S + LZ_B + k - 1));
     }
     s->rho = rho;
     return MHS_OK;

@@ -264,16 +264,17 @@ hipError_t launch_amg_ready(hipStream_t st, const DevTopo &T, const DevAmg &A, c
                             const double *dinv0, bool mixed);
 hipError_t launch_amg_setup(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype,
                             const double *val64, bool mixed, const double *elem64 = nullptr, bool ap_only = false);
-// Lanczos on D^-1/2 A_l D^-1/2 (FP64) for the Jacobi weight of level l:
-// start vector w with |w|^2 partials; one step v = scale w, y = D^-1/2 A
-// D^-1/2 v with <v, y> partials; w = y - a v - b vp with |w|^2 partials.
-// Partials: one per 256 rows (level 0: T.nfp rows, else A.lev[l].n).
-hipError_t launch_lanczos_init(hipStream_t st, int n, double *w, double *part);
-hipError_t launch_lanczos_step(hipStream_t st, const DevTopo &T, const DevAmg &A, int level, const double *val0,
-                               const double *dinv0, const double *w, double scale, double *v, double *u,
-                               double *y, double *part);
-hipError_t launch_lanczos_update(hipStream_t st, int n, const double *y, const double *v, const double *vp,
-                                 double a, double b, double *w, double *part);
+// Lanczos steps on D^-1/2 A_l D^-1/2 (FP64) of every smoothed level at once, for
+// the Jacobi weights: all launches on the stream, the scalars stay on the
+// device.  w, v0, v1, u, y: lanczos_rows() doubles each, part: lanczos_parts();
+// state: kLzState doubles per level, on return [LZ_COUNT] coefficients, the
+// diagonal from LZ_A and the off-diagonal from LZ_B.
+constexpr int kLzSteps = 12;
+enum { LZ_BETA = 0, LZ_DONE, LZ_COUNT, LZ_A, LZ_B = LZ_A + kLzSteps, kLzState = 32 };
+size_t lanczos_rows(const DevTopo &T, const DevAmg &A);
+size_t lanczos_parts(const DevTopo &T, const DevAmg &A);
+hipError_t launch_lanczos(hipStream_t st, const DevTopo &T, const DevAmg &A, const double *val0, const double *dinv0,
+                          double *w, double *v0, double *v1, double *u, double *y, double *part, double *state);
 // One level-0 Jacobi sweep with the <b, xo> partials (the last multigrid
 // smoothing sweep alone; the autotuner times it).
 template <typename VT>

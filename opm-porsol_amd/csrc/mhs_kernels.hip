@@ -22,6 +22,7 @@
 #include "mhs_structure.h"
 #include "mhs_amg.h"
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -2891,11 +2892,31 @@ struct FinRes {
 };
 
 // ---------------------------------------------------------------------------
-// Lanczos steps on M = D^-1/2 A D^-1/2 of one multigrid level (FP64), for the
-// largest eigenvalue of D^-1 A that sets the level's Jacobi weight.  Each
-// kernel writes one partial sum per 256-row workgroup, summed on the host.
+// Lanczos steps on M = D^-1/2 A D^-1/2 of every smoothed multigrid level (FP64),
+// for the largest eigenvalue of D^-1 A that sets the level's Jacobi weight.
+// The levels share every launch and the scalars stay in the per-level state, so
+// the 12 steps are 62 launches back to back with one read by the host at the
+// end; level by level with a host sum after each reduction they were about 150
+// launches with 100 synchronisations.  Latency bound.
+struct LzLevels {
+    int nl;
+    int n[kMaxLevels];                // rows (level 0: the padded face rows)
+    int off[kMaxLevels];              // first row in the concatenated vectors
+    int vblk[kMaxLevels + 1];         // first workgroup of each level: 256 rows each,
+    int mblk[kMaxLevels + 1];         // and in the product 256 / g rows each
+    int g[kMaxLevels];                // lanes per row of the product
+    const int *row_ptr[kMaxLevels], *col[kMaxLevels];
+    const double *val[kMaxLevels], *dinv[kMaxLevels];
+    double *state;
+};
+__device__ __forceinline__ int lz_level(const int *blk, int nl) {
+    int l = 0;
+    while (l + 1 < nl && (int)blockIdx.x >= blk[l + 1]) ++l;
+    return l;
+}
 
-__device__ __forceinline__ void block_sum256(double v, double *out) {
+// One partial sum per workgroup.
+__device__ __forceinline__ void lz_partial(double v, double *out) {
     __shared__ double red[4];
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
@@ -2905,73 +2926,106 @@ __device__ __forceinline__ void block_sum256(double v, double *out) {
 }
 
 // w = a fixed pseudo-random start vector in [-1, 1); partials of |w|^2
-__global__ __launch_bounds__(256) void k_lz_init(int n, double *__restrict__ w, double *__restrict__ part) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(256) void k_lz_init(LzLevels Z, double *__restrict__ w, double *__restrict__ part) {
+    const int l = lz_level(Z.vblk, Z.nl), i = (blockIdx.x - Z.vblk[l]) * 256 + threadIdx.x;
     double t = 0.0;
-    if (i < n) {
+    if (i < Z.n[l]) {
         unsigned h = (unsigned)i * 2654435761u;
         h ^= h >> 16;
         h *= 2246822519u;
         h ^= h >> 13;
         const double v = (double)h * (2.0 / 4294967296.0) - 1.0;
-        w[i] = v;
+        w[Z.off[l] + i] = v;
         t = v * v;
     }
-    block_sum256(t, part);
+    lz_partial(t, part);
 }
 
-// v = scale w, u = D^-1/2 v
-__global__ __launch_bounds__(256) void k_lz_prep(int n, const double *__restrict__ dinv,
-                                                 const double *__restrict__ w, double scale,
-                                                 double *__restrict__ v, double *__restrict__ u) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const double vi = w[i] * scale;
-    v[i] = vi;
-    u[i] = sqrt(dinv[i]) * vi;
+// The level's sum (one workgroup per level) and the scalar step it feeds.
+// what: 0 |w|^2 of the start, 1 a = <v, y>, 2 |w|^2 after step j.
+__global__ __launch_bounds__(256) void k_lz_scalar(LzLevels Z, const double *__restrict__ part, int what, int j) {
+    const int l = blockIdx.x;
+    double *S = Z.state + l * kLzState;
+    if (what != 0 && S[LZ_DONE] != 0.0) return;
+    const int *blk = what == 1 ? Z.mblk : Z.vblk;
+    double t = 0.0;
+    for (int i = blk[l] + threadIdx.x; i < blk[l + 1]; i += 256) t += part[i];
+    __shared__ double red[4];
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) t += __shfl_xor(t, m, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    t = (red[0] + red[1]) + (red[2] + red[3]);
+    if (what == 0) {
+        S[LZ_BETA] = sqrt(t);
+        S[LZ_COUNT] = 0.0;
+        S[LZ_DONE] = t > 0.0 ? 0.0 : 1.0;
+    } else if (what == 1) {
+        S[LZ_A + j] = t;
+        S[LZ_COUNT] = j + 1.0;
+    } else {
+        const double bn = sqrt(t);
+        S[LZ_B + j] = bn;
+        S[LZ_BETA] = bn;
+        if (!(bn > 1e-12 * fabs(S[LZ_A + j]))) S[LZ_DONE] = 1.0;   // invariant subspace found
+    }
 }
 
-// y = D^-1/2 A u on the face matrix; partials of <v, y>
-__global__ __launch_bounds__(256) void k_lz_sell(DevTopo T, const double *__restrict__ val,
-                                                 const double *__restrict__ dinv, const double *__restrict__ u,
-                                                 const double *__restrict__ v, double *__restrict__ y,
-                                                 double *__restrict__ part) {
-    const int f = blockIdx.x * 256 + threadIdx.x;   // T.nfp is a multiple of 256
-    double acc[1];
-    sell_row<double, double, double, 1>(T, val, u, f, acc);
-    const double yi = sqrt(dinv[f]) * acc[0];
-    y[f] = yi;
-    block_sum256(v[f] * yi, part);
+// v = w / beta, u = D^-1/2 v
+__global__ __launch_bounds__(256) void k_lz_prep(LzLevels Z, const double *__restrict__ w, double *__restrict__ v,
+                                                 double *__restrict__ u) {
+    const int l = lz_level(Z.vblk, Z.nl), i = (blockIdx.x - Z.vblk[l]) * 256 + threadIdx.x;
+    const double *S = Z.state + l * kLzState;
+    if (i >= Z.n[l] || S[LZ_DONE] != 0.0) return;
+    const double vi = w[Z.off[l] + i] / S[LZ_BETA];
+    v[Z.off[l] + i] = vi;
+    u[Z.off[l] + i] = sqrt(Z.dinv[l][i]) * vi;
 }
 
-// y = D^-1/2 A u on a coarse (CSR) level; partials of <v, y>
-__global__ __launch_bounds__(256) void k_lz_csr(DevAmgLevel L, const double *__restrict__ u,
+// y = D^-1/2 A u (SELL on the face level, CSR rows shared by g lanes below);
+// partials of <v, y>
+__global__ __launch_bounds__(256) void k_lz_mul(LzLevels Z, DevTopo T, const double *__restrict__ u,
                                                 const double *__restrict__ v, double *__restrict__ y,
                                                 double *__restrict__ part) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    double t = 0.0;
-    if (i < L.n) {
-        double acc = 0.0;
-        for (int e = L.row_ptr[i]; e < L.row_ptr[i + 1]; ++e) acc += L.val64[e] * u[L.col[e]];
-        const double yi = sqrt(L.dinv64[i]) * acc;
-        y[i] = yi;
-        t = v[i] * yi;
+    const int l = lz_level(Z.mblk, Z.nl), t = (blockIdx.x - Z.mblk[l]) * 256 + threadIdx.x;
+    if (Z.state[l * kLzState + LZ_DONE] != 0.0) return;
+    const int g = Z.g[l], i = t / g, sub = t % g, o = Z.off[l];
+    double yi = 0.0, s = 0.0;
+    if (i < Z.n[l]) {
+        if (l == 0) {
+            double acc[1];
+            sell_row<double, double, double, 1>(T, Z.val[0], u, i, acc);
+            yi = acc[0];
+        } else {
+            const int e1 = Z.row_ptr[l][i + 1];
+            for (int e = Z.row_ptr[l][i] + sub; e < e1; e += g) yi += Z.val[l][e] * u[o + Z.col[l][e]];
+        }
     }
-    block_sum256(t, part);
+    for (int m = g >> 1; m >= 1; m >>= 1) yi += __shfl_xor(yi, m, 64);
+    if (i < Z.n[l] && sub == 0) {
+        yi *= sqrt(Z.dinv[l][i]);
+        y[o + i] = yi;
+        s = v[o + i] * yi;
+    }
+    lz_partial(s, part);
 }
 
-// w = y - a v - b vp (vp null: first step); partials of |w|^2
-__global__ __launch_bounds__(256) void k_lz_update(int n, const double *__restrict__ y, const double *__restrict__ v,
-                                                   const double *__restrict__ vp, double a, double b,
+// w = y - a v - beta vp (first: no vp); partials of |w|^2
+__global__ __launch_bounds__(256) void k_lz_update(LzLevels Z, int j, const double *__restrict__ y,
+                                                   const double *__restrict__ v, const double *__restrict__ vp,
                                                    double *__restrict__ w, double *__restrict__ part) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int l = lz_level(Z.vblk, Z.nl), i = (blockIdx.x - Z.vblk[l]) * 256 + threadIdx.x;
+    const double *S = Z.state + l * kLzState;
+    if (S[LZ_DONE] != 0.0) return;
     double t = 0.0;
-    if (i < n) {
-        const double wi = y[i] - a * v[i] - (vp ? b * vp[i] : 0.0);
-        w[i] = wi;
+    if (i < Z.n[l]) {
+        const int q = Z.off[l] + i;
+        const double wi = y[q] - S[LZ_A + j] * v[q] - (j ? S[LZ_BETA] * vp[q] : 0.0);
+        w[q] = wi;
         t = wi * wi;
     }
-    block_sum256(t, part);
+    lz_partial(t, part);
 }
 
 // gterm[h] = omega[c] * (x_f - x_c) . g, one half-face per thread
@@ -3415,29 +3469,48 @@ hipError_t launch_amg_ready(hipStream_t st, const DevTopo &T, const DevAmg &A, c
     return hipGetLastError();
 }
 
-static inline unsigned lz_blocks(int n) { return (unsigned)((n + 255) / 256); }
-
-hipError_t launch_lanczos_init(hipStream_t st, int n, double *w, double *part) {
-    k_lz_init<<<lz_blocks(n), 256, 0, st>>>(n, w, part);
-    return hipGetLastError();
+static LzLevels lz_levels(const DevTopo &T, const DevAmg &A, const double *val0, const double *dinv0,
+                          double *state) {
+    LzLevels Z{};
+    Z.nl = A.nlev - 1;
+    Z.state = state;
+    for (int l = 0; l < Z.nl; ++l) {
+        const DevAmgLevel &L = A.lev[l];
+        Z.n[l] = l == 0 ? T.nfp : L.n;
+        Z.g[l] = l == 0 ? 1 : lanes_per_row(L.nnz, L.n);
+        Z.row_ptr[l] = L.row_ptr;
+        Z.col[l] = L.col;
+        Z.val[l] = l == 0 ? val0 : L.val64;
+        Z.dinv[l] = l == 0 ? dinv0 : L.dinv64;
+        Z.off[l] = l == 0 ? 0 : Z.off[l - 1] + Z.n[l - 1];
+        Z.vblk[l + 1] = Z.vblk[l] + (int)row_blocks(Z.n[l], 1);
+        Z.mblk[l + 1] = Z.mblk[l] + (int)row_blocks(Z.n[l], Z.g[l]);
+    }
+    return Z;
 }
-
-hipError_t launch_lanczos_step(hipStream_t st, const DevTopo &T, const DevAmg &A, int level, const double *val0,
-                               const double *dinv0, const double *w, double scale, double *v, double *u,
-                               double *y, double *part) {
-    const int n = level == 0 ? T.nfp : A.lev[level].n;
-    const double *dinv = level == 0 ? dinv0 : A.lev[level].dinv64;
-    k_lz_prep<<<lz_blocks(n), 256, 0, st>>>(n, dinv, w, scale, v, u);
-    if (level == 0)
-        k_lz_sell<<<lz_blocks(n), 256, 0, st>>>(T, val0, dinv, u, v, y, part);
-    else
-        k_lz_csr<<<lz_blocks(n), 256, 0, st>>>(A.lev[level], u, v, y, part);
-    return hipGetLastError();
+size_t lanczos_rows(const DevTopo &T, const DevAmg &A) {
+    const LzLevels Z = lz_levels(T, A, nullptr, nullptr, nullptr);
+    return Z.nl ? (size_t)Z.off[Z.nl - 1] + Z.n[Z.nl - 1] : 0;
 }
-
-hipError_t launch_lanczos_update(hipStream_t st, int n, const double *y, const double *v, const double *vp,
-                                 double a, double b, double *w, double *part) {
-    k_lz_update<<<lz_blocks(n), 256, 0, st>>>(n, y, v, vp, a, b, w, part);
+size_t lanczos_parts(const DevTopo &T, const DevAmg &A) {
+    const LzLevels Z = lz_levels(T, A, nullptr, nullptr, nullptr);
+    return (size_t)std::max(Z.vblk[Z.nl], Z.mblk[Z.nl]);
+}
+hipError_t launch_lanczos(hipStream_t st, const DevTopo &T, const DevAmg &A, const double *val0, const double *dinv0,
+                          double *w, double *v0, double *v1, double *u, double *y, double *part, double *state) {
+    const LzLevels Z = lz_levels(T, A, val0, dinv0, state);
+    const int nv = Z.vblk[Z.nl], nm = Z.mblk[Z.nl];
+    if (Z.nl < 1 || nv == 0) return hipSuccess;
+    k_lz_init<<<nv, 256, 0, st>>>(Z, w, part);
+    k_lz_scalar<<<Z.nl, 256, 0, st>>>(Z, part, 0, 0);
+    for (int j = 0; j < kLzSteps; ++j) {
+        double *v = j & 1 ? v1 : v0, *vp = j & 1 ? v0 : v1;
+        k_lz_prep<<<nv, 256, 0, st>>>(Z, w, v, u);
+        k_lz_mul<<<nm, 256, 0, st>>>(Z, T, u, v, y, part);
+        k_lz_scalar<<<Z.nl, 256, 0, st>>>(Z, part, 1, j);
+        k_lz_update<<<nv, 256, 0, st>>>(Z, j, y, v, vp, w, part);
+        k_lz_scalar<<<Z.nl, 256, 0, st>>>(Z, part, 2, j);
+    }
     return hipGetLastError();
 }
 
