@@ -611,6 +611,8 @@ int mhs_init_system_structure(mhs_solver *s, const int *hf_bc_type, const int *h
     d.uniform_ncf = 1;
     for (int c = 0; c < T.nc && d.uniform_ncf; ++c)
         if (T.facepos[c + 1] - T.facepos[c] != T.max_ncf) d.uniform_ncf = 0;
+    d.max_iblk = 0;
+    for (int t = 0; t < T.ninst; ++t) d.max_iblk = std::max(d.max_iblk, T.seg_blk[t + 1] - T.seg_blk[t]);
     d.max_w = 0;
     for (int sl = 0; sl < T.nslices; ++sl)
         d.max_w = std::max(d.max_w, (int)((T.slice_ptr[sl + 1] - T.slice_ptr[sl]) / kSlice));
@@ -645,6 +647,7 @@ int mhs_init_system_structure(mhs_solver *s, const int *hf_bc_type, const int *h
         D = DevEbe{};
         D.ncolours = E.ncolours;
         D.nblk = E.nblk;
+        for (int t = 0; t < T.ninst; ++t) D.max_slots = std::max(D.max_slots, E.inst_slot[t + 1] - E.inst_slot[t]);
         for (int k = 0; k <= E.ncolours; ++k) D.colour_blk[k] = E.colour_blk[k];
         for (int k = 0; k < E.ncolours; ++k) D.colour_split[k] = E.colour_split[k];
         D.blk_info = reinterpret_cast<const int4 *>(dupload(s, L, E.blk_info, &he));
@@ -841,7 +844,7 @@ int ensure_solve_buffers(mhs_solver *s, int nrhs, bool mixed) {
     if (ok()) s->in_bcval = dalloc<double>(s, L, (size_t)nrhs * T.nhf, &e);
     if (ok()) s->ftype = dalloc<uint8_t>(s, L, (size_t)T.nhf, &e);
     if (ok()) s->inst_reg = dalloc<int>(s, L, (size_t)T.ninst, &e);
-    if (ok()) s->R.partials = dalloc<double>(s, L, (size_t)(nfp / kRowBlock) * 16, &e);
+    if (ok()) s->R.partials = dalloc<double>(s, L, (size_t)(nfp / kRowBlock) * 32, &e);
     if (ok()) s->R.counters = dalloc<int>(s, L, (size_t)T.ninst, &e);
     // sc, act, iters and status share one block so that the host reads the
     // solver's progress with a single copy (read_state)
@@ -854,6 +857,12 @@ int ensure_solve_buffers(mhs_solver *s, int nrhs, bool mixed) {
         s->S.status = s->S.iters + nsys;
     }
     if (ok()) s->S.upd = dalloc<int>(s, L, nsys, &e);
+    if (ok()) s->S.sc2 = dalloc<double>(s, L, nsys * SC_N, &e);
+    if (ok()) s->S.act2 = dalloc<int>(s, L, 3 * nsys, &e);
+    if (ok()) {
+        s->S.iters2 = s->S.act2 + nsys;
+        s->S.upd2 = s->S.iters2 + nsys;
+    }
     if (ok()) s->maxbits = dalloc<unsigned long long>(s, L, 1, &e);
     s->z64 = nullptr;
     s->z32 = nullptr;

@@ -16,6 +16,7 @@ struct DevTopo {
     int nc, nhf, nfp, ninst, nslices, nblk;
     int max_w;                      // widest SELL slice (stored entries per row)
     int max_ncf;                    // most faces of a cell (stride of the slot map)
+    int max_iblk;                   // most 1024-row blocks of an instance
     int uniform_ncf;                // 1: every cell has max_ncf faces (per-cell loops of fixed length)
     const int *facepos, *hf_dof, *hf_cell, *hf_col, *hf_ppart, *hf_twin;
     const uint8_t *hf_redirect;
@@ -49,7 +50,7 @@ struct DevCellSys {
 
 // Segmented-reduction workspace shared by all PCG kernels.
 struct DevRed {
-    double *partials;  // [16][nblk]
+    double *partials;  // [32][nblk]: the product's quantities from 0, the updates' from 16
     int nblk;
     int *counters;     // [ninst]
     const int *block_seg, *seg_blk;
@@ -63,6 +64,11 @@ struct DevScal {
     int *iters;        // [nsys]
     int *upd;          // [nsys] 1: FP64 residual replacement due, 2: also restart p
     int *status;       // [4]: 0 nactive, 1 breakdown count
+    // second copy of sc, act, iters and upd: where the finishers are fused into
+    // the vector updates, every workgroup of an instance works out the step
+    // from one copy while its first workgroup writes the result to the other
+    double *sc2;
+    int *act2, *iters2, *upd2;
     int mixed;         // FP32 iteration with FP64 residual replacement
     int amg;           // multigrid preconditioner (z stored, beta from <r, z>)
     double rf2;        // replacement trigger: |r|^2 <= rf2 * |r at last replacement|^2
@@ -88,6 +94,7 @@ __host__ __device__ constexpr long long ebe_slot(int local, int q, int ncomp) {
 }
 struct DevEbe {
     int ncolours = 0, nblk = 0;
+    int max_slots = 0;                      // most partial slots of an instance
     int colour_blk[kEbeColours + 1] = {};
     int colour_split[kEbeColours] = {};     // first block of each colour that is not hexahedra
     // per block: (face count, instance, cells in the block, partial slot) and

@@ -140,9 +140,130 @@ __global__ __launch_bounds__(256) void k_finish(DevRed R, DevScal S, FinArgs A) 
             acc[q] += a[0];
         }
     }
-    __shared__ double lds[4 * NQ];
+    __shared__ double lds[4 * NQ], tot[NQ];
     block_sum256<NQ>(acc, lds);
-    if (threadIdx.x == 0) Fin::run(s, acc, S, A);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) tot[q] = acc[q];
+    __syncthreads();
+    if (threadIdx.x < Fin::nsys) Fin::run(s, threadIdx.x, tot, S, A);
+}
+
+// Where an instance has few partials, its finisher runs inside the kernel that
+// needs the result: every workgroup sums the instance's partials itself, one
+// wavefront per quantity, in the same order, so all of them find the same step.
+// One launch less, each about 4.3 us of waiting for a few dozen numbers.  Above
+// kFuseParts the reads of all workgroups would cost more than the launch.
+constexpr int kFuseParts = 512;
+template <int NQ>
+__device__ __forceinline__ void inst_totals(const DevRed &R, int s, int nq, double (&tot)[NQ]) {
+    const int b0 = R.seg_blk[s], b1 = R.seg_blk[s + 1];
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int q0 = 0; q0 < NQ; q0 += 4) {
+        const int q = q0 + (threadIdx.x >> 6);
+        if (q >= NQ || q >= nq) continue;          // wave-uniform
+        const double *pq = R.partials + (size_t)q * R.nblk;
+        double a[kFuseParts / 64];
+#pragma unroll
+        for (int u = 0; u < kFuseParts / 64; ++u) {
+            const int i = b0 + 64 * u + lane;
+            a[u] = i < b1 ? pq[i] : 0.0;
+        }
+#pragma unroll
+        for (int u = 1; u < kFuseParts / 64; ++u) a[0] += a[u];
+        const double t = wave_sum(a[0]);
+        if (lane == 0) tot[q] = t;
+    }
+    __syncthreads();
+}
+
+// The scalars of one system (see DevScal), and the steps of the CG recurrence on
+// them.  lead: count the system's changes in the status words.
+struct SysState {
+    double sc[SC_N];
+    int act, iters, upd;
+};
+__device__ __forceinline__ SysState load_state(const DevScal &S, int i) {
+    SysState t;
+#pragma unroll
+    for (int e = 0; e < SC_N; ++e) t.sc[e] = S.sc[(size_t)i * SC_N + e];
+    t.act = S.act[i];
+    t.iters = S.iters[i];
+    t.upd = S.upd[i];
+    return t;
+}
+__device__ __forceinline__ void store_state(const DevScal &S, int i, const SysState &t) {
+#pragma unroll
+    for (int e = 0; e < SC_N; ++e) S.sc[(size_t)i * SC_N + e] = t.sc[e];
+    S.act[i] = t.act;
+    S.iters[i] = t.iters;
+    S.upd[i] = t.upd;
+}
+
+// after the product: alpha = rz / <p, Ap>; with REL also the FP64 residual
+// replacement (the true residual decides convergence of the FP32 iteration;
+// rel: |r64|^2, r.M^-1 r and |r|^2 of the replaced residual).
+template <bool REL>
+__device__ __forceinline__ void step_pq(SysState &t, double pq, const double *rel, const DevScal &S, bool lead) {
+    if (!t.act) return;
+    if (REL && t.upd) {
+        const double rrt = rel[0];
+        t.sc[SC_RRT] = rrt;
+        t.sc[SC_RRL] = rrt;
+        if (!S.amg) t.sc[SC_RZ] = rel[1];
+        t.sc[SC_RR] = rel[2];
+        t.upd = 0;
+        if (lead) atomicAdd(&S.status[2], 1);
+        if (rrt <= t.sc[SC_THR]) {
+            t.act = 0;
+            t.sc[SC_ALPHA] = 0.0;
+            if (lead) atomicSub(&S.status[0], 1);
+            return;
+        }
+    }
+    t.sc[SC_PQ] = pq;
+    if (!(pq > 0.0)) {
+        t.sc[SC_ALPHA] = 0.0;
+        if (REL) {          // FP32 breakdown: restart p, then replace the residual
+            t.upd = 2;
+        } else {
+            t.act = 0;
+            if (lead) {
+                atomicSub(&S.status[0], 1);
+                atomicAdd(&S.status[1], 1);
+            }
+        }
+    } else {
+        t.sc[SC_ALPHA] = t.sc[SC_RZ] / pq;
+    }
+}
+
+// after update_xr: convergence test (FP64) or replacement request (FP32), beta
+__device__ __forceinline__ void step_xr(SysState &t, double rz, double rr, const DevScal &S, bool lead) {
+    if (!t.act) return;
+    t.iters += 1;
+    t.sc[SC_RR] = rr;
+    if (S.mixed) {
+        // FP32 recursion: ask for the FP64 true residual once the recursive
+        // one has dropped by replace_factor (or reached the tolerance).
+        if (t.upd == 0 && (rr <= t.sc[SC_THR] || rr <= S.rf2 * t.sc[SC_RRL])) t.upd = 1;
+    } else if (rr <= t.sc[SC_THR]) {
+        t.act = 0;
+        if (lead) atomicSub(&S.status[0], 1);
+        return;
+    }
+    if (!S.amg) {
+        t.sc[SC_BETA] = rz / t.sc[SC_RZ];
+        t.sc[SC_RZ] = rz;
+    }
+}
+
+// after the multigrid V-cycle: beta = <r, z> / <r, z>_old (init: p = z)
+__device__ __forceinline__ void step_rz(SysState &t, double rz, bool init) {
+    if (!t.act) return;
+    t.sc[SC_BETA] = (init || t.upd == 2) ? 0.0 : rz / t.sc[SC_RZ];
+    t.sc[SC_RZ] = rz;
 }
 
 // 16-byte vector access to a thread's contiguous chunk of N elements.
@@ -995,21 +1116,50 @@ __global__ __launch_bounds__(256) void k_ebe(DevEbe E, int blk0, Gate gt, DevSca
     }
 }
 
-template <typename VT, int NRHS>
+// The finisher fused into a vector update of instance s (see inst_totals):
+// sums the nq quantities of R, applies step(state, k, totals) to each system's
+// state from S and, in the instance's first workgroup (lead), stores it in So.
+// st: the new states, for every thread.
+template <int NRHS, int NQ, class Step>
+__device__ __forceinline__ void fused_finish(const DevRed &R, const DevScal &S, const DevScal &So, int s, bool lead,
+                                             int nq, SysState (&st)[NRHS], Step step) {
+    __shared__ double tot[NQ];
+    SysState t;
+    if (threadIdx.x < NRHS) t = load_state(S, s * NRHS + threadIdx.x);
+    inst_totals<NQ>(R, s, nq, tot);
+    if (threadIdx.x < NRHS) {
+        step(t, (int)threadIdx.x, tot);
+        st[threadIdx.x] = t;
+        if (lead) store_state(So, s * NRHS + threadIdx.x, t);
+    }
+    __syncthreads();
+}
+// An instance that has finished: its state still moves to the other copy.
+template <int NRHS>
+__device__ __forceinline__ void pass_state(const DevScal &S, const DevScal &So, int s, bool lead) {
+    if (lead && threadIdx.x < NRHS)
+        store_state(So, s * NRHS + threadIdx.x, load_state(S, s * NRHS + threadIdx.x));
+}
+
+// x += alpha p, r -= alpha q (with x0s also the first multigrid smoothing step
+// x0 = w D^-1 r), and the partials of r.D^-1 r and r.r.  FUSE: alpha from the
+// product's partials in Rq, the state passing from S to So; 2: the FP32
+// iteration, with its residual replacement.
+template <typename VT, int NRHS, int FUSE>
 __global__ __launch_bounds__(256) void k_update_xr(DevTopo T, const VT *__restrict__ dinv,
                                                    VT *__restrict__ x, VT *__restrict__ r,
                                                    const VT *__restrict__ p,
-                                                   const VT *__restrict__ q, DevRed R,
-                                                   DevScal S, VT *__restrict__ x0s = nullptr,
-                                                   VT w = VT(0)) {
+                                                   const VT *__restrict__ q, DevRed Rq, DevRed R,
+                                                   DevScal S, DevScal So, VT *__restrict__ x0s,
+                                                   VT w) {
     const int b = xcd_block(gridDim.x);
     const int s = block_inst(T, b);
+    const bool lead = FUSE && b == T.seg_blk[s];
     int act[NRHS];
-    if (!load_act<NRHS>(S.act, s, act)) return;
-    VT al[NRHS];
-#pragma unroll
-    for (int k = 0; k < NRHS; ++k)
-        al[k] = act[k] ? (VT)S.sc[(size_t)(s * NRHS + k) * SC_N + SC_ALPHA] : VT(0);
+    if (!load_act<NRHS>(S.act, s, act)) {
+        if constexpr (FUSE != 0) pass_state<NRHS>(S, So, s, lead);
+        return;
+    }
     const int f0 = b * kRowBlock + 4 * threadIdx.x;
     const size_t e0 = (size_t)f0 * NRHS;
     VT d[4], xv[4 * NRHS], rv[4 * NRHS], pv[4 * NRHS], qv[4 * NRHS];
@@ -1018,6 +1168,30 @@ __global__ __launch_bounds__(256) void k_update_xr(DevTopo T, const VT *__restri
     vload<VT, 4 * NRHS>(r + e0, rv);
     vload<VT, 4 * NRHS>(p + e0, pv);
     vload<VT, 4 * NRHS>(q + e0, qv);
+    VT al[NRHS];
+    if constexpr (FUSE != 0) {
+        __shared__ SysState st[NRHS];
+        int nq = NRHS;
+        if constexpr (FUSE == 2)
+#pragma unroll
+            for (int k = 0; k < NRHS; ++k)
+                if (act[k] && S.upd[s * NRHS + k]) nq = 4 * NRHS;
+        fused_finish<NRHS, FUSE == 2 ? 4 * NRHS : NRHS>(Rq, S, So, s, lead, nq, st,
+                                                        [&](SysState &t, int k, const double *tot) {
+                                                            step_pq<FUSE == 2>(t, tot[k], tot + NRHS + 3 * k, S, lead);
+                                                        });
+        bool any = false;
+#pragma unroll
+        for (int k = 0; k < NRHS; ++k) {
+            any |= st[k].act != 0;
+            al[k] = st[k].act ? (VT)st[k].sc[SC_ALPHA] : VT(0);
+        }
+        if (!any) return;
+    } else {
+#pragma unroll
+        for (int k = 0; k < NRHS; ++k)
+            al[k] = act[k] ? (VT)S.sc[(size_t)(s * NRHS + k) * SC_N + SC_ALPHA] : VT(0);
+    }
     double part[2 * NRHS];
 #pragma unroll
     for (int k = 0; k < 2 * NRHS; ++k) part[k] = 0.0;
@@ -1033,7 +1207,7 @@ __global__ __launch_bounds__(256) void k_update_xr(DevTopo T, const VT *__restri
         }
     vstore<VT, 4 * NRHS>(x + e0, xv);
     vstore<VT, 4 * NRHS>(r + e0, rv);
-    if (x0s) {  // first multigrid smoothing step, x0 = w D^-1 r
+    if (x0s) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -1043,24 +1217,21 @@ __global__ __launch_bounds__(256) void k_update_xr(DevTopo T, const VT *__restri
     block_partials<2 * NRHS>(part, b, R);
 }
 
-template <typename VT, int NRHS>
+// p = D^-1 r + beta p (beta = 0 on a restart); in FP32 also fold x32 into x64 for
+// systems whose residual replacement is due.  FUSE: beta from update_xr's
+// partials in R, the state passing from S to So.
+template <typename VT, int NRHS, bool FUSE>
 __global__ __launch_bounds__(256) void k_update_p(DevTopo T, const VT *__restrict__ dinv,
                                                   const VT *__restrict__ r,
                                                   VT *__restrict__ p, VT *__restrict__ x,
-                                                  double *__restrict__ x64, DevScal S) {
+                                                  double *__restrict__ x64, DevRed R, DevScal S, DevScal So) {
     const int b = xcd_block(gridDim.x);
     const int s = block_inst(T, b);
+    const bool lead = FUSE && b == T.seg_blk[s];
     int act[NRHS];
-    if (!load_act<NRHS>(S.act, s, act)) return;
-    VT be[NRHS];
-    int u[NRHS];
-    bool any_u = false;
-#pragma unroll
-    for (int k = 0; k < NRHS; ++k) {
-        const int sys = s * NRHS + k;
-        u[k] = (x64 && act[k]) ? S.upd[sys] : 0;
-        any_u |= u[k] != 0;
-        be[k] = (u[k] == 2) ? VT(0) : (VT)S.sc[(size_t)sys * SC_N + SC_BETA];
+    if (!load_act<NRHS>(S.act, s, act)) {
+        if constexpr (FUSE) pass_state<NRHS>(S, So, s, lead);
+        return;
     }
     const int f0 = b * kRowBlock + 4 * threadIdx.x;
     const size_t e0 = (size_t)f0 * NRHS;
@@ -1068,6 +1239,25 @@ __global__ __launch_bounds__(256) void k_update_p(DevTopo T, const VT *__restric
     vload<VT, 4>(dinv + f0, d);
     vload<VT, 4 * NRHS>(r + e0, rv);
     vload<VT, 4 * NRHS>(p + e0, pv);
+    VT be[NRHS];
+    int u[NRHS];
+    bool any_u = false, any = false;
+    __shared__ SysState st[FUSE ? NRHS : 1];
+    if constexpr (FUSE)
+        fused_finish<NRHS, 2 * NRHS>(R, S, So, s, lead, 2 * NRHS, st, [&](SysState &t, int k, const double *tot) {
+            step_xr(t, tot[2 * k], tot[2 * k + 1], S, lead);
+        });
+#pragma unroll
+    for (int k = 0; k < NRHS; ++k) {
+        const int sys = s * NRHS + k;
+        if constexpr (FUSE) act[k] = st[k].act;
+        const int up = FUSE ? st[FUSE ? k : 0].upd : S.upd[sys];
+        u[k] = (x64 && act[k]) ? up : 0;
+        any_u |= u[k] != 0;
+        any |= act[k] != 0;
+        be[k] = (u[k] == 2) ? VT(0) : (VT)(FUSE ? st[FUSE ? k : 0].sc[SC_BETA] : S.sc[(size_t)sys * SC_N + SC_BETA]);
+    }
+    if (FUSE && !any) return;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -1671,16 +1861,13 @@ __device__ __forceinline__ void up_sa_row(const DevAmgLevel &F, const VT *__rest
     }
 }
 
-// Level 0, one more Jacobi sweep: xo = x + w D^-1 (b - A x~), x~ = x + alpha P xc
-// (xc == nullptr: no coarse correction).  With z/partials: the final sweep of
-// the V-cycle writes the preconditioned residual and <r, z> partials.
+// Level 0, one more Jacobi sweep: xo = x + w D^-1 (b - A x).  LAST: the final sweep
+// of the V-cycle writes the preconditioned residual and <r, z> partials.
 template <typename VT, int NRHS, bool LAST, int TB>
 __global__ __launch_bounds__(TB) void k_vc0_up(DevTopo T, const VT *__restrict__ val,
                                                const VT *__restrict__ dinv,
-                                               const int *__restrict__ agg,
                                                const VT *__restrict__ b, const VT *__restrict__ x,
-                                               const VT *__restrict__ xc, VT *__restrict__ xo,
-                                               VT w, VT alpha, DevRed R) {
+                                               VT *__restrict__ xo, VT w, DevRed R) {
     const int blk = T.sweep_xcd ? xcd_block(gridDim.x) : (int)blockIdx.x;
     double part[NRHS];
 #pragma unroll
@@ -1688,36 +1875,13 @@ __global__ __launch_bounds__(TB) void k_vc0_up(DevTopo T, const VT *__restrict__
 #pragma unroll
     for (int j = 0; j < kRowBlock / TB; ++j) {
         const int f = blk * kRowBlock + j * TB + threadIdx.x;
-        const int slice = f >> 6, lane = f & 63;
-        const long long s0 = T.slice_ptr[slice];
-        const int wd = (int)((T.slice_ptr[slice + 1] - s0) >> 6);
         VT acc[NRHS];
-        if (!xc) {
-            sell_row<VT, VT, VT, NRHS>(T, val, x, f, acc);
-        } else {
-#pragma unroll
-            for (int k = 0; k < NRHS; ++k) acc[k] = VT(0);
-            for (int e = 0; e < wd; ++e) {
-                const long long o = s0 + lane + 64LL * e;
-                const int c = __builtin_nontemporal_load(T.col + o);
-                const VT a = __builtin_nontemporal_load(val + o);
-                const int gc = agg[c];
-#pragma unroll
-                for (int k = 0; k < NRHS; ++k) {
-                    VT xv = x[(size_t)c * NRHS + k];
-                    if (gc >= 0) xv += alpha * xc[(size_t)gc * NRHS + k];
-                    acc[k] += a * xv;
-                }
-            }
-        }
+        sell_row<VT, VT, VT, NRHS>(T, val, x, f, acc);
         const VT d = w * dinv[f];
-        const int g = xc ? agg[f] : -1;
 #pragma unroll
         for (int k = 0; k < NRHS; ++k) {
             const size_t i = (size_t)f * NRHS + k;
-            VT xv = x[i];
-            if (g >= 0) xv += alpha * xc[(size_t)g * NRHS + k];
-            const VT out = xv + d * (b[i] - acc[k]);
+            const VT out = x[i] + d * (b[i] - acc[k]);
             xo[i] = out;
             if (LAST) part[k] += (double)b[i] * (double)out;
         }
@@ -2369,30 +2533,45 @@ __global__ __launch_bounds__(256) void k_tail_pack(TailPack<VT> P) {
 }
 
 // p = z + beta p (beta = 0 on a restart); in FP32 also fold x32 into x64 for
-// systems whose residual replacement is due.
-template <typename VT, int NRHS>
+// systems whose residual replacement is due.  FUSE: the step after the V-cycle
+// (FinXRZ) from the partials in R, the state passing from S to So.
+template <typename VT, int NRHS, bool FUSE>
 __global__ __launch_bounds__(256) void k_update_pz(DevTopo T, const VT *__restrict__ z,
                                                    VT *__restrict__ p, VT *__restrict__ x,
-                                                   double *__restrict__ x64, DevScal S) {
+                                                   double *__restrict__ x64, DevRed R, DevScal S, DevScal So) {
     const int b = xcd_block(gridDim.x);
     const int s = block_inst(T, b);
+    const bool lead = FUSE && b == T.seg_blk[s];
     int act[NRHS];
-    if (!load_act<NRHS>(S.act, s, act)) return;
-    VT be[NRHS];
-    int u[NRHS];
-    bool any_u = false;
-#pragma unroll
-    for (int k = 0; k < NRHS; ++k) {
-        const int sys = s * NRHS + k;
-        u[k] = (x64 && act[k]) ? S.upd[sys] : 0;
-        any_u |= u[k] != 0;
-        be[k] = (VT)S.sc[(size_t)sys * SC_N + SC_BETA];
+    if (!load_act<NRHS>(S.act, s, act)) {
+        if constexpr (FUSE) pass_state<NRHS>(S, So, s, lead);
+        return;
     }
     const int f0 = b * kRowBlock + 4 * threadIdx.x;
     const size_t e0 = (size_t)f0 * NRHS;
     VT zv[4 * NRHS], pv[4 * NRHS];
     vload<VT, 4 * NRHS>(z + e0, zv);
     vload<VT, 4 * NRHS>(p + e0, pv);
+    VT be[NRHS];
+    int u[NRHS];
+    bool any_u = false, any = false;
+    __shared__ SysState st[FUSE ? NRHS : 1];
+    if constexpr (FUSE)
+        fused_finish<NRHS, 3 * NRHS>(R, S, So, s, lead, 3 * NRHS, st, [&](SysState &t, int k, const double *tot) {
+            step_xr(t, tot[2 * k], tot[2 * k + 1], S, lead);
+            step_rz(t, tot[2 * NRHS + k], false);
+        });
+#pragma unroll
+    for (int k = 0; k < NRHS; ++k) {
+        const int sys = s * NRHS + k;
+        if constexpr (FUSE) act[k] = st[k].act;
+        const int up = FUSE ? st[FUSE ? k : 0].upd : S.upd[sys];
+        u[k] = (x64 && act[k]) ? up : 0;
+        any_u |= u[k] != 0;
+        any |= act[k] != 0;
+        be[k] = (VT)(FUSE ? st[FUSE ? k : 0].sc[SC_BETA] : S.sc[(size_t)sys * SC_N + SC_BETA]);
+    }
+    if (FUSE && !any) return;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -2705,10 +2884,9 @@ __device__ __forceinline__ bool none_set(const int *flags, int s) {
     return !any;
 }
 
-// after k_spmv_pq: alpha = rz / <p, Ap>; with REL also the FP64 residual
-// replacement (the true residual decides convergence of the FP32 iteration).
 template <int NRHS, bool REL>
 struct FinPQ {
+    static constexpr int nsys = NRHS;
     __device__ static bool skip(int s, const DevScal &S, const FinArgs &) { return none_set<NRHS>(S.act, s); }
     __device__ static int nq(int s, const DevScal &S) {
         if (!REL) return NRHS;
@@ -2717,93 +2895,34 @@ struct FinPQ {
             if (S.act[s * NRHS + k] && S.upd[s * NRHS + k]) return 4 * NRHS;
         return NRHS;
     }
-    __device__ static void run(int s, const double *tot, DevScal &S, const FinArgs &) {
-#pragma unroll
-        for (int k = 0; k < NRHS; ++k) {
-            const int i = s * NRHS + k;
-            if (!S.act[i]) continue;
-            double *sc = S.sc + (size_t)i * SC_N;
-            if (REL && S.upd[i]) {
-                const double rrt = tot[NRHS + 3 * k];
-                sc[SC_RRT] = rrt;
-                sc[SC_RRL] = rrt;
-                if (!S.amg) sc[SC_RZ] = tot[NRHS + 3 * k + 1];
-                sc[SC_RR] = tot[NRHS + 3 * k + 2];
-                S.upd[i] = 0;
-                atomicAdd(&S.status[2], 1);
-                if (rrt <= sc[SC_THR]) {
-                    S.act[i] = 0;
-                    sc[SC_ALPHA] = 0.0;
-                    atomicSub(&S.status[0], 1);
-                    continue;
-                }
-            }
-            const double pq = tot[k];
-            sc[SC_PQ] = pq;
-            if (!(pq > 0.0)) {
-                sc[SC_ALPHA] = 0.0;
-                if (REL) {          // FP32 breakdown: restart p, then replace the residual
-                    S.upd[i] = 2;
-                } else {
-                    S.act[i] = 0;
-                    atomicSub(&S.status[0], 1);
-                    atomicAdd(&S.status[1], 1);
-                }
-            } else {
-                sc[SC_ALPHA] = sc[SC_RZ] / pq;
-            }
-        }
+    __device__ static void run(int s, int k, const double *tot, DevScal &S, const FinArgs &) {
+        SysState t = load_state(S, s * NRHS + k);
+        step_pq<REL>(t, tot[k], tot + NRHS + 3 * k, S, true);
+        store_state(S, s * NRHS + k, t);
     }
 };
 
-// after k_update_xr: convergence test (FP64) or replacement request (FP32), beta
 template <int NRHS>
 struct FinXR {
+    static constexpr int nsys = NRHS;
     __device__ static bool skip(int s, const DevScal &S, const FinArgs &) { return none_set<NRHS>(S.act, s); }
     __device__ static int nq(int, const DevScal &) { return 2 * NRHS; }
-    __device__ static void run(int s, const double *tot, DevScal &S, const FinArgs &) {
-#pragma unroll
-        for (int k = 0; k < NRHS; ++k) {
-            const int i = s * NRHS + k;
-            if (!S.act[i]) continue;
-            double *sc = S.sc + (size_t)i * SC_N;
-            S.iters[i] += 1;
-            const double rz = tot[2 * k], rr = tot[2 * k + 1];
-            sc[SC_RR] = rr;
-            if (S.mixed) {
-                // FP32 recursion: ask for the FP64 true residual once the recursive
-                // one has dropped by replace_factor (or reached the tolerance).
-                if (S.upd[i] == 0 && (rr <= sc[SC_THR] || rr <= S.rf2 * sc[SC_RRL])) S.upd[i] = 1;
-                if (!S.amg) {
-                    sc[SC_BETA] = rz / sc[SC_RZ];
-                    sc[SC_RZ] = rz;
-                }
-            } else if (rr <= sc[SC_THR]) {
-                S.act[i] = 0;
-                atomicSub(&S.status[0], 1);
-            } else if (!S.amg) {
-                sc[SC_BETA] = rz / sc[SC_RZ];
-                sc[SC_RZ] = rz;
-            }
-        }
+    __device__ static void run(int s, int k, const double *tot, DevScal &S, const FinArgs &) {
+        SysState t = load_state(S, s * NRHS + k);
+        step_xr(t, tot[2 * k], tot[2 * k + 1], S, true);
+        store_state(S, s * NRHS + k, t);
     }
 };
 
-// after the multigrid V-cycle: beta = <r, z> / <r, z>_old (init: p = z)
 template <int NRHS>
 struct FinRZ {
+    static constexpr int nsys = NRHS;
     __device__ static bool skip(int s, const DevScal &S, const FinArgs &) { return none_set<NRHS>(S.act, s); }
     __device__ static int nq(int, const DevScal &) { return NRHS; }
-    __device__ static void run(int s, const double *tot, DevScal &S, const FinArgs &A) {
-#pragma unroll
-        for (int k = 0; k < NRHS; ++k) {
-            const int i = s * NRHS + k;
-            if (!S.act[i]) continue;
-            double *sc = S.sc + (size_t)i * SC_N;
-            const double rz = tot[k];
-            sc[SC_BETA] = (A.init || S.upd[i] == 2) ? 0.0 : rz / sc[SC_RZ];
-            sc[SC_RZ] = rz;
-        }
+    __device__ static void run(int s, int k, const double *tot, DevScal &S, const FinArgs &A) {
+        SysState t = load_state(S, s * NRHS + k);
+        step_rz(t, tot[k], A.init);
+        store_state(S, s * NRHS + k, t);
     }
 };
 
@@ -2815,79 +2934,78 @@ struct FinRZ {
 // reads.
 template <int NRHS>
 struct FinXRZ {
+    static constexpr int nsys = NRHS;
     __device__ static bool skip(int s, const DevScal &S, const FinArgs &) { return none_set<NRHS>(S.act, s); }
     __device__ static int nq(int, const DevScal &) { return 3 * NRHS; }
-    __device__ static void run(int s, const double *tot, DevScal &S, const FinArgs &A) {
-        FinXR<NRHS>::run(s, tot, S, A);
-        FinRZ<NRHS>::run(s, tot + 2 * NRHS, S, A);
+    __device__ static void run(int s, int k, const double *tot, DevScal &S, const FinArgs &) {
+        SysState t = load_state(S, s * NRHS + k);
+        step_xr(t, tot[2 * k], tot[2 * k + 1], S, true);
+        step_rz(t, tot[2 * NRHS + k], false);
+        store_state(S, s * NRHS + k, t);
     }
 };
 
 // after k_start64: |r0|, thresholds, activation (dune CGSolver: def0 < 1e-30 -> done)
 template <int NRHS>
 struct FinStart {
+    static constexpr int nsys = NRHS;
     __device__ static bool skip(int, const DevScal &, const FinArgs &) { return false; }
     __device__ static int nq(int, const DevScal &) { return 2 * NRHS; }
-    __device__ static void run(int s, const double *tot, DevScal &S, const FinArgs &A) {
-#pragma unroll
-        for (int k = 0; k < NRHS; ++k) {
-            const int i = s * NRHS + k;
-            double *sc = S.sc + (size_t)i * SC_N;
-            const double rr0 = tot[2 * k + 1];
-            sc[SC_RZ] = tot[2 * k];
-            sc[SC_RR] = rr0;
-            sc[SC_RR0] = rr0;
-            sc[SC_RRT] = rr0;
-            sc[SC_THR] = A.tol2 * rr0;
-            S.iters[i] = 0;
-            const int a = (rr0 >= 1e-60) ? 1 : 0;
-            S.act[i] = a;
-            if (a) atomicAdd(&S.status[0], 1);
-        }
+    __device__ static void run(int s, int k, const double *tot, DevScal &S, const FinArgs &A) {
+        const int i = s * NRHS + k;
+        double *sc = S.sc + (size_t)i * SC_N;
+        const double rr0 = tot[2 * k + 1];
+        sc[SC_RZ] = tot[2 * k];
+        sc[SC_RR] = rr0;
+        sc[SC_RR0] = rr0;
+        sc[SC_RRT] = rr0;
+        sc[SC_THR] = A.tol2 * rr0;
+        S.iters[i] = 0;
+        const int a = (rr0 >= 1e-60) ? 1 : 0;
+        S.act[i] = a;
+        if (a) atomicAdd(&S.status[0], 1);
     }
 };
 
 // after k_reliable: the FP64 true residual decides convergence
 template <int NRHS>
 struct FinRel {
+    static constexpr int nsys = NRHS;
     __device__ static bool skip(int s, const DevScal &S, const FinArgs &A) {
         return !A.init && none_set<NRHS>(S.upd, s);
     }
     __device__ static int nq(int, const DevScal &) { return 3 * NRHS; }
-    __device__ static void run(int s, const double *tot, DevScal &S, const FinArgs &A) {
-#pragma unroll
-        for (int k = 0; k < NRHS; ++k) {
-            const int i = s * NRHS + k;
-            if (!A.init && !S.upd[i]) continue;
-            double *sc = S.sc + (size_t)i * SC_N;
-            const double rrt = tot[3 * k];
-            if (A.init) {
-                sc[SC_RR0] = rrt;
-                sc[SC_THR] = A.tol2 * rrt;
-                S.iters[i] = 0;
-            }
-            sc[SC_RRT] = rrt;
-            sc[SC_RRL] = rrt;
-            sc[SC_RZ] = tot[3 * k + 1];
-            sc[SC_RR] = tot[3 * k + 2];
-            S.upd[i] = 0;
-            if (!A.init) atomicAdd(&S.status[2], 1);
-            const int was = A.init ? 0 : S.act[i];
-            const int now = (rrt <= sc[SC_THR] || sc[SC_RR0] < 1e-60) ? 0 : 1;
-            S.act[i] = now;
-            if (now != was) atomicAdd(&S.status[0], now - was);
+    __device__ static void run(int s, int k, const double *tot, DevScal &S, const FinArgs &A) {
+        const int i = s * NRHS + k;
+        if (!A.init && !S.upd[i]) return;
+        double *sc = S.sc + (size_t)i * SC_N;
+        const double rrt = tot[3 * k];
+        if (A.init) {
+            sc[SC_RR0] = rrt;
+            sc[SC_THR] = A.tol2 * rrt;
+            S.iters[i] = 0;
         }
+        sc[SC_RRT] = rrt;
+        sc[SC_RRL] = rrt;
+        sc[SC_RZ] = tot[3 * k + 1];
+        sc[SC_RR] = tot[3 * k + 2];
+        S.upd[i] = 0;
+        if (!A.init) atomicAdd(&S.status[2], 1);
+        const int was = A.init ? 0 : S.act[i];
+        const int now = (rrt <= sc[SC_THR] || sc[SC_RR0] < 1e-60) ? 0 : 1;
+        S.act[i] = now;
+        if (now != was) atomicAdd(&S.status[0], now - was);
     }
 };
 
 // after k_resnorm
 template <int NRHS>
 struct FinRes {
+    static constexpr int nsys = NRHS;
     __device__ static bool skip(int, const DevScal &, const FinArgs &) { return false; }
     __device__ static int nq(int, const DevScal &) { return NRHS; }
-    __device__ static void run(int s, const double *tot, DevScal &S, const FinArgs &) {
-#pragma unroll
-        for (int k = 0; k < NRHS; ++k) S.sc[(size_t)(s * NRHS + k) * SC_N + SC_RRT] = tot[k];
+    __device__ static void run(int s, int k, const double *tot, DevScal &S, const FinArgs &) {
+        S.sc[(size_t)(s * NRHS + k) * SC_N + SC_RRT] = tot[k];
     }
 };
 
@@ -3259,6 +3377,38 @@ hipError_t launch_fill(hipStream_t st, const DevTopo &T, int nrhs, const DevCell
     });
 }
 
+// Whether every instance has few enough partials for the fused finishers.
+static inline bool fuse_finishers(const DevTopo &T, const DevEbe *E) {
+    return T.max_iblk <= kFuseParts && (!E || E->max_slots <= kFuseParts);
+}
+static inline DevScal other_copy(DevScal S) {
+    std::swap(S.sc, S.sc2);
+    std::swap(S.act, S.act2);
+    std::swap(S.iters, S.iters2);
+    std::swap(S.upd, S.upd2);
+    return S;
+}
+
+// q = A p with the <p, q> partials (in FP32 with the fused residual
+// replacement), element by element when E is given; returns where they are.
+template <typename MT, typename VT, int NR, bool REL>
+static DevRed product(hipStream_t st, const DevTopo &T, const MT *val, const VT *p, VT *q, DevRed R, DevScal S,
+                      const RelArgs &L, const DevEbe *E, double *r64) {
+    if constexpr (REL) {
+        if (E) {
+            ebe_apply<NR, EBE_SPMV, true>(st, T.max_ncf, *E, Gate{S.act}, S, p, q, nullptr, L, r64);
+            return E->R;
+        }
+    }
+    with_tb(T.spmv_tb, [&](auto tb) {
+        constexpr int TBv = decltype(tb)::value;
+        with_chunk(T.max_w, [&](auto ch) {
+            launch_spmv_kernel<MT, VT, NR, REL, TBv, decltype(ch)::value>(st, T.nblk, T, val, p, q, R, S, L);
+        });
+    });
+    return R;
+}
+
 template <typename MT, typename VT>
 hipError_t launch_pcg_iteration(hipStream_t st, const DevTopo &T, int nrhs, const MT *val,
                                 const VT *dinv, VT *x, VT *r, VT *p, VT *q, DevRed R,
@@ -3266,34 +3416,26 @@ hipError_t launch_pcg_iteration(hipStream_t st, const DevTopo &T, int nrhs, cons
                                 double tol2, const DevEbe *E, double *r64) {
     return with_nrhs(nrhs, [&](auto nr) {
         constexpr int NR = decltype(nr)::value;
-        const FinArgs A{tol2, 0};
         constexpr bool REL = std::is_same<VT, float>::value;
-        RelArgs L{};
-        if constexpr (REL) L = RelArgs{val64, x64, b, dinv, r};
-        bool ebe = false;
-        if constexpr (REL) {
-            if (E) {
-                ebe_apply<NR, EBE_SPMV, true>(st, T.max_ncf, *E, Gate{S.act}, S, p, q, nullptr, L, r64);
-                k_finish<4 * NR, FinPQ<NR, true>><<<T.ninst, 256, 0, st>>>(E->R, S, A);
-                ebe = true;
-            }
+        const RelArgs L = REL ? RelArgs{val64, x64, b, (const float *)dinv, (float *)r} : RelArgs{};
+        const FinArgs A{tol2, 0};
+        const bool fuse = fuse_finishers(T, E);
+        const DevRed Rq = product<MT, VT, NR, REL>(st, T, val, p, q, R, S, L, E, r64);
+        DevRed Rx = R;
+        Rx.partials += (size_t)16 * R.nblk;
+        if (fuse) {
+            const DevScal S2 = other_copy(S);
+            k_update_xr<VT, NR, REL ? 2 : 1><<<T.nblk, 256, 0, st>>>(T, dinv, x, r, p, q, Rq, Rx, S, S2, nullptr,
+                                                                   VT(0));
+            k_update_p<VT, NR, true><<<T.nblk, 256, 0, st>>>(T, dinv, r, p, x, REL ? x64 : nullptr, Rx, S2, S);
+            return;
         }
-        if (!ebe) {
-            with_tb(T.spmv_tb, [&](auto tb) {
-                constexpr int TBv = decltype(tb)::value;
-                with_chunk(T.max_w, [&](auto ch) {
-                    launch_spmv_kernel<MT, VT, NR, REL, TBv, decltype(ch)::value>(st, T.nblk, T, val, p, q, R, S,
-                                                                                  L);
-                });
-            });
-            k_finish<REL ? 4 * NR : NR, FinPQ<NR, REL>><<<T.ninst, 256, 0, st>>>(R, S, A);
-        }
-        k_update_xr<VT, NR><<<T.nblk, 256, 0, st>>>(T, dinv, x, r, p, q, R, S);
-        k_finish<2 * NR, FinXR<NR>><<<T.ninst, 256, 0, st>>>(R, S, A);
-        k_update_p<VT, NR><<<T.nblk, 256, 0, st>>>(T, dinv, r, p, x, REL ? x64 : nullptr, S);
+        k_finish<REL ? 4 * NR : NR, FinPQ<NR, REL>><<<T.ninst, 256, 0, st>>>(Rq, S, A);
+        k_update_xr<VT, NR, 0><<<T.nblk, 256, 0, st>>>(T, dinv, x, r, p, q, Rq, Rx, S, S, nullptr, VT(0));
+        k_finish<2 * NR, FinXR<NR>><<<T.ninst, 256, 0, st>>>(Rx, S, A);
+        k_update_p<VT, NR, false><<<T.nblk, 256, 0, st>>>(T, dinv, r, p, x, REL ? x64 : nullptr, Rx, S, S);
     });
 }
-
 template hipError_t launch_pcg_iteration<double, double>(hipStream_t, const DevTopo &, int,
                                                          const double *, const double *,
                                                          double *, double *, double *,
@@ -3548,8 +3690,7 @@ static void sweep0(hipStream_t st, const DevTopo &T, const VT *val0, const VT *d
                    VT *xo, VT w, DevRed R) {
     with_tb(T.sweep_tb, [&](auto tb) {
         constexpr int TBv = decltype(tb)::value;
-        k_vc0_up<VT, NR, LAST, TBv><<<T.nblk, TBv, 0, st>>>(T, val0, dinv0, nullptr, b, x, nullptr, xo, w,
-                                                            VT(0), R);
+        k_vc0_up<VT, NR, LAST, TBv><<<T.nblk, TBv, 0, st>>>(T, val0, dinv0, b, x, xo, w, R);
     });
 }
 
@@ -3830,32 +3971,30 @@ hipError_t launch_pcg_iteration_amg(hipStream_t st, const DevTopo &T, const DevA
         constexpr int NR = decltype(nr)::value;
         const FinArgs Af{tol2, 0};
         constexpr bool REL = std::is_same<VT, float>::value;
-        RelArgs L{};
-        if constexpr (REL) L = RelArgs{val64, x64, b, dinv, r};
-        bool ebe = false;
-        if constexpr (REL) {
-            if (E) {
-                ebe_apply<NR, EBE_SPMV, true>(st, T.max_ncf, *E, Gate{S.act}, S, p, q, nullptr, L, r64);
-                k_finish<4 * NR, FinPQ<NR, true>><<<T.ninst, 256, 0, st>>>(E->R, S, Af);
-                ebe = true;
-            }
-        }
-        if (!ebe) {
-            with_tb(T.spmv_tb, [&](auto tb) {
-                constexpr int TBv = decltype(tb)::value;
-                with_chunk(T.max_w, [&](auto ch) {
-                    launch_spmv_kernel<MT, VT, NR, REL, TBv, decltype(ch)::value>(st, T.nblk, T, val, p, q, R, S, L);
-                });
-            });
-            k_finish<REL ? 4 * NR : NR, FinPQ<NR, REL>><<<T.ninst, 256, 0, st>>>(R, S, Af);
-        }
-        k_update_xr<VT, NR><<<T.nblk, 256, 0, st>>>(T, dinv, x, r, p, q, R, S, (VT *)A.x0, (VT)A.omega_l[0]);
+        const RelArgs L = REL ? RelArgs{val64, x64, b, (const float *)dinv, (float *)r} : RelArgs{};
+        const bool fuse = fuse_finishers(T, E);
+        const DevRed Rq = product<MT, VT, NR, REL>(st, T, val, p, q, R, S, L, E, r64);
+        DevRed Rx = R;
+        Rx.partials += (size_t)16 * R.nblk;
         // the V-cycle's <r, z> partials after update_xr's: one finisher for both
-        DevRed Rz = R;
+        DevRed Rz = Rx;
         Rz.partials += (size_t)2 * NR * R.nblk;
-        vcycle_impl<VT, NR>(st, Gate{S.act}, T, A, ftype, val, dinv, r, z, Rz, true, E);
-        k_finish<3 * NR, FinXRZ<NR>><<<T.ninst, 256, 0, st>>>(R, S, Af);
-        k_update_pz<VT, NR><<<T.nblk, 256, 0, st>>>(T, z, p, x, REL ? x64 : nullptr, S);
+        const DevScal S2 = fuse ? other_copy(S) : S;
+        if (fuse) {
+            k_update_xr<VT, NR, REL ? 2 : 1><<<T.nblk, 256, 0, st>>>(T, dinv, x, r, p, q, Rq, Rx, S, S2, (VT *)A.x0,
+                                                                   (VT)A.omega_l[0]);
+        } else {
+            k_finish<REL ? 4 * NR : NR, FinPQ<NR, REL>><<<T.ninst, 256, 0, st>>>(Rq, S, Af);
+            k_update_xr<VT, NR, 0><<<T.nblk, 256, 0, st>>>(T, dinv, x, r, p, q, Rq, Rx, S, S, (VT *)A.x0,
+                                                           (VT)A.omega_l[0]);
+        }
+        vcycle_impl<VT, NR>(st, Gate{S2.act}, T, A, ftype, val, dinv, r, z, Rz, true, E);
+        if (fuse) {
+            k_update_pz<VT, NR, true><<<T.nblk, 256, 0, st>>>(T, z, p, x, REL ? x64 : nullptr, Rx, S2, S);
+        } else {
+            k_finish<3 * NR, FinXRZ<NR>><<<T.ninst, 256, 0, st>>>(Rx, S, Af);
+            k_update_pz<VT, NR, false><<<T.nblk, 256, 0, st>>>(T, z, p, x, REL ? x64 : nullptr, Rx, S, S);
+        }
     });
 }
 template hipError_t launch_pcg_iteration_amg<double, double>(hipStream_t, const DevTopo &, const DevAmg &,
@@ -3878,7 +4017,7 @@ hipError_t launch_amg_start(hipStream_t st, const DevTopo &T, const DevAmg &A, c
         constexpr int NR = decltype(nr)::value;
         vcycle_impl<VT, NR>(st, Gate{}, T, A, ftype, val0, dinv0, r, z, R, false, E);
         k_finish<NR, FinRZ<NR>><<<T.ninst, 256, 0, st>>>(R, S, FinArgs{0.0, 1});
-        k_update_pz<VT, NR><<<T.nblk, 256, 0, st>>>(T, z, p, x, nullptr, S);
+        k_update_pz<VT, NR, false><<<T.nblk, 256, 0, st>>>(T, z, p, x, nullptr, R, S, S);
     });
 }
 template hipError_t launch_amg_start<double>(hipStream_t, const DevTopo &, const DevAmg &, const uint8_t *, int, const double *,
