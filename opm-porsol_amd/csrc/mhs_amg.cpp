@@ -4,11 +4,101 @@
 #include <algorithm>
 #include <array>
 #include <cmath>
+#include <exception>
 #include <numeric>
+#include <thread>
 
 namespace mhs {
 
 namespace {
+
+// Host threads for the row loops below (each row's lists depend on that row
+// alone): fn(t, begin, end) on contiguous ranges of [0, n), at least `least`
+// items each.  The hierarchy of 128x128x64 cells is 100M list entries.
+constexpr int kMaxThreads = 8;
+int ranges(int n, int least) {
+    const int hw = std::max(1u, std::thread::hardware_concurrency());
+    return std::max(1, std::min({n / std::max(1, least), hw, kMaxThreads}));
+}
+template <class Fn>
+void in_ranges(int n, int nt, Fn fn) {
+    std::vector<std::exception_ptr> err(nt);
+    auto run = [&](int t) {
+        try {
+            fn(t, int((long long)n * t / nt), int((long long)n * (t + 1) / nt));
+        } catch (...) {
+            err[t] = std::current_exception();
+        }
+    };
+    std::vector<std::thread> pool;
+    pool.reserve(nt);
+    int t = 1;
+    try {
+        for (; t < nt; ++t) pool.emplace_back(run, t);
+    } catch (...) {   // no more threads to be had: the rest runs here
+    }
+    run(0);
+    for (int u = t; u < nt; ++u) run(u);
+    for (auto &th : pool) th.join();
+    for (auto &e : err)
+        if (e) std::rethrow_exception(e);
+}
+// Appends the ranges' lists in order; returns where each one starts.
+std::vector<size_t> append(std::vector<int> &out, const std::vector<std::vector<int>> &parts) {
+    std::vector<size_t> at(parts.size() + 1, out.size());
+    for (size_t t = 0; t < parts.size(); ++t) at[t + 1] = at[t] + parts[t].size();
+    out.resize(at.back());
+    in_ranges(int(parts.size()), int(parts.size()), [&](int, int b, int e) {
+        for (int t = b; t < e; ++t) std::copy(parts[t].begin(), parts[t].end(), out.begin() + at[t]);
+    });
+    return at;
+}
+
+// Rows of a CSR pattern whose entries each carry a list, built range by range:
+// row(i, R) appends the row's columns to R.col and, per entry, its sources to
+// R.src (and R.src2) and their end to R.end.
+struct RowPart {
+    std::vector<int> col, src, src2, end, len;
+};
+template <class Row>
+void build_rows(int n, std::vector<int> &ptr, std::vector<int> &col, std::vector<int> &src_ptr, std::vector<int> &src,
+                std::vector<int> *src2, Row row) {
+    const int nt = ranges(n, 2048);
+    std::vector<RowPart> P(nt);
+    in_ranges(n, nt, [&](int t, int b, int e) {
+        RowPart &R = P[t];
+        R.len.reserve(e - b);
+        for (int i = b; i < e; ++i) {
+            const size_t c0 = R.col.size();
+            row(i, R);
+            R.len.push_back(int(R.col.size() - c0));
+        }
+    });
+    ptr.assign(n + 1, 0);
+    std::vector<std::vector<int>> cols(nt), srcs(nt), srcs2(nt), ends(nt);
+    for (int t = 0, i = 0; t < nt; ++t) {
+        for (int l : P[t].len) {
+            ptr[i + 1] = ptr[i] + l;
+            ++i;
+        }
+        cols[t].swap(P[t].col);
+        srcs[t].swap(P[t].src);
+        srcs2[t].swap(P[t].src2);
+        ends[t].swap(P[t].end);
+    }
+    col.clear();
+    src.clear();
+    append(col, cols);
+    const std::vector<size_t> at = append(src, srcs);
+    for (int t = 0; t < nt; ++t)
+        for (int &e : ends[t]) e += int(at[t]);
+    src_ptr.assign(1, 0);
+    append(src_ptr, ends);
+    if (src2) {
+        src2->clear();
+        append(*src2, srcs2);
+    }
+}
 
 void children(AmgLevel &C, int nf) {
     const bool two = !C.agg2.empty();
@@ -27,6 +117,14 @@ void children(AmgLevel &C, int nf) {
     }
 }
 
+// Position of each row's diagonal entry (-1: none).
+void find_diagonal(AmgLevel &C) {
+    C.diag.assign(C.n, -1);
+    for (int I = 0; I < C.n; ++I)
+        for (int e = C.row_ptr[I]; e < C.row_ptr[I + 1]; ++e)
+            if (C.col[e] == I) C.diag[I] = e;
+}
+
 // Sparsity of P'AP and the gather lists, coarse row by coarse row: the
 // entries (agg(j), pos) of the coarse row's children are sorted locally.
 // row_entries(i, emit) must call emit(j, pos) for every stored entry of
@@ -34,13 +132,8 @@ void children(AmgLevel &C, int nf) {
 // those of A P).  Requires children() to have run.
 template <bool COARSE = false, class RowEntries>
 void galerkin_pattern(AmgLevel &C, RowEntries row_entries) {
-    C.row_ptr.assign(C.n + 1, 0);
-    C.col.clear();
-    C.src_ptr.assign(1, 0);
-    C.src.clear();
-    C.diag.assign(C.n, -1);
-    std::vector<std::pair<int, int>> buf;
-    for (int I = 0; I < C.n; ++I) {
+    build_rows(C.n, C.row_ptr, C.col, C.src_ptr, C.src, nullptr, [&](int I, RowPart &R) {
+        thread_local std::vector<std::pair<int, int>> buf;
         buf.clear();
         for (int k = C.child_ptr[I]; k < C.child_ptr[I + 1]; ++k)
             row_entries(C.child[k], [&](int j, int pos) {
@@ -53,66 +146,85 @@ void galerkin_pattern(AmgLevel &C, RowEntries row_entries) {
         });
         for (size_t k = 0; k < buf.size(); ++k) {
             if (k == 0 || buf[k].first != buf[k - 1].first) {
-                if (k > 0) C.src_ptr.push_back(int(C.src.size()));
-                if (buf[k].first == I) C.diag[I] = int(C.col.size());
-                C.col.push_back(buf[k].first);
+                if (k > 0) R.end.push_back(int(R.src.size()));
+                R.col.push_back(buf[k].first);
             }
-            C.src.push_back(buf[k].second);
+            R.src.push_back(buf[k].second);
         }
-        if (!buf.empty()) C.src_ptr.push_back(int(C.src.size()));
-        C.row_ptr[I + 1] = int(C.col.size());
-    }
+        if (!buf.empty()) R.end.push_back(int(R.src.size()));
+    });
+    find_diagonal(C);
 }
 
 void build_ap(ApPattern &P, const Topology &T, const std::vector<int> &agg, const std::vector<int> &agg2) {
-    const int ns = T.nslices;
-    // a row's entries (aggregate, position; ~position: half the entry), sorted
-    std::vector<std::pair<int, int>> buf;
-    auto row = [&](int f) {
-        buf.clear();
-        const long long base = T.slice_ptr[f / kSlice] + f % kSlice;
-        for (int e = 0; e < T.row_len[f]; ++e) {
-            const long long pos = base + (long long)e * kSlice;
-            const int j = T.col[pos], J = agg[j], J2 = agg2[j];
-            if (J >= 0) buf.emplace_back(J, J2 >= 0 ? ~int(pos) : int(pos));
-            if (J2 >= 0) buf.emplace_back(J2, ~int(pos));
-        }
-        std::sort(buf.begin(), buf.end());
-    };
+    const int ns = T.nslices, nt = ranges(ns, 32);
     P.slice_ptr.assign(ns + 1, 0);
+    // slice by slice: the rows' entries (aggregate, position; ~position: half the
+    // entry), sorted, then the slots and their lists in slot order
+    struct Run { int J, n, at; };
+    struct Part { std::vector<int> slice, col, end, src; };
+    std::vector<Part> parts(nt);
+    std::vector<int> width(ns, 0);
+    in_ranges(ns, nt, [&](int t, int b, int e) {
+        Part &Q = parts[t];
+        std::vector<std::pair<int, int>> buf;
+        std::vector<std::vector<Run>> runs(kSlice);
+        std::vector<int> pos;
+        for (int sl = b; sl < e; ++sl) {
+            size_t w = 0;
+            pos.clear();
+            for (int l = 0; l < kSlice; ++l) {
+                const int f = sl * kSlice + l;
+                const long long base = T.slice_ptr[sl] + l;
+                buf.clear();
+                for (int k = 0; k < T.row_len[f]; ++k) {
+                    const long long p = base + (long long)k * kSlice;
+                    const int j = T.col[p], J = agg[j], J2 = agg2[j];
+                    if (J >= 0) buf.emplace_back(J, J2 >= 0 ? ~int(p) : int(p));
+                    if (J2 >= 0) buf.emplace_back(J2, ~int(p));
+                }
+                std::sort(buf.begin(), buf.end());
+                auto &r = runs[l];
+                r.clear();
+                for (const auto &q : buf) {
+                    if (r.empty() || r.back().J != q.first) r.push_back({q.first, 0, int(pos.size())});
+                    r.back().n++;
+                    pos.push_back(q.second);
+                }
+                w = std::max(w, r.size());
+            }
+            width[sl] = int(w);
+            for (size_t k = 0; k < w; ++k) {
+                Q.slice.push_back(sl);
+                for (int l = 0; l < kSlice; ++l) {
+                    const bool in = k < runs[l].size();
+                    Q.col.push_back(in ? runs[l][k].J : 0);
+                    if (in)
+                        Q.src.insert(Q.src.end(), pos.begin() + runs[l][k].at,
+                                     pos.begin() + runs[l][k].at + runs[l][k].n);
+                    Q.end.push_back(int(Q.src.size()));
+                }
+            }
+        }
+    });
+    for (int sl = 0; sl < ns; ++sl) P.slice_ptr[sl + 1] = P.slice_ptr[sl] + (long long)width[sl] * kSlice;
+    std::vector<std::vector<int>> slices(nt), cols(nt), ends(nt), srcs(nt);
+    for (int t = 0; t < nt; ++t) {
+        slices[t].swap(parts[t].slice);
+        cols[t].swap(parts[t].col);
+        ends[t].swap(parts[t].end);
+        srcs[t].swap(parts[t].src);
+    }
     P.slice.clear();
     P.col.clear();
-    P.src_ptr.assign(1, 0);
     P.src.clear();
-    // slice by slice: the rows' entries, then the slots and their lists in slot order
-    struct Run { int J, n, at; };
-    std::vector<std::vector<Run>> runs(kSlice);
-    std::vector<int> pos;
-    for (int sl = 0; sl < ns; ++sl) {
-        size_t w = 0;
-        pos.clear();
-        for (int l = 0; l < kSlice; ++l) {
-            row(sl * kSlice + l);
-            auto &r = runs[l];
-            r.clear();
-            for (const auto &q : buf) {
-                if (r.empty() || r.back().J != q.first) r.push_back({q.first, 0, int(pos.size())});
-                r.back().n++;
-                pos.push_back(q.second);
-            }
-            w = std::max(w, r.size());
-        }
-        for (size_t e = 0; e < w; ++e) {
-            P.slice.push_back(sl);
-            for (int l = 0; l < kSlice; ++l) {
-                const bool in = e < runs[l].size();
-                P.col.push_back(in ? runs[l][e].J : 0);
-                if (in) P.src.insert(P.src.end(), pos.begin() + runs[l][e].at, pos.begin() + runs[l][e].at + runs[l][e].n);
-                P.src_ptr.push_back(int(P.src.size()));
-            }
-        }
-        P.slice_ptr[sl + 1] = P.slice_ptr[sl] + (long long)w * kSlice;
-    }
+    append(P.slice, slices);
+    append(P.col, cols);
+    const std::vector<size_t> at = append(P.src, srcs);
+    for (int t = 0; t < nt; ++t)
+        for (int &e : ends[t]) e += int(at[t]);
+    P.src_ptr.assign(1, 0);
+    append(P.src_ptr, ends);
 }
 
 // Smoothed-aggregation transfer F -> C (C.agg set, F's CSR pattern known):
@@ -121,27 +233,24 @@ void build_ap(ApPattern &P, const Topology &T, const std::vector<int> &agg, cons
 void sa_transfer(AmgLevel &F, AmgLevel &C) {
     const int n = F.n;
     F.sa_out = true;
-    F.p_ptr.assign(n + 1, 0);
-    F.p_col.clear();
     F.p_own.assign(n, -1);
-    F.p_src_ptr.assign(1, 0);
-    F.p_src.clear();
-    std::vector<std::pair<int, int>> buf;
-    for (int i = 0; i < n; ++i) {
+    build_rows(n, F.p_ptr, F.p_col, F.p_src_ptr, F.p_src, nullptr, [&](int i, RowPart &R) {
+        thread_local std::vector<std::pair<int, int>> buf;
         buf.clear();
         for (int k = F.row_ptr[i]; k < F.row_ptr[i + 1]; ++k) buf.emplace_back(C.agg[F.col[k]], k);
         std::sort(buf.begin(), buf.end());
         for (size_t k = 0; k < buf.size(); ++k) {
             if (k == 0 || buf[k].first != buf[k - 1].first) {
-                if (k > 0) F.p_src_ptr.push_back(int(F.p_src.size()));
-                if (buf[k].first == C.agg[i]) F.p_own[i] = int(F.p_col.size());
-                F.p_col.push_back(buf[k].first);
+                if (k > 0) R.end.push_back(int(R.src.size()));
+                R.col.push_back(buf[k].first);
             }
-            F.p_src.push_back(buf[k].second);
+            R.src.push_back(buf[k].second);
         }
-        if (!buf.empty()) F.p_src_ptr.push_back(int(F.p_src.size()));
-        F.p_ptr[i + 1] = int(F.p_col.size());
-    }
+        if (!buf.empty()) R.end.push_back(int(R.src.size()));
+    });
+    for (int i = 0; i < n; ++i)
+        for (int q = F.p_ptr[i]; q < F.p_ptr[i + 1]; ++q)
+            if (F.p_col[q] == C.agg[i]) F.p_own[i] = q;
     // P' (rows of C)
     F.pt_ptr.assign(C.n + 1, 0);
     for (int J : F.p_col) F.pt_ptr[J + 1]++;
@@ -159,59 +268,40 @@ void sa_transfer(AmgLevel &F, AmgLevel &C) {
         F.p_tpos.assign(F.p_col.size(), 0);
         for (size_t e = 0; e < F.pt_map.size(); ++e) F.p_tpos[F.pt_map[e]] = int(e);
     }
-    // T = A P
-    std::vector<std::array<int, 3>> tb;
-    F.t_ptr.assign(n + 1, 0);
-    F.t_col.clear();
-    F.t_pair_ptr.assign(1, 0);
-    F.t_pa.clear();
-    F.t_pb.clear();
-    for (int i = 0; i < n; ++i) {
+    // T = A P, then A_C = P' T: sorted triples (column, the two factors' positions)
+    using Triples = std::vector<std::array<int, 3>>;
+    auto emit = [](Triples &tb, RowPart &R) {
+        std::sort(tb.begin(), tb.end());
+        for (size_t k = 0; k < tb.size(); ++k) {
+            if (k == 0 || tb[k][0] != tb[k - 1][0]) {
+                if (k > 0) R.end.push_back(int(R.src.size()));
+                R.col.push_back(tb[k][0]);
+            }
+            R.src.push_back(tb[k][1]);
+            R.src2.push_back(tb[k][2]);
+        }
+        if (!tb.empty()) R.end.push_back(int(R.src.size()));
+    };
+    build_rows(n, F.t_ptr, F.t_col, F.t_pair_ptr, F.t_pa, &F.t_pb, [&](int i, RowPart &R) {
+        thread_local Triples tb;
         tb.clear();
         for (int k = F.row_ptr[i]; k < F.row_ptr[i + 1]; ++k) {
             const int j = F.col[k];
             for (int q = F.p_ptr[j]; q < F.p_ptr[j + 1]; ++q) tb.push_back({F.p_col[q], k, q});
         }
-        std::sort(tb.begin(), tb.end());
-        for (size_t k = 0; k < tb.size(); ++k) {
-            if (k == 0 || tb[k][0] != tb[k - 1][0]) {
-                if (k > 0) F.t_pair_ptr.push_back(int(F.t_pa.size()));
-                F.t_col.push_back(tb[k][0]);
-            }
-            F.t_pa.push_back(tb[k][1]);
-            F.t_pb.push_back(tb[k][2]);
-        }
-        if (!tb.empty()) F.t_pair_ptr.push_back(int(F.t_pa.size()));
-        F.t_ptr[i + 1] = int(F.t_col.size());
-    }
-
-    // A_C = P' T
+        emit(tb, R);
+    });
     C.sa_in = true;
-    C.row_ptr.assign(C.n + 1, 0);
-    C.col.clear();
-    C.src_ptr.assign(1, 0);
-    C.src.clear();
-    C.src2.clear();
-    C.diag.assign(C.n, -1);
-    for (int I = 0; I < C.n; ++I) {
+    build_rows(C.n, C.row_ptr, C.col, C.src_ptr, C.src, &C.src2, [&](int I, RowPart &R) {
+        thread_local Triples tb;
         tb.clear();
         for (int e = F.pt_ptr[I]; e < F.pt_ptr[I + 1]; ++e) {
             const int i = F.pt_col[e], q = F.pt_map[e];
             for (int t = F.t_ptr[i]; t < F.t_ptr[i + 1]; ++t) tb.push_back({F.t_col[t], q, t});
         }
-        std::sort(tb.begin(), tb.end());
-        for (size_t k = 0; k < tb.size(); ++k) {
-            if (k == 0 || tb[k][0] != tb[k - 1][0]) {
-                if (k > 0) C.src_ptr.push_back(int(C.src.size()));
-                if (tb[k][0] == I) C.diag[I] = int(C.col.size());
-                C.col.push_back(tb[k][0]);
-            }
-            C.src.push_back(tb[k][1]);
-            C.src2.push_back(tb[k][2]);
-        }
-        if (!tb.empty()) C.src_ptr.push_back(int(C.src.size()));
-        C.row_ptr[I + 1] = int(C.col.size());
-    }
+        emit(tb, R);
+    });
+    find_diagonal(C);
 }
 
 // Block factors for one transfer: 2 along the coarsenable directions whose
