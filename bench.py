@@ -45,18 +45,22 @@ def _problem(pkg, seed):
     return g, perm, bt, bv
 
 
-def _vcycle_kernels(nf, v, lev_rows, lev_nnz, p_nnz, t_nnz, ap_nnz, sa_level):
+def _vcycle_kernels(nf, v, lev_rows, lev_nnz, p_nnz, t_nnz, ap_nnz, sa_level, blocks):
     """Algorithmic bytes of the kernels of one multigrid V(1,1) cycle outside
     the level-0 operator pass (the pre-smoothing residual is counted by the
     caller), as [(kernel, bytes)]: each array once per kernel at its stored
     precision v, 4-byte indices, gathered vectors once.  lev_rows / lev_nnz
     hold levels 0 (faces) .. L-1; sa_level is the level whose transfer to the
-    next is smoothed (-1: none)."""
+    next is smoothed (-1: none); blocks are the logical block factors of the
+    first transfer."""
     L = len(lev_rows)
     out = []
     n1 = lev_rows[1]
-    # faces -> level 1 (children lists): child pointers, children, res0, b1
-    out.append(("k_restrict (faces -> level 1)", nf * (4 + v) + n1 * (4 + v)))
+    # faces -> level 1 (children lists): child pointers, children (a face between
+    # two blocks is in both lists: every face across a direction that is not
+    # coarsened, half of them across one that is), res0, b1
+    kids = 1.0 + sum(1.0 / max(1, int(b)) for b in blocks) / 3.0
+    out.append(("k_restrict (faces -> level 1)", int(nf * (4 * kids + v)) + n1 * (4 + v)))
     for l in range(1, L - 1):
         n, nnz, nc = lev_rows[l], lev_nnz[l], lev_rows[l + 1]
         # down-sweep from zero: row pointers, matrix, b, D^-1, x and res written
@@ -73,9 +77,9 @@ def _vcycle_kernels(nf, v, lev_rows, lev_nnz, p_nnz, t_nnz, ap_nnz, sa_level):
             out.append((f"up-sweep level {l}", 8 * nnz + n * (8 + 3 * v) + nc * v))
     m = lev_rows[L - 1]
     out.append(("coarsest dense solve", m * m * v + 2 * m * v))
-    # post-smoothing on level 0 with A P: its SELL entries, the aggregate map,
-    # x0, res0, r, D^-1 read, z written, x_1 gathered
-    out.append(("k_vc0_post", ap_nnz * (v + 4) + nf * (4 + 5 * v) + n1 * v))
+    # post-smoothing on level 0: the SELL entries of M0 = P - w D^-1 A P, res0, r,
+    # D^-1 read, z written, x_1 gathered
+    out.append(("k_vc0_post", ap_nnz * (v + 4) + nf * 4 * v + n1 * v))
     return out
 
 
@@ -116,7 +120,8 @@ def _alg_bytes(g, nnz, nf, rep=None):
             # first smoothing step x0 = w D^-1 r: x, r, p, q, D^-1 read, x, r, x0 written
             upd_xr = ("k_update_xr", 8 * nf * v)
             upd_pz = ("k_update_pz", 3 * nf * v)        # p = z + b p
-            vc = _vcycle_kernels(nf, v, lev_rows, lev_nnz, p_nnz, t_nnz, int(rep["ap_nnz"]), sa_level)
+            vc = _vcycle_kernels(nf, v, lev_rows, lev_nnz, p_nnz, t_nnz, int(rep["ap_nnz"]), sa_level,
+                                 rep["coarsening"][0])
             ks = [("SpMV q = A p", out["spmv" + tag]), upd_xr, ("pre-smoothing residual", out["resid" + tag])]
             out["kernels" + tag] = ks + vc + [upd_pz]
             out["amg_iter" + tag] = sum(b for _, b in out["kernels" + tag])
@@ -734,11 +739,11 @@ def bench_impes(args, pkg, torch, dev):
     small = sum(x[2] for x in log)
     t_press = sum(x[0] for x in log)
     t_trans = sum(x[1] for x in log)
-    # roofline of the small-step kernel: saturation in and out, pore volume,
-    # facepos, and per half-face the cell across (int) and the face's flux,
-    # gravity and capillary coefficients (FP64); Dirichlet saturations
+    # roofline of the small-step kernel: saturation in and out, pore volume, facepos,
+    # and per half-face the cell across (int) and the face's flux and gravity
+    # coefficients (FP64; capillary pressure is off); Dirichlet saturations
     ndir = int(np.sum(np.asarray(g.nb) < 0))
-    alg = nc * (8 + 8 + 8) + (nc + 1) * 4 + nhf * (4 + 3 * 8) + ndir * 8
+    alg = nc * (8 + 8 + 8) + (nc + 1) * 4 + nhf * (4 + 2 * 8) + ndir * 8
     ms_k = t.time_step(reps=50)
     ach = alg / (ms_k * 1e-3) / 1e9
     roof = {"kernel": "k_tr_step (explicit upstream small step, one thread per cell)", "bound": "hbm",

@@ -81,7 +81,11 @@ typedef struct {
                                   previous solve's: the multigrid coarse levels, smoothed
                                   transfer and coarsest inverses are kept (the face system
                                   is still assembled; the PCG uses it) */
-    double prolongate_factor;  /* (:667) multigrid coarse-correction factor (default 1.6) */
+    double prolongate_factor;  /* (:667) multigrid coarse-correction factor a (default 1.6, the
+                                  reference's damping): tentative transfers take
+                                  1 + (a - 1) 5/6 below the smoothed one and
+                                  1 + (a - 1) / 2 above it; the smoothed one and the
+                                  averaging one from the faces take 1 */
     int smooth_steps;          /* (:668) multigrid smoothing sweeps before and after
                                   the coarse correction */
     int precision;             /* enum mhs_precision */
@@ -109,7 +113,8 @@ typedef struct {
     int sweep_threads;         /* same for the multigrid smoothing sweep */
     int tail_rows;             /* -1: from autotune (0 when autotune is 0); >= 0: coarse
                                   levels whose largest instance has at most this many
-                                  rows run in one workgroup per instance */
+                                  rows, as far as they fit in LDS, run in one workgroup
+                                  per instance */
     int element_operator;      /* mixed precision: apply the face operator of the PCG
                                   product, its FP64 residual replacement and the
                                   multigrid pre-smoothing residual cell by cell from the

@@ -2308,6 +2308,7 @@ int transport_coeffs(mhs_transport *t, const double *grav, int cap) {
         t->coeff_grav[1] == grav[1] && t->coeff_grav[2] == grav[2])
         return MHS_OK;
     const int has_g = grav[0] != 0.0 || grav[1] != 0.0 || grav[2] != 0.0;
+    t->D.has_g = has_g;
     TCHECK(launch_tr_coeffs(s->stream, t->D, s->dT, s->dG, s->perm, grav, has_g, cap));
     double dt_g = 1e100;
     if (has_g) {
@@ -2546,12 +2547,12 @@ int mhs_transport_init(mhs_transport *t, const double *porosity, const double *s
     D.F = t->F;
     D.G = t->G;
     D.C = t->C;
-    D.visc_w = fluid->viscosity[0];
-    D.visc_o = fluid->viscosity[1];
+    D.ivisc_w = 1.0 / fluid->viscosity[0];
+    D.ivisc_o = 1.0 / fluid->viscosity[1];
     D.rho_w = fluid->density[0];
     D.rho_o = fluid->density[1];
     D.drho = fluid->density[0] - fluid->density[1];
-    cfl_factors(D.visc_w, D.visc_o, t->fac);
+    cfl_factors(fluid->viscosity[0], fluid->viscosity[1], t->fac);
     t->topo_key = s->struct_gen;
     t->timed_ok = false;
     t->coeff_gen = -1;

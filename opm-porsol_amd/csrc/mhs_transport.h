@@ -23,8 +23,9 @@ struct DevTransport {
     const double *pv = nullptr;      // [nc] pore volume
     double *F = nullptr, *G = nullptr, *C = nullptr;  // [max_ncf * nc] owner-oriented flux, gravity and capillary
                                                       // coefficients, slot-major
-    double visc_w = 1.0, visc_o = 1.0, rho_w = 0.0, rho_o = 0.0, drho = 0.0;
+    double ivisc_w = 1.0, ivisc_o = 1.0, rho_w = 0.0, rho_o = 0.0, drho = 0.0;
     int method_viscous = 1, method_gravity = 1, method_capillary = 1;
+    int has_g = 1;                   // the gravity vector of G is not zero
 };
 
 // Gravity and capillary coefficients (per permeability and gravity vector).

@@ -390,3 +390,28 @@ def test_transport_on_a_batch_with_two_rhs(pkg):
             np.testing.assert_allclose(s_gpu[c0:c1], ref, rtol=0, atol=1e-12)
             same += 1
     assert same >= 1
+
+
+# One size on each side of a block of 256 cells (box: six faces on every cell,
+# all loaded at once), and a faulted grid (the cell's own face count).
+@pytest.mark.parametrize("dims,fault", [((1, 1, 1), 0), ((17, 5, 3), 0), ((16, 4, 4), 0), ((257, 1, 1), 0),
+                                        ((9, 7, 4), 0.3)])
+@pytest.mark.parametrize("grav", [(0.0, 0.0, 0.0), GRAV])
+@pytest.mark.parametrize("cap", [False, True])
+def test_residual_terms_left_out(pkg, dims, fault, grav, cap):
+    """Gravity and capillary coefficients are read only where their term is on;
+    the gravity flux switched off, and back on, on the same object."""
+    g = pkg.grids.corner_point(*dims, 2.0, 2.0, 1.0, seed=6, fault_frac=fault) if fault else \
+        pkg.grids.cartesian(*dims, 2.0, 2.0, 1.0)
+    nc = g.num_cells
+    rng = np.random.default_rng(nc)
+    perm = pkg.fields.perm_c1(nc, 6)
+    bt, bv = cases.xdrop_bc(g, 2 * BAR, 0.0)
+    sat, sat_bc = rng.uniform(0.0, 1.0, nc), rng.uniform(0.0, 1.0, g.num_half_faces)
+    s, flux = _flow(pkg, g, perm, bt, bv, sat)
+    t = pkg.EulerUpstream(s, np.full(nc, 0.2), sat_bc, VISC, RHO)
+    for mg in (True, False, True):
+        r_gpu = t.computeResidual(sat, grav, None, True, mg, cap)
+        r_orc = tr.residual(g, perm, sat, flux, grav, DRHO, VISC, None, sat_bc, None, True, mg, cap)
+        # FP64 sums of at most a dozen faces on the same fluxes, as above
+        assert cases.rel_err(r_gpu, r_orc) < 1e-12
