@@ -1574,35 +1574,39 @@ int solve_impl(mhs_solver *s, const double *totmob, const double *rhomob, const 
             // the face level's part of the cycle, follows the new assembly
             mg_reused = opt.same_matrix && attempt == 0 && s->setup_gen == s->perm_gen &&
                         (s->setup_mixed || !mixed) && s->setup_aniso == (binv_use != nullptr);
+            // Jacobi weights: the caller's, or 4 / (3 rho(D^-1 A)) per level with
+            // rho estimated on the first multigrid solve of this hierarchy
+            auto set_weights = [&]() {
+                for (int l = 0; l < kMaxLevels; ++l) {
+                    const double r = l < (int)s->rho.size() ? s->rho[l] : 0.0;
+                    s->dA.omega_l[l] = opt.smoother_weight > 0.0 ? opt.smoother_weight
+                                       : r > 0.0 ? std::min(1.0, std::max(0.2, 4.0 / (3.0 * r)))
+                                                 : 0.7;
+                }
+            };
+            const bool known = opt.smoother_weight > 0.0 || !s->rho.empty();
+            if (known) set_weights();
             // A P from the element values when no face matrix was filled
             HIPCHECK(launch_amg_setup(s->stream, s->dT, s->dA, s->ftype, s->val64, mixed,
-                                      s->mat_valid ? nullptr : s->dE.val64, mg_reused));
+                                      s->mat_valid ? nullptr : s->dE.val64, mg_reused,
+                                      known && mixed ? s->dinv64 : nullptr));
             if (!mg_reused) {
                 s->setup_gen = s->perm_gen;
                 s->setup_mixed = mixed;
                 s->setup_aniso = binv_use != nullptr;
             }
-            // Jacobi weights: the caller's, or 4 / (3 rho(D^-1 A)) per level with
-            // rho estimated on the first multigrid solve of this hierarchy
-            if (opt.smoother_weight > 0.0) {
-                for (int l = 0; l < kMaxLevels; ++l) s->dA.omega_l[l] = opt.smoother_weight;
-            } else {
-                if (s->rho.empty()) {
-                    rc = estimate_rho(s);
-                    if (rc) return rc;
-                    s->rho_gen = s->perm_gen;
-                    s->rho_aniso = binv_use != nullptr;
-                    rho_fresh = true;
-                }
-                for (int l = 0; l < kMaxLevels; ++l) {
-                    const double r = l < (int)s->rho.size() ? s->rho[l] : 0.0;
-                    s->dA.omega_l[l] = r > 0.0 ? std::min(1.0, std::max(0.2, 4.0 / (3.0 * r))) : 0.7;
-                }
+            if (!known) {
+                rc = estimate_rho(s);
+                if (rc) return rc;
+                s->rho_gen = s->perm_gen;
+                s->rho_aniso = binv_use != nullptr;
+                rho_fresh = true;
+                set_weights();
             }
             if (!mg_reused) HIPCHECK(launch_amg_combine(s->stream, s->dA, mixed));
             // (also for kept levels: A P is new, and their last solve may have had the
             // other precision)
-            HIPCHECK(launch_amg_ready(s->stream, s->dT, s->dA, s->ftype, s->dinv64, mixed));
+            HIPCHECK(launch_amg_ready(s->stream, s->dT, s->dA, s->ftype, s->dinv64, mixed, known && mixed));
         }
 
         // --- launch shapes -------------------------------------------------------

@@ -268,9 +268,12 @@ hipError_t launch_resnorm(hipStream_t st, const DevTopo &T, int nrhs, const doub
 // in the PCG's precision.
 hipError_t launch_amg_combine(hipStream_t st, const DevAmg &A, bool mixed);
 hipError_t launch_amg_ready(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype,
-                            const double *dinv0, bool mixed);
+                            const double *dinv0, bool mixed, bool m0_done);
+// m0_dinv (mixed only, else null): the weights are known, so A P's launch also
+// writes M0 (the face rows' inverse diagonal).
 hipError_t launch_amg_setup(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype,
-                            const double *val64, bool mixed, const double *elem64 = nullptr, bool ap_only = false);
+                            const double *val64, bool mixed, const double *elem64,
+                            bool ap_only, const double *m0_dinv);
 // Lanczos steps on D^-1/2 A_l D^-1/2 (FP64) of every smoothed level at once, for
 // the Jacobi weights: all launches on the stream, the scalars stay on the
 // device.  w, v0, v1, u, y: lanczos_rows() doubles each, part: lanczos_parts();

@@ -1483,13 +1483,25 @@ __global__ __launch_bounds__(256) void k_galerkin(int nnz, const int *__restrict
     if (out32) out32[e] = (float)s[0];
 }
 
+// Entry of M0 = P - w D^-1 A P at a slot of row f (see k_ap_m0).
+__device__ __forceinline__ double m0_entry(double ap, bool empty, bool dir, int J, int g, int g2, double wd) {
+    if (empty || dir) return 0.0;
+    return (J == g || J == g2 ? (g2 >= 0 ? 0.5 : 1.0) : 0.0) - wd * ap;
+}
+
 // A P, one lane per slot: the slot's list of face-matrix (or element) values,
 // zero on Dirichlet rows (the cycle leaves them out: their residual is zero).
-// ~2.7 list entries per slot, so one lane each keeps the loads coalesced.
+// About 2.7 list entries per slot, so one lane each keeps the loads coalesced.
+// M0: also the post-smoothing operator in FP32, where the weight is known already
+// (one pass over the slots instead of two: 295 + 139 -> 321 us at 128x128x64).
+template <bool M0>
 __global__ __launch_bounds__(256) void k_ap_fill(long long slots, const int *__restrict__ slot_slice,
                                                  const int *__restrict__ dof_hf, const uint8_t *__restrict__ ftype,
                                                  const int *__restrict__ src_ptr, const int *__restrict__ src,
-                                                 const double *__restrict__ fine, double *__restrict__ out) {
+                                                 const double *__restrict__ fine, double *__restrict__ out,
+                                                 const int *__restrict__ col, const int *__restrict__ agg,
+                                                 const int *__restrict__ agg2, const double *__restrict__ dinv,
+                                                 double w, float *__restrict__ m0) {
     const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
     if (q >= slots) return;
     const int f = slot_slice[q >> 6] * 64 + (int)(q & 63), h = dof_hf[f];
@@ -1503,7 +1515,10 @@ __global__ __launch_bounds__(256) void k_ap_fill(long long slots, const int *__r
         for (int u = 0; u < 4; ++u)
             if (k + u < k1) s += listed(fine, p[u]);
     }
-    out[q] = h >= 0 && ftype[h] == FT_DIRICHLET ? 0.0 : s;
+    const bool dir = h < 0 || ftype[h] == FT_DIRICHLET;
+    if (h >= 0 && dir) s = 0.0;
+    out[q] = s;
+    if constexpr (M0) m0[q] = (float)m0_entry(s, k1 == k0, dir, col[q], agg[f], agg2[f], w * dinv[f]);
 }
 
 // The post-smoothing operator M0 = P - w D^-1 A P on A P's pattern (which
@@ -1518,11 +1533,8 @@ __global__ __launch_bounds__(256) void k_ap_m0(long long slots, const int *__res
     const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
     if (q >= slots) return;
     const int f = slot_slice[q >> 6] * 64 + (int)(q & 63), h = dof_hf[f];
-    const int J = col[q], g = agg[f], g2 = agg2[f];
-    double v = 0.0;
-    if (src_ptr[q + 1] > src_ptr[q] && h >= 0 && ftype[h] != FT_DIRICHLET)
-        v = (J == g || J == g2 ? (g2 >= 0 ? 0.5 : 1.0) : 0.0) - w * dinv[f] * ap[q];
-    out[q] = (VT)v;
+    const bool dir = h < 0 || ftype[h] == FT_DIRICHLET;
+    out[q] = (VT)m0_entry(ap[q], src_ptr[q + 1] == src_ptr[q], dir, col[q], agg[f], agg2[f], w * dinv[f]);
 }
 
 __global__ __launch_bounds__(256) void k_coarse_diag(int n, const int *__restrict__ diag,
@@ -3518,14 +3530,20 @@ hipError_t launch_resnorm(hipStream_t st, const DevTopo &T, int nrhs, const doub
 
 
 hipError_t launch_amg_setup(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype,
-                            const double *val64, bool mixed, const double *elem64, bool ap_only) {
+                            const double *val64, bool mixed, const double *elem64, bool ap_only,
+                            const double *m0_dinv) {
     // A P of the level-1 aggregates first: level 1's Galerkin sums its slots.
     // elem64: from the FP64 element values (no face matrix filled)
     if (A.ap_slots > 0) {
         const bool el = elem64 != nullptr;
-        k_ap_fill<<<(unsigned)((A.ap_slots + 255) / 256), 256, 0, st>>>(
-            A.ap_slots, A.ap_slice, T.dof_hf, ftype, el ? A.ap_esrc_ptr : A.ap_src_ptr, el ? A.ap_esrc : A.ap_src,
-            el ? elem64 : val64, A.ap64);
+        auto fill = [&](auto m0) {
+            k_ap_fill<decltype(m0)::value><<<(unsigned)((A.ap_slots + 255) / 256), 256, 0, st>>>(
+                A.ap_slots, A.ap_slice, T.dof_hf, ftype, el ? A.ap_esrc_ptr : A.ap_src_ptr,
+                el ? A.ap_esrc : A.ap_src, el ? elem64 : val64, A.ap64, A.ap_col, A.lev[1].agg, A.agg2, m0_dinv,
+                A.omega_l[0], A.ap32);
+        };
+        if (mixed && m0_dinv) fill(std::true_type{});
+        else fill(std::false_type{});
     }
     if (ap_only) return hipGetLastError();   // the coarse levels are kept
     for (int l = 1; l < A.nlev; ++l) {
@@ -3594,8 +3612,8 @@ static void tail_pack(hipStream_t st, const DevAmg &A, VT *out, const VT *cinv) 
     k_tail_pack<VT><<<dim3(A.ninst, 4, A.nlev - A.tail_first), 256, 0, st>>>(P);
 }
 hipError_t launch_amg_ready(hipStream_t st, const DevTopo &T, const DevAmg &A, const uint8_t *ftype,
-                            const double *dinv0, bool mixed) {
-    const unsigned nb = (unsigned)((A.ap_slots + 255) / 256);
+                            const double *dinv0, bool mixed, bool m0_done) {
+    const unsigned nb = m0_done ? 0 : (unsigned)((A.ap_slots + 255) / 256);
     auto m0 = [&](auto *out) {
         if (nb)
             k_ap_m0<<<nb, 256, 0, st>>>(A.ap_slots, A.ap_slice, T.dof_hf, ftype, A.ap_src_ptr, A.ap_col, A.lev[1].agg,
