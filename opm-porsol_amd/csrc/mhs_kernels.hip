@@ -152,9 +152,11 @@ __global__ __launch_bounds__(256) void k_finish(DevRed R, DevScal S, FinArgs A) 
 // Where an instance has few partials, its finisher runs inside the kernel that
 // needs the result: every workgroup sums the instance's partials itself, one
 // wavefront per quantity, in the same order, so all of them find the same step.
-// One launch less, each about 4.3 us of waiting for a few dozen numbers.  Above
-// kFuseParts the reads of all workgroups would cost more than the launch.
-constexpr int kFuseParts = 512;
+// One launch less, each about 4.3 us of waiting for a few dozen numbers (and the
+// gap to the next).  The reads of all workgroups grow with the square of the
+// partials: at 763 (80x80x40) a solve takes 6.74 ms with the launches and 6.57
+// without, at 3105 (128x128x64) they would read 230 MB, more than the launch costs.
+constexpr int kFuseParts = 1024;
 template <int NQ>
 __device__ __forceinline__ void inst_totals(const DevRed &R, int s, int nq, double (&tot)[NQ]) {
     const int b0 = R.seg_blk[s], b1 = R.seg_blk[s + 1];
@@ -164,15 +166,19 @@ __device__ __forceinline__ void inst_totals(const DevRed &R, int s, int nq, doub
         const int q = q0 + (threadIdx.x >> 6);
         if (q >= NQ || q >= nq) continue;          // wave-uniform
         const double *pq = R.partials + (size_t)q * R.nblk;
-        double a[kFuseParts / 64];
+        double t = 0.0;
+        for (int i0 = b0; i0 < b1; i0 += 512) {    // eight loads in flight
+            double a[8];
 #pragma unroll
-        for (int u = 0; u < kFuseParts / 64; ++u) {
-            const int i = b0 + 64 * u + lane;
-            a[u] = i < b1 ? pq[i] : 0.0;
+            for (int u = 0; u < 8; ++u) {
+                const int i = i0 + 64 * u + lane;
+                a[u] = i < b1 ? pq[i] : 0.0;
+            }
+#pragma unroll
+            for (int u = 1; u < 8; ++u) a[0] += a[u];
+            t += a[0];
         }
-#pragma unroll
-        for (int u = 1; u < kFuseParts / 64; ++u) a[0] += a[u];
-        const double t = wave_sum(a[0]);
+        t = wave_sum(t);
         if (lane == 0) tot[q] = t;
     }
     __syncthreads();

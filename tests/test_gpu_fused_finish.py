@@ -1,6 +1,6 @@
 """The CG scalars worked out inside the vector updates (instances of few row
 blocks) against the separate finisher: a small instance solved alone takes
-the first, in a batch with one of more than 512 blocks the second."""
+the first, in a batch with one of more than 1024 blocks the second."""
 import numpy as np
 import pytest
 
@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("solver,nrhs", [(0, 1), (1, 1), (1, 2)])
 def test_small_instance_alone_and_beside_a_large_one(pkg, orc, solver, nrhs, precision):
-    small, large = pkg.grids.cartesian(9, 8, 7), pkg.grids.cartesian(56, 56, 56)
+    small, large = pkg.grids.cartesian(9, 8, 7), pkg.grids.cartesian(72, 72, 72)
     perm = pkg.fields.perm_c1(small.num_cells, 40)
     bt, bv = cases.xdrop_bc(small)
     G, icp = pkg.grids.concat([small, large])
@@ -37,3 +37,23 @@ def test_small_instance_alone_and_beside_a_large_one(pkg, orc, solver, nrhs, pre
     assert cases.rel_err(alone.getSolution()[2], ref.outflux) < 1e-8
     for k in range(nrhs):
         assert cases.rel_err(v[k], (1 + k) * ref.outflux) < 1e-8
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("solver", [0, 1])
+@pytest.mark.parametrize("n", [55, 56, 69])
+def test_more_partials_than_one_round_of_loads(pkg, solver, precision, n):
+    """Around 512 and just below 1024 partials (rows of 1024 faces), each summed
+    eight loads at a time; a uniform medium has the closed form v = k dp / L."""
+    g = pkg.grids.cartesian(n, n, n)
+    nc = g.num_cells
+    bt, bv = cases.xdrop_bc(g, 1.0, 0.0)
+    s = pkg.HybridSolver(0)
+    s.init(g, pkg.fields.diag_perm(np.ones(nc), np.ones(nc), np.ones(nc)), (0, 0, 0), bt, None)
+    tm, rm = cases.unit_fluid(nc)
+    s.solve(tm, rm, np.zeros(nc), bt, bv, residual_tolerance=1e-12, precision=precision, linsolver_type=solver)
+    exact = np.zeros(g.num_half_faces)
+    exact[g.side == 1], exact[g.side == 0] = 1.0 / n, -1.0 / n
+    v = np.asarray(s.getSolution()[2]).reshape(-1)
+    # solves to 1e-12 of a system with a condition number of about n^2 < 5e3
+    assert np.max(np.abs(v - exact)[(g.side == 0) | (g.side == 1)]) < 1e-8
