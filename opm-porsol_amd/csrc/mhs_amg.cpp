@@ -44,7 +44,8 @@ void in_ranges(int n, int nt, Fn fn) {
         if (e) std::rethrow_exception(e);
 }
 // Appends the ranges' lists in order; returns where each one starts.
-std::vector<size_t> append(std::vector<int> &out, const std::vector<std::vector<int>> &parts) {
+template <class I>
+std::vector<size_t> append(std::vector<I> &out, const std::vector<std::vector<I>> &parts) {
     std::vector<size_t> at(parts.size() + 1, out.size());
     for (size_t t = 0; t < parts.size(); ++t) at[t + 1] = at[t] + parts[t].size();
     out.resize(at.back());
@@ -54,15 +55,27 @@ std::vector<size_t> append(std::vector<int> &out, const std::vector<std::vector<
     return at;
 }
 
+size_t total(const std::vector<std::vector<int>> &parts) {
+    size_t n = 0;
+    for (const auto &p : parts) n += p.size();
+    return n;
+}
+// What the lists of one pattern may hold: positions of its entries are 32-bit
+// signed (~pos marks a half entry), the ends of its lists 32-bit unsigned.
+bool too_long(size_t entries, size_t list, size_t max_list) {
+    return entries > std::min<size_t>(max_list, 0x7fffffff) || list > std::min(max_list, kMaxList);
+}
+
 // Rows of a CSR pattern whose entries each carry a list, built range by range:
 // row(i, R) appends the row's columns to R.col and, per entry, its sources to
-// R.src (and R.src2) and their end to R.end.
+// R.src (and R.src2) and their end to R.end.  False: too long.
 struct RowPart {
-    std::vector<int> col, src, src2, end, len;
+    std::vector<int> col, src, src2, len;
+    std::vector<ListEnd> end;
 };
 template <class Row>
-void build_rows(int n, std::vector<int> &ptr, std::vector<int> &col, std::vector<int> &src_ptr, std::vector<int> &src,
-                std::vector<int> *src2, Row row) {
+bool build_rows(int n, std::vector<int> &ptr, std::vector<int> &col, std::vector<ListEnd> &src_ptr,
+                std::vector<int> &src, std::vector<int> *src2, size_t max_list, Row row) {
     const int nt = ranges(n, 2048);
     std::vector<RowPart> P(nt);
     in_ranges(n, nt, [&](int t, int b, int e) {
@@ -74,30 +87,34 @@ void build_rows(int n, std::vector<int> &ptr, std::vector<int> &col, std::vector
             R.len.push_back(int(R.col.size() - c0));
         }
     });
-    ptr.assign(n + 1, 0);
-    std::vector<std::vector<int>> cols(nt), srcs(nt), srcs2(nt), ends(nt);
-    for (int t = 0, i = 0; t < nt; ++t) {
-        for (int l : P[t].len) {
-            ptr[i + 1] = ptr[i] + l;
-            ++i;
-        }
+    std::vector<std::vector<int>> cols(nt), srcs(nt), srcs2(nt);
+    std::vector<std::vector<ListEnd>> ends(nt);
+    for (int t = 0; t < nt; ++t) {
         cols[t].swap(P[t].col);
         srcs[t].swap(P[t].src);
         srcs2[t].swap(P[t].src2);
         ends[t].swap(P[t].end);
     }
+    if (too_long(total(cols), total(srcs), max_list)) return false;
+    ptr.assign(n + 1, 0);
+    for (int t = 0, i = 0; t < nt; ++t)
+        for (int l : P[t].len) {
+            ptr[i + 1] = ptr[i] + l;
+            ++i;
+        }
     col.clear();
     src.clear();
     append(col, cols);
     const std::vector<size_t> at = append(src, srcs);
     for (int t = 0; t < nt; ++t)
-        for (int &e : ends[t]) e += int(at[t]);
+        for (ListEnd &e : ends[t]) e += ListEnd(at[t]);
     src_ptr.assign(1, 0);
     append(src_ptr, ends);
     if (src2) {
         src2->clear();
         append(*src2, srcs2);
     }
+    return true;
 }
 
 void children(AmgLevel &C, int nf) {
@@ -131,8 +148,8 @@ void find_diagonal(AmgLevel &C) {
 // finer row i (COARSE: j is already the coarse column, the entries being
 // those of A P).  Requires children() to have run.
 template <bool COARSE = false, class RowEntries>
-void galerkin_pattern(AmgLevel &C, RowEntries row_entries) {
-    build_rows(C.n, C.row_ptr, C.col, C.src_ptr, C.src, nullptr, [&](int I, RowPart &R) {
+bool galerkin_pattern(AmgLevel &C, size_t max_list, RowEntries row_entries) {
+    const bool ok = build_rows(C.n, C.row_ptr, C.col, C.src_ptr, C.src, nullptr, max_list, [&](int I, RowPart &R) {
         thread_local std::vector<std::pair<int, int>> buf;
         buf.clear();
         for (int k = C.child_ptr[I]; k < C.child_ptr[I + 1]; ++k)
@@ -146,23 +163,26 @@ void galerkin_pattern(AmgLevel &C, RowEntries row_entries) {
         });
         for (size_t k = 0; k < buf.size(); ++k) {
             if (k == 0 || buf[k].first != buf[k - 1].first) {
-                if (k > 0) R.end.push_back(int(R.src.size()));
+                if (k > 0) R.end.push_back(ListEnd(R.src.size()));
                 R.col.push_back(buf[k].first);
             }
             R.src.push_back(buf[k].second);
         }
-        if (!buf.empty()) R.end.push_back(int(R.src.size()));
+        if (!buf.empty()) R.end.push_back(ListEnd(R.src.size()));
     });
-    find_diagonal(C);
+    if (ok) find_diagonal(C);
+    return ok;
 }
 
-void build_ap(ApPattern &P, const Topology &T, const std::vector<int> &agg, const std::vector<int> &agg2) {
+// False: too long.
+bool build_ap(ApPattern &P, const Topology &T, const std::vector<int> &agg, const std::vector<int> &agg2,
+              size_t max_list) {
     const int ns = T.nslices, nt = ranges(ns, 32);
     P.slice_ptr.assign(ns + 1, 0);
     // slice by slice: the rows' entries (aggregate, position; ~position: half the
     // entry), sorted, then the slots and their lists in slot order
     struct Run { int J, n, at; };
-    struct Part { std::vector<int> slice, col, end, src; };
+    struct Part { std::vector<int> slice, col, src; std::vector<ListEnd> end; };
     std::vector<Part> parts(nt);
     std::vector<int> width(ns, 0);
     in_ranges(ns, nt, [&](int t, int b, int e) {
@@ -202,19 +222,21 @@ void build_ap(ApPattern &P, const Topology &T, const std::vector<int> &agg, cons
                     if (in)
                         Q.src.insert(Q.src.end(), pos.begin() + runs[l][k].at,
                                      pos.begin() + runs[l][k].at + runs[l][k].n);
-                    Q.end.push_back(int(Q.src.size()));
+                    Q.end.push_back(ListEnd(Q.src.size()));
                 }
             }
         }
     });
     for (int sl = 0; sl < ns; ++sl) P.slice_ptr[sl + 1] = P.slice_ptr[sl] + (long long)width[sl] * kSlice;
-    std::vector<std::vector<int>> slices(nt), cols(nt), ends(nt), srcs(nt);
+    std::vector<std::vector<int>> slices(nt), cols(nt), srcs(nt);
+    std::vector<std::vector<ListEnd>> ends(nt);
     for (int t = 0; t < nt; ++t) {
         slices[t].swap(parts[t].slice);
         cols[t].swap(parts[t].col);
         ends[t].swap(parts[t].end);
         srcs[t].swap(parts[t].src);
     }
+    if (too_long(total(cols), total(srcs), max_list)) return false;
     P.slice.clear();
     P.col.clear();
     P.src.clear();
@@ -222,32 +244,33 @@ void build_ap(ApPattern &P, const Topology &T, const std::vector<int> &agg, cons
     append(P.col, cols);
     const std::vector<size_t> at = append(P.src, srcs);
     for (int t = 0; t < nt; ++t)
-        for (int &e : ends[t]) e += int(at[t]);
+        for (ListEnd &e : ends[t]) e += ListEnd(at[t]);
     P.src_ptr.assign(1, 0);
     append(P.src_ptr, ends);
+    return true;
 }
 
 // Smoothed-aggregation transfer F -> C (C.agg set, F's CSR pattern known):
 // the patterns of P, P', T = A_F P and A_C = P' T, with the gather / pair
 // lists that let every solve fill their values on the device.
-void sa_transfer(AmgLevel &F, AmgLevel &C) {
+bool sa_transfer(AmgLevel &F, AmgLevel &C, size_t max_list) {
     const int n = F.n;
     F.sa_out = true;
     F.p_own.assign(n, -1);
-    build_rows(n, F.p_ptr, F.p_col, F.p_src_ptr, F.p_src, nullptr, [&](int i, RowPart &R) {
+    if (!build_rows(n, F.p_ptr, F.p_col, F.p_src_ptr, F.p_src, nullptr, max_list, [&](int i, RowPart &R) {
         thread_local std::vector<std::pair<int, int>> buf;
         buf.clear();
         for (int k = F.row_ptr[i]; k < F.row_ptr[i + 1]; ++k) buf.emplace_back(C.agg[F.col[k]], k);
         std::sort(buf.begin(), buf.end());
         for (size_t k = 0; k < buf.size(); ++k) {
             if (k == 0 || buf[k].first != buf[k - 1].first) {
-                if (k > 0) R.end.push_back(int(R.src.size()));
+                if (k > 0) R.end.push_back(ListEnd(R.src.size()));
                 R.col.push_back(buf[k].first);
             }
             R.src.push_back(buf[k].second);
         }
-        if (!buf.empty()) R.end.push_back(int(R.src.size()));
-    });
+        if (!buf.empty()) R.end.push_back(ListEnd(R.src.size()));
+    })) return false;
     for (int i = 0; i < n; ++i)
         for (int q = F.p_ptr[i]; q < F.p_ptr[i + 1]; ++q)
             if (F.p_col[q] == C.agg[i]) F.p_own[i] = q;
@@ -274,15 +297,15 @@ void sa_transfer(AmgLevel &F, AmgLevel &C) {
         std::sort(tb.begin(), tb.end());
         for (size_t k = 0; k < tb.size(); ++k) {
             if (k == 0 || tb[k][0] != tb[k - 1][0]) {
-                if (k > 0) R.end.push_back(int(R.src.size()));
+                if (k > 0) R.end.push_back(ListEnd(R.src.size()));
                 R.col.push_back(tb[k][0]);
             }
             R.src.push_back(tb[k][1]);
             R.src2.push_back(tb[k][2]);
         }
-        if (!tb.empty()) R.end.push_back(int(R.src.size()));
+        if (!tb.empty()) R.end.push_back(ListEnd(R.src.size()));
     };
-    build_rows(n, F.t_ptr, F.t_col, F.t_pair_ptr, F.t_pa, &F.t_pb, [&](int i, RowPart &R) {
+    if (!build_rows(n, F.t_ptr, F.t_col, F.t_pair_ptr, F.t_pa, &F.t_pb, max_list, [&](int i, RowPart &R) {
         thread_local Triples tb;
         tb.clear();
         for (int k = F.row_ptr[i]; k < F.row_ptr[i + 1]; ++k) {
@@ -290,9 +313,9 @@ void sa_transfer(AmgLevel &F, AmgLevel &C) {
             for (int q = F.p_ptr[j]; q < F.p_ptr[j + 1]; ++q) tb.push_back({F.p_col[q], k, q});
         }
         emit(tb, R);
-    });
+    })) return false;
     C.sa_in = true;
-    build_rows(C.n, C.row_ptr, C.col, C.src_ptr, C.src, &C.src2, [&](int I, RowPart &R) {
+    if (!build_rows(C.n, C.row_ptr, C.col, C.src_ptr, C.src, &C.src2, max_list, [&](int I, RowPart &R) {
         thread_local Triples tb;
         tb.clear();
         for (int e = F.pt_ptr[I]; e < F.pt_ptr[I + 1]; ++e) {
@@ -300,8 +323,9 @@ void sa_transfer(AmgLevel &F, AmgLevel &C) {
             for (int t = F.t_ptr[i]; t < F.t_ptr[i + 1]; ++t) tb.push_back({F.t_col[t], q, t});
         }
         emit(tb, R);
-    });
+    })) return false;
     find_diagonal(C);
+    return true;
 }
 
 // Block factors for one transfer: 2 along the coarsenable directions whose
@@ -469,8 +493,9 @@ std::vector<std::array<int, 3>> coarsening_plan(const Strength &strength, const 
 }
 
 std::string build_amg(AmgHierarchy &H, const Topology &T, const std::vector<int> &ijk, const Strength &strength,
-                      bool smoothed) {
+                      bool smoothed, size_t max_list) {
     H = AmgHierarchy();
+    const char *const kTooLong = "grid too large for the 32-bit multigrid gather lists";
     const int ninst = T.ninst;
     if (T.slice_ptr[T.nslices] > 0x7fffffffLL)
         return "face matrix too large for the 32-bit multigrid gather lists";
@@ -520,9 +545,9 @@ std::string build_amg(AmgHierarchy &H, const Topology &T, const std::vector<int>
         children(L1, T.nfp);
         // A_1 = P' (A P): each entry sums the A P slots of its row's faces
         // (about 7 per face row) instead of the face matrix's entries (11)
-        build_ap(H.ap, T, L1.agg, L1.agg2);
+        if (!build_ap(H.ap, T, L1.agg, L1.agg2, max_list)) return kTooLong;
         const ApPattern &ap = H.ap;
-        galerkin_pattern<true>(L1, [&](int child, auto emit) {
+        const bool fits = galerkin_pattern<true>(L1, max_list, [&](int child, auto emit) {
             const bool half = child < 0;
             const int f = half ? ~child : child;
             const long long base = ap.slice_ptr[f / kSlice] + f % kSlice;
@@ -532,6 +557,7 @@ std::string build_amg(AmgHierarchy &H, const Topology &T, const std::vector<int>
                 if (ap.src_ptr[q + 1] > ap.src_ptr[q]) emit(ap.col[q], half ? ~int(q) : int(q));   // padding slots sum nothing
             }
         });
+        if (!fits) return kTooLong;
         H.lev.push_back(std::move(L1));
     }
     // ---- coarser levels: group the blocks again until every instance is small
@@ -569,7 +595,7 @@ std::string build_amg(AmgHierarchy &H, const Topology &T, const std::vector<int>
         // every stencil)
         if (smoothed && !sa_done && 8LL * Fr.n <= (long long)T.nf_total) {
             sa_done = true;
-            sa_transfer(Fr, C);
+            if (!sa_transfer(Fr, C, max_list)) return kTooLong;
             // the up-sweep stores M = P - w D^-1 T on T's pattern, which holds
             // P's (A holds its diagonal; both rows sorted)
             Fr.t_p.assign(Fr.t_col.size(), -1);
@@ -583,9 +609,10 @@ std::string build_amg(AmgHierarchy &H, const Topology &T, const std::vector<int>
                 }
             }
         } else {
-            galerkin_pattern(C, [&](int r, auto emit) {
+            const bool fits = galerkin_pattern(C, max_list, [&](int r, auto emit) {
                 for (int k = Fr.row_ptr[r]; k < Fr.row_ptr[r + 1]; ++k) emit(Fr.col[k], k);
             });
+            if (!fits) return kTooLong;
         }
         H.lev.push_back(std::move(C));
     }

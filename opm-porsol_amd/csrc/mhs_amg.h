@@ -11,6 +11,8 @@
 #pragma once
 
 #include <array>
+#include <cstddef>
+#include <cstdint>
 #include <string>
 #include <vector>
 
@@ -20,13 +22,21 @@ namespace mhs {
 
 constexpr int kMaxCoarsest = 64;  // largest coarsest system per instance (dense inverse)
 
+// Ends of the gather lists.  Positions in the lists fit 31 bits, but a list is
+// longer than the array it gathers from: a face between two blocks is in both
+// blocks' lists, so A P's hold up to twice the face matrix's entries (which
+// stay below 2^31), level 1's about 1.6 times and level 2's pairs 1.5 times.
+// kMaxList leaves room below 2^32 for the widest step of the kernels' loops.
+using ListEnd = uint32_t;
+constexpr size_t kMaxList = 0xffff0000u;
+
 struct AmgLevel {
     int n = 0;                      // rows (all instances, unpadded)
     std::vector<int> inst_ptr;      // [ninst+1] first row of each instance
     std::vector<int> dims;          // [3 * ninst] block dimensions per instance
     std::vector<int> row_ptr, col;  // CSR pattern (columns sorted)
     std::vector<int> diag;          // position of the diagonal in each row
-    std::vector<int> src_ptr;       // [nnz+1] gather list ranges
+    std::vector<ListEnd> src_ptr;   // [nnz+1] gather list ranges
     std::vector<int> src;           // positions in the finer level's value array (level 1, ~pos: half of it)
     std::vector<int> agg;           // [n_finer] row of this level each finer row feeds (-1: none)
     // level 1: second aggregate of a face between two blocks (-1: the face lies
@@ -44,11 +54,13 @@ struct AmgLevel {
     // level, T = A P, and P transposed for the restriction.
     bool sa_out = false;
     std::vector<int> p_ptr, p_col, p_own;      // P rows; p_own[i]: entry of row i in its own aggregate
-    std::vector<int> p_src_ptr, p_src;         // per P entry: positions of this level's values
+    std::vector<ListEnd> p_src_ptr;
+    std::vector<int> p_src;                    // per P entry: positions of this level's values
     std::vector<int> pt_ptr, pt_col, pt_map;   // rows of the coarser level: fine row, P position
     std::vector<int> p_tpos;                   // per P entry: its position in the P' rows (inverse of pt_map)
     std::vector<int> t_ptr, t_col;             // T = A P
-    std::vector<int> t_pair_ptr, t_pa, t_pb;   // per T entry: (value position, P position)
+    std::vector<ListEnd> t_pair_ptr;
+    std::vector<int> t_pa, t_pb;               // per T entry: (value position, P position)
     std::vector<int> t_p;                      // per T entry: the P entry of the same row and column, or -1
 };
 
@@ -60,7 +72,7 @@ struct AmgLevel {
 struct ApPattern {
     std::vector<long long> slice_ptr;  // [nslices+1]
     std::vector<int> col;              // level-1 row of each slot
-    std::vector<int> src_ptr;          // [slots+1]
+    std::vector<ListEnd> src_ptr;      // [slots+1]
     std::vector<int> src;              // face-matrix SELL positions (~pos: half the entry)
     std::vector<int> slice;            // [slots/64] slice of each group of 64 slots
 };
@@ -123,8 +135,10 @@ std::string instance_dims(const Topology &T, const std::vector<int> &ijk, std::v
 // matrix to level 1 is the tentative (piecewise-constant) one; with smoothed
 // = true one coarse transfer is smoothed (the first from a level with at most
 // an eighth as many rows as faces), the others stay tentative.  Returns an
-// empty string on success.
+// empty string on success.  A grid whose lists would pass max_list entries is
+// refused.
 std::string build_amg(AmgHierarchy &H, const Topology &T, const std::vector<int> &ijk,
-                      const Strength &strength = {1.0, 1.0, 1.0}, bool smoothed = true);
+                      const Strength &strength = {1.0, 1.0, 1.0}, bool smoothed = true,
+                      size_t max_list = kMaxList);
 
 }  // namespace mhs

@@ -129,6 +129,7 @@ struct mhs_solver {
     // multigrid hierarchy
     std::vector<int> ijk;
     bool has_amg = false;
+    bool ap_elements_off = false;       // no A P lists over the element values (see ensure_ap_elements)
     AmgHierarchy H;
     DevAmg dA{};
     std::vector<DevBuf> amg_bufs;       // structure of the hierarchy on the device
@@ -229,7 +230,7 @@ void mhs_solver::free_amg() {
     amg_planned = false;
     dA = DevAmg{};
     setup_gen = -1;
-    has_amg = false;
+    has_amg = ap_elements_off = false;
     H = AmgHierarchy();
     rho.clear();
     shapes.clear();
@@ -999,16 +1000,21 @@ int ensure_matrix(mhs_solver *s) {
 }
 
 // Gather lists of the level-1 A P slots over the FP64 element values (built
-// on first need, kept with the hierarchy).
+// on first need, kept with the hierarchy).  Where they cannot be had
+// (ap_elements_off) the solves fill the face matrix and sum A P from it.
 int ensure_ap_elements(mhs_solver *s) {
     DevAmg &A = s->dA;
-    if (A.ap_esrc_ptr) return MHS_OK;
+    if (A.ap_esrc_ptr || s->ap_elements_off) return MHS_OK;
     if (!s->ebe_ok || A.nlev < 2) return fail(s, MHS_ERR_STATE, "element A P: no element layout or hierarchy");
-    std::vector<int> ptr, src;
+    std::vector<ListEnd> ptr;
+    std::vector<int> src;
     const std::string e = ebe_ap_lists(s->EL, s->T, s->H.ap, s->H.lev[1].agg, s->H.lev[1].agg2, ptr, src);
-    if (!e.empty()) return fail(s, MHS_ERR_INVALID, "element A P: " + e);
+    if (!e.empty()) {
+        s->ap_elements_off = true;
+        return MHS_OK;
+    }
     hipError_t he = hipSuccess;
-    const int *dp = dupload(s, s->amg_bufs, ptr, &he);
+    const ListEnd *dp = dupload(s, s->amg_bufs, ptr, &he);
     const int *ds = he == hipSuccess ? dupload(s, s->amg_bufs, src, &he) : nullptr;
     if (he != hipSuccess) return fail(s, MHS_ERR_ALLOC, std::string("element A P: ") + hipGetErrorString(he));
     A.ap_esrc_ptr = dp;
@@ -1500,10 +1506,11 @@ int solve_impl(mhs_solver *s, const double *totmob, const double *rhomob, const 
         const bool rho_known = opt.smoother_weight > 0.0 ||
                                (!s->rho.empty() && s->rho_gen == s->perm_gen &&
                                 s->rho_aniso == (binv_use != nullptr));
-        const bool no_matrix = mixed && ebe_settled && !fill32 && (!will_amg || rho_known);
+        bool no_matrix = mixed && ebe_settled && !fill32 && (!will_amg || rho_known);
         if (no_matrix && will_amg) {
             const int ra = ensure_ap_elements(s);
             if (ra) return ra;
+            no_matrix = s->dA.ap_esrc_ptr != nullptr;
         }
         HIPCHECK(launch_fill(s->stream, s->dT, nrhs, s->C, s->ftype, d_bv, s->inst_reg, dguess, s->val64,
                              fill32, s->b, s->dinv64, s->dinv32, s->x64, s->r64, no_matrix ? FILL_VEC : FILL_ALL));

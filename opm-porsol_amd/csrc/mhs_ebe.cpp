@@ -48,7 +48,8 @@ int greedy_colours(int nc, const int *facepos, const int *nb, std::vector<int> &
 }
 
 std::string ebe_ap_lists(const EbeLayout &E, const Topology &T, const ApPattern &ap, const std::vector<int> &agg,
-                         const std::vector<int> &agg2, std::vector<int> &ptr, std::vector<int> &src) {
+                         const std::vector<int> &agg2, std::vector<ListEnd> &ptr, std::vector<int> &src,
+                         size_t max_list) {
     const long long slots = (long long)ap.col.size();
     if (slots >= 0x7fffffffLL || E.nval >= 0x7fffffffLL) return "too many values for 32-bit lists";
     // slot of (row f, aggregate J): the row's slots are few (about 7)
@@ -65,10 +66,13 @@ std::string ebe_ap_lists(const EbeLayout &E, const Topology &T, const ApPattern 
     ptr.assign(slots + 1, 0);
     // two passes: counts, then the lists in slot order
     for (int pass = 0; pass < 2; ++pass) {
-        std::vector<int> fill;
+        std::vector<ListEnd> fill;
         if (pass == 1) {
+            size_t n = 0;
+            for (long long q = 0; q < slots; ++q) n += ptr[q + 1];
+            if (n > std::min(max_list, kMaxList)) return "too many entries for 32-bit lists";
             for (long long q = 0; q < slots; ++q) ptr[q + 1] += ptr[q];
-            src.assign(ptr[slots], 0);
+            src.assign(n, 0);
             fill.assign(ptr.begin(), ptr.end() - 1);
         }
         for (int c = 0; c < T.nc; ++c) {

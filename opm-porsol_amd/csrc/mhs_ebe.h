@@ -65,9 +65,11 @@ int greedy_colours(int nc, const int *facepos, const int *nb, std::vector<int> &
 // every cell whose local face i is row f and whose local face j has its row in
 // aggregate J (half the entry, listed as ~position, when that row has two).  With the Dirichlet rules inside the element values this is
 // the face matrix's A P.  ptr[slots + 1], src: positions in the packed values.
-// Returns "" or why the layout does not cover the pattern.
+// Returns "" or why the layout does not cover the pattern (or the lists would
+// pass max_list entries).
 std::string ebe_ap_lists(const EbeLayout &E, const Topology &T, const ApPattern &ap, const std::vector<int> &agg,
-                         const std::vector<int> &agg2, std::vector<int> &ptr, std::vector<int> &src);
+                         const std::vector<int> &agg2, std::vector<ListEnd> &ptr, std::vector<int> &src,
+                         size_t max_list = kMaxList);
 
 // Builds the layout for a structure; returns an empty string, or the reason
 // why the element-by-element operator does not apply (periodic faces, whose

@@ -115,7 +115,8 @@ struct DevAmgLevel {
     int n, nnz;
     long long nsrc;                 // entries of the src (and src2) lists
     const int *inst_ptr;            // [ninst+1] first row of each instance
-    const int *row_ptr, *col, *diag, *src_ptr, *src;
+    const int *row_ptr, *col, *diag, *src;
+    const uint32_t *src_ptr;        // (ends of lists: see ListEnd)
     const int *agg;                 // rows of the finer level -> rows of this level
     const int *child_ptr, *child;   // rows of this level -> rows of the finer level (level 1: ~f with half weight)
     size_t nchild;
@@ -128,12 +129,13 @@ struct DevAmgLevel {
     int sa_in, sa_out, p_nnz, t_nnz;
     long long t_npair;              // entries of the T pair lists
     const int *src2;
-    const int *p_ptr, *p_col, *p_own, *p_src_ptr, *p_src;
+    const int *p_ptr, *p_col, *p_own, *p_src;
+    const uint32_t *p_src_ptr, *t_pair_ptr;
     const int *pt_ptr, *pt_col, *pt_map;
     const int *p_tpos;              // per P entry: its position in the P' rows
     double *pt_val64;               // P values in P' row order (refilled with P)
     float *pt_val32;
-    const int *t_ptr, *t_col, *t_pair_ptr, *t_pa, *t_pb;
+    const int *t_ptr, *t_col, *t_pa, *t_pb;
     double *p_val64, *t_val64;
     float *p_val32, *t_val32;
     // M = P - w D^-1 T on T's pattern: the up-sweep's prolongation and
@@ -177,13 +179,15 @@ struct DevAmg {
     const int *agg2;
     const int *ap_slice;            // slice of each group of 64 slots
     const long long *ap_slice_ptr;
-    const int *ap_col, *ap_src_ptr, *ap_src;
+    const uint32_t *ap_src_ptr;
+    const int *ap_col, *ap_src;
     long long ap_slots, ap_nsrc;
     double *ap64;
     float *ap32;
     // the same slots as sums of the FP64 element values S'_c (element-by-
     // element layout), for solves that fill no face matrix (null: none)
-    const int *ap_esrc_ptr, *ap_esrc;
+    const uint32_t *ap_esrc_ptr;
+    const int *ap_esrc;
     long long ap_ensrc;
 };
 

@@ -1464,7 +1464,7 @@ __device__ __forceinline__ VT listed(const VT *__restrict__ v, int p) {
 // out[e] = sum of fine[src[k]] over the gather list of entry e, G lanes per
 // entry (coalesced list reads, several gathers in flight per lane).
 template <int G>
-__global__ __launch_bounds__(256) void k_galerkin(int nnz, const int *__restrict__ src_ptr,
+__global__ __launch_bounds__(256) void k_galerkin(int nnz, const uint32_t *__restrict__ src_ptr,
                                                   const int *__restrict__ src,
                                                   const double *__restrict__ fine,
                                                   double *__restrict__ out64,
@@ -1474,8 +1474,8 @@ __global__ __launch_bounds__(256) void k_galerkin(int nnz, const int *__restrict
     const int e = t / G, sub = t % G;
     if (e >= nnz) return;
     double s[1] = {0.0};
-    const int k1 = src_ptr[e + 1];
-    for (int k = src_ptr[e] + sub; k < k1; k += G * KC) {
+    const uint32_t k1 = src_ptr[e + 1];   // (k + G KC cannot wrap: kMaxList)
+    for (uint32_t k = src_ptr[e] + sub; k < k1; k += G * KC) {
         int q[KC];
 #pragma unroll
         for (int u = 0; u < KC; ++u) q[u] = k + G * u < k1 ? src[k + G * u] : 0;
@@ -1503,7 +1503,7 @@ __device__ __forceinline__ double m0_entry(double ap, bool empty, bool dir, int 
 template <bool M0>
 __global__ __launch_bounds__(256) void k_ap_fill(long long slots, const int *__restrict__ slot_slice,
                                                  const int *__restrict__ dof_hf, const uint8_t *__restrict__ ftype,
-                                                 const int *__restrict__ src_ptr, const int *__restrict__ src,
+                                                 const uint32_t *__restrict__ src_ptr, const int *__restrict__ src,
                                                  const double *__restrict__ fine, double *__restrict__ out,
                                                  const int *__restrict__ col, const int *__restrict__ agg,
                                                  const int *__restrict__ agg2, const double *__restrict__ dinv,
@@ -1511,9 +1511,9 @@ __global__ __launch_bounds__(256) void k_ap_fill(long long slots, const int *__r
     const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
     if (q >= slots) return;
     const int f = slot_slice[q >> 6] * 64 + (int)(q & 63), h = dof_hf[f];
-    const int k0 = src_ptr[q], k1 = src_ptr[q + 1];
+    const uint32_t k0 = src_ptr[q], k1 = src_ptr[q + 1];
     double s = 0.0;
-    for (int k = k0; k < k1; k += 4) {
+    for (uint32_t k = k0; k < k1; k += 4) {
         int p[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) p[u] = k + u < k1 ? src[k + u] : 0;
@@ -1533,7 +1533,7 @@ __global__ __launch_bounds__(256) void k_ap_fill(long long slots, const int *__r
 template <typename VT>
 __global__ __launch_bounds__(256) void k_ap_m0(long long slots, const int *__restrict__ slot_slice,
                                                const int *__restrict__ dof_hf, const uint8_t *__restrict__ ftype,
-                                               const int *__restrict__ src_ptr, const int *__restrict__ col,
+                                               const uint32_t *__restrict__ src_ptr, const int *__restrict__ col,
                                                const int *__restrict__ agg, const int *__restrict__ agg2,
                                                const double *__restrict__ dinv, double w, const double *ap, VT *out) {
     const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
@@ -1564,7 +1564,7 @@ __global__ __launch_bounds__(256) void k_sa_p(DevAmgLevel F, double wp) {
     const double d = F.dinv64[i];
     for (int q = F.p_ptr[i] + sub; q < F.p_ptr[i + 1]; q += G) {
         double s = 0.0;
-        for (int k = F.p_src_ptr[q]; k < F.p_src_ptr[q + 1]; ++k) s += F.val64[F.p_src[k]];
+        for (uint32_t k = F.p_src_ptr[q]; k < F.p_src_ptr[q + 1]; ++k) s += F.val64[F.p_src[k]];
         const double v = (q == F.p_own[i] ? 1.0 : 0.0) - wp * d * s;
         F.p_val64[q] = v;
         if (F.p_val32) F.p_val32[q] = (float)v;
@@ -1598,7 +1598,7 @@ __global__ __launch_bounds__(256) void k_sa_m(DevAmgLevel F, double w) {
 // out[e] = sum over the pairs of entry e of a[pa] * b[pb] (T = A P, A_c = P' T),
 // G lanes per entry.
 template <int G>
-__global__ __launch_bounds__(256) void k_pair_sum(int n, const int *__restrict__ ptr,
+__global__ __launch_bounds__(256) void k_pair_sum(int n, const uint32_t *__restrict__ ptr,
                                                   const int *__restrict__ pa, const int *__restrict__ pb,
                                                   const double *__restrict__ a, const double *__restrict__ b,
                                                   double *__restrict__ out64, float *__restrict__ out32) {
@@ -1607,8 +1607,8 @@ __global__ __launch_bounds__(256) void k_pair_sum(int n, const int *__restrict__
     const int e = t / G, sub = t % G;
     if (e >= n) return;
     double s[1] = {0.0};
-    const int k1 = ptr[e + 1];
-    for (int k = ptr[e] + sub; k < k1; k += G * KC) {
+    const uint32_t k1 = ptr[e + 1];
+    for (uint32_t k = ptr[e] + sub; k < k1; k += G * KC) {
         int ia[KC], ib[KC];
 #pragma unroll
         for (int u = 0; u < KC; ++u) {

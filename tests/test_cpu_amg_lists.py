@@ -1,0 +1,44 @@
+"""Host-side gather lists of the multigrid set-up: what their 32-bit ends can
+hold is checked on the lists themselves (a face between two blocks is in both
+blocks' lists, so they are longer than the face matrix)."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+STRENGTHS = [("1", "1", "1"), ("1", "1", "0.1"), ("0.1", "0.1", "1")]   # blocks 2x2x2, 2x2x1, 1x1x2
+
+
+@pytest.fixture(scope="module")
+def checker(pkg, tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("amg") / "amg_lists_check")
+    here = os.path.join(ROOT, "opm-porsol_amd")
+    cmd = ["g++", "-O1", "-std=c++17", "-Wall", "-pthread", "-I", os.path.join(here, "csrc"), "-I",
+           os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "amg_lists_check.cpp"), "-o", exe, "-L", here,
+           "-lmhs", f"-Wl,-rpath,{here}"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout + res.stderr
+
+    def run(strength, dims, limit=0, element_limit=0, threads=2):
+        cmd = [exe, str(threads), *strength, str(limit), str(element_limit), *map(str, dims)]
+        res = subprocess.run(cmd, capture_output=True, text=True, timeout=120)
+        assert res.returncode == 0, res.stdout + res.stderr
+        return dict(line.split(" ", 1) for line in res.stdout.splitlines())
+
+    return run
+
+
+@pytest.mark.parametrize("strength", STRENGTHS)
+@pytest.mark.parametrize("dims", [(12, 11, 9), (8, 8, 8, 5, 4, 7)])
+def test_lists_past_the_limit_are_refused(checker, strength, dims):
+    ok = checker(strength, dims)
+    assert ok["amg"] == ok["element"] == "ok"
+    # longer than the face matrix that used to bound them, by less than the ends' extra bit
+    assert int(ok["matrix"]) < int(ok["ap"]) <= 2 * int(ok["matrix"])
+    assert int(ok["longest"]) <= 2 * int(ok["matrix"])
+    n, m = int(ok["longest"]), int(ok["element_list"])
+    assert checker(strength, dims, limit=n)["hash"] == ok["hash"]
+    assert "too large" in checker(strength, dims, limit=n - 1)["amg"]
+    assert checker(strength, dims, element_limit=m)["hash"] == ok["hash"]
+    assert "too many entries" in checker(strength, dims, element_limit=m - 1)["element"]
