@@ -1543,13 +1543,17 @@ __global__ __launch_bounds__(256) void k_ap_m0(long long slots, const int *__res
     out[q] = (VT)m0_entry(ap[q], src_ptr[q + 1] == src_ptr[q], dir, col[q], agg[f], agg2[f], w * dinv[f]);
 }
 
+// Inverse diagonals of a coarse level.  A block all of whose faces are Dirichlet
+// faces (a one-cell instance, a cell cut off from the others) has a zero row and
+// column: the cycle leaves those faces out, its residual is zero, and with 1 for
+// the diagonal so is its correction.
 __global__ __launch_bounds__(256) void k_coarse_diag(int n, const int *__restrict__ diag,
                                                      const double *__restrict__ val,
                                                      double *__restrict__ dinv64,
                                                      float *__restrict__ dinv32) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    const double d = 1.0 / val[diag[i]];
+    const double a = val[diag[i]], d = a != 0.0 ? 1.0 / a : 1.0;
     dinv64[i] = d;
     if (dinv32) dinv32[i] = (float)d;
 }
@@ -1626,7 +1630,8 @@ __global__ __launch_bounds__(256) void k_pair_sum(int n, const uint32_t *__restr
 }
 
 // Dense inverse of each instance's coarsest operator (Gauss-Jordan, no
-// pivoting: the Galerkin operators are symmetric positive definite).  Per
+// pivoting: the Galerkin operators are symmetric positive definite, but for
+// zero rows and columns, which get 1 on the diagonal as in k_coarse_diag).  Per
 // pivot: the scaled pivot row and the pivot column go to their own arrays,
 // then every thread updates its own entries of the matrix; two barriers.
 __global__ __launch_bounds__(1024) void k_coarse_inverse(DevAmgLevel L, const int *__restrict__ inst_ptr,
@@ -1642,8 +1647,10 @@ __global__ __launch_bounds__(1024) void k_coarse_inverse(DevAmgLevel L, const in
     for (int e = tid; e < M * M; e += NT) A[e / M][e % M] = 0.0;
     __syncthreads();
     for (int i = tid; i < m; i += NT)
-        for (int k = L.row_ptr[r0 + i]; k < L.row_ptr[r0 + i + 1]; ++k)
-            A[i][L.col[k] - r0] = L.val64[k];
+        for (int k = L.row_ptr[r0 + i]; k < L.row_ptr[r0 + i + 1]; ++k) {
+            const int j = L.col[k] - r0;
+            A[i][j] = j == i && L.val64[k] == 0.0 ? 1.0 : L.val64[k];
+        }
     __syncthreads();
     for (int k = 0; k < m; ++k) {
         if (tid < M) {
