@@ -47,7 +47,7 @@ struct TempBufs {
 
 struct GraphCache {
     hipGraphExec_t exec = nullptr;
-    int precision = -1, nrhs = 0, chunk = 0, amg = -1, nu = -1, ebe = -1;
+    int precision = -1, nrhs = 0, chunk = 0, amg = -1, nu = -1, ebe = -1, dirichlet_res = -1;
     int shape[5] = {-1, -1, -1, -1, -1};
     double tol2 = -1.0, rf2 = -1.0, alpha = -1.0;
     double omega[kMaxLevels] = {};
@@ -945,7 +945,7 @@ int run_chunk(mhs_solver *s, int nrhs, int chunk, bool use_graph, const MT *val,
         if (!(G.exec && G.precision == precision && G.nrhs == nrhs && G.chunk == chunk && G.ebe == ebe &&
               G.key == (const void *)val && G.tol2 == tol2 && G.rf2 == s->S.rf2 && G.amg == int(amg) &&
               std::equal(G.omega, G.omega + kMaxLevels, s->dA.omega_l) && G.alpha == s->dA.alpha &&
-              G.nu == s->dA.nu &&
+              G.nu == s->dA.nu && G.dirichlet_res == s->dA.dirichlet_res &&
               std::equal(shape, shape + 5, G.shape))) {
             if (G.exec) (void)hipGraphExecDestroy(G.exec);
             G = GraphCache{};
@@ -977,6 +977,7 @@ int run_chunk(mhs_solver *s, int nrhs, int chunk, bool use_graph, const MT *val,
             std::copy(s->dA.omega_l, s->dA.omega_l + kMaxLevels, G.omega);
             G.alpha = s->dA.alpha;
             G.nu = s->dA.nu;
+            G.dirichlet_res = s->dA.dirichlet_res;
             std::copy(shape, shape + 5, G.shape);
         }
         HIPCHECK(hipGraphLaunch(G.exec, s->stream));
@@ -1474,9 +1475,7 @@ int solve_impl(mhs_solver *s, const double *totmob, const double *rhomob, const 
     s->solved = false;
     s->last_aniso = binv_use != nullptr;
     const double *binv = binv_use ? binv_use : s->binv, *gflux = gflux_use ? gflux_use : s->gflux;
-    // AMG types start from the Dirichlet guess (:1521-1532); the multigrid cycle
-    // leaves Dirichlet rows out, so with it their residual must be zero
-    const int dguess = opt.linsolver_type != 0 || (opt.precond == 1 && s->has_amg);
+    const int dguess = opt.linsolver_type != 0;  // AMG types start from the Dirichlet guess (:1521-1532)
     float *fill32 = nullptr;
     bool filled_matrix = true;
     auto assemble = [&]() -> int {
@@ -1575,6 +1574,7 @@ int solve_impl(mhs_solver *s, const double *totmob, const double *rhomob, const 
             s->dA.alpha = 1.0 + (opt.prolongate_factor - 1.0) * (5.0 / 6.0);
             s->dA.alpha_f = 1.0 + (opt.prolongate_factor - 1.0) * 0.5;
             s->dA.nu = std::max(1, opt.smooth_steps);
+            s->dA.dirichlet_res = dguess ? 0 : 1;
             // same_matrix (the caller's promise, :1491): the coarse levels,
             // the smoothed transfer and the coarsest inverses of the previous
             // solve are kept, as the reference keeps its AMG hierarchy; A P,

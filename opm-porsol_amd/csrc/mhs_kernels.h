@@ -167,6 +167,7 @@ struct DevAmg {
     float *tail_val32;
     int tail_first;
     int tail_iend[kMaxLevels], tail_vend[kMaxLevels], tail_vec[kMaxLevels];
+    int dirichlet_res;              // 1: the residual of Dirichlet rows is not zero (see k_clear_dirichlet)
     int nu;                         // smoothing sweeps before and after the coarse correction
     int max_rows[kMaxLevels];       // rows of the largest instance on each level
     int max_children[kMaxLevels];   // most finer rows aggregated into one row of each level

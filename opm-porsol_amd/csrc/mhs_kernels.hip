@@ -1886,6 +1886,20 @@ __device__ __forceinline__ void up_sa_row(const DevAmgLevel &F, const VT *__rest
     }
 }
 
+// Clears the residual of the Dirichlet rows.  The cycle leaves them out (the
+// transfers to and from level 1 hold no entry for them), and where the iteration
+// starts from zero theirs is not zero: restricting it would make the cycle
+// unsymmetric.  The smoother still sees it in r.
+template <typename VT, int NRHS>
+__global__ __launch_bounds__(256) void k_clear_dirichlet(const int *__restrict__ dof_hf,
+                                                         const uint8_t *__restrict__ ftype, VT *__restrict__ res) {
+    const int f = blockIdx.x * 256 + threadIdx.x;
+    const int h = dof_hf[f];
+    if (h < 0 || ftype[h] != FT_DIRICHLET) return;
+#pragma unroll
+    for (int k = 0; k < NRHS; ++k) res[(size_t)f * NRHS + k] = VT(0);
+}
+
 // Level 0, one more Jacobi sweep: xo = x + w D^-1 (b - A x).  LAST: the final sweep
 // of the V-cycle writes the preconditioned residual and <r, z> partials.
 template <typename VT, int NRHS, bool LAST, int TB>
@@ -3781,6 +3795,7 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
             });
         });
     }
+    if (A.dirichlet_res) k_clear_dirichlet<VT, NR><<<rows_blocks, 256, 0, st>>>(T.dof_hf, ftype, res0);
     {
         const DevAmgLevel &C = A.lev[1];
         with_lanes(lanes_per_row((long long)C.nchild, C.n), [&](auto g) {

@@ -89,3 +89,34 @@ def test_post_sweep_written_with_known_weights(pkg, orc, dims, element_operator)
         assert cases.rel_err(s.getSolution()[2], ref.outflux) < 1e-8
     # the same preconditioner up to the order of FP32 sums
     assert max(its) - min(its) <= 2
+
+
+@pytest.mark.parametrize("precision,element_operator", [("fp64", 0), ("mixed", 0), ("mixed", 2)])
+@pytest.mark.parametrize("precond", [0, 1])
+@pytest.mark.parametrize("smooth_steps", [1, 2])
+@pytest.mark.parametrize("solver", [0, 1])
+def test_reduction_is_relative_to_the_solver_types_start(pkg, solver, smooth_steps, precond, precision,
+                                                         element_operator):
+    """Solver type 0 starts from zero, the others from the Dirichlet values, with
+    either preconditioner: the residual that the tolerance is relative to."""
+    import scipy.sparse as sp
+    g = pkg.grids.cartesian(13, 10, 6, 1.0, 1.0, 0.5)
+    nc = g.num_cells
+    bt, bv = cases.xdrop_bc(g, 30.0, 29.0)
+    tm, rm = cases.unit_fluid(nc)
+    s = pkg.HybridSolver(0)
+    s.init(g, pkg.fields.perm_c1(nc, 8), (0, 0, 0), bt, None)
+    s.solve(tm, rm, np.zeros(nc), bt, bv, residual_tolerance=1e-5, precision=precision, precond=precond,
+            linsolver_type=solver, smooth_steps=smooth_steps, element_operator=element_operator)
+    x = np.asarray(s.getSolution()[1])
+    ptr, col, val, b = s.system()
+    A = sp.csr_matrix((val, col, ptr), shape=(b.shape[0],) * 2)
+    x0 = np.zeros_like(b)
+    if solver:
+        # Dirichlet rows are the ones with a single nonzero entry
+        off = np.asarray(abs(A - sp.diags(A.diagonal())).sum(axis=1)).reshape(-1)
+        x0 = np.where(off == 0, b / A.diagonal(), 0.0)
+    r, r0 = np.linalg.norm(b - A @ x), np.linalg.norm(b - A @ x0)
+    assert s.report.reduction <= 1e-5
+    # the report's own FP64 residual of the same x, up to the rounding of A x (1e-16 of |b|)
+    assert abs(s.report.reduction - r / r0) < 1e-4 * s.report.reduction + 1e-12
