@@ -510,6 +510,7 @@ int build_amg_device(mhs_solver *s, const Strength &strength) {
         if (he == hipSuccess) A.tail_val64 = dalloc<double>(s, L, (size_t)s->H.tail.nval, &he);
         if (he == hipSuccess) A.tail_val32 = dalloc<float>(s, L, (size_t)s->H.tail.nval, &he);
         A.tail_first = s->H.tail.first;
+        A.tail_lds = tail_lds_limit();
         for (int l = 0; l < A.nlev; ++l) {
             A.tail_iend[l] = s->H.tail.iend[l];
             A.tail_vend[l] = s->H.tail.vend[l];

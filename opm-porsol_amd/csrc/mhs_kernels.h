@@ -166,6 +166,7 @@ struct DevAmg {
     double *tail_val64;
     float *tail_val32;
     int tail_first;
+    int tail_lds;                   // LDS the tail may take (tail_lds_limit on the hierarchy's device)
     int tail_iend[kMaxLevels], tail_vend[kMaxLevels], tail_vec[kMaxLevels];
     int dirichlet_res;              // 1: the residual of Dirichlet rows is not zero (see k_clear_dirichlet)
     int nu;                         // smoothing sweeps before and after the coarse correction
@@ -264,6 +265,10 @@ hipError_t launch_merge_all(hipStream_t st, const DevTopo &T, int nrhs, double *
 hipError_t launch_clear_state(hipStream_t st, const DevScal &S, int nsys, float *x32, long long nx);
 hipError_t launch_resnorm(hipStream_t st, const DevTopo &T, int nrhs, const double *val64,
                           const double *b, const double *x64, DevRed R, DevScal S);
+
+// LDS that the one-workgroup tail may take on the current device: kTailBytes, or
+// what a launch may take without asking where asking is refused.
+int tail_lds_limit();
 
 // Multigrid: per-solve set-up (Galerkin products, diagonals, coarsest inverses)
 // and the preconditioned iteration pieces.

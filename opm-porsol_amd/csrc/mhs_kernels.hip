@@ -3761,7 +3761,22 @@ static inline long long tail_bytes(const DevAmg &A, int lt) {
 }
 template <typename VT, int NR>
 static inline bool tail_fits(const DevAmg &A, int lt) {
-    return lt >= A.tail_first && tail_bytes<VT, NR>(A, lt) <= kTailBytes;
+    return lt >= A.tail_first && tail_bytes<VT, NR>(A, lt) <= A.tail_lds;
+}
+// The attribute belongs to the kernels of the current device: every hierarchy
+// asks for it on its own.
+int tail_lds_limit() {
+    const void *const kernels[] = {
+        reinterpret_cast<const void *>(&k_vcycle_tail<double, 1>), reinterpret_cast<const void *>(&k_vcycle_tail<double, 2>),
+        reinterpret_cast<const void *>(&k_vcycle_tail<double, 3>), reinterpret_cast<const void *>(&k_vcycle_tail<double, 4>),
+        reinterpret_cast<const void *>(&k_vcycle_tail<float, 1>),  reinterpret_cast<const void *>(&k_vcycle_tail<float, 2>),
+        reinterpret_cast<const void *>(&k_vcycle_tail<float, 3>),  reinterpret_cast<const void *>(&k_vcycle_tail<float, 4>)};
+    for (const void *k : kernels)
+        if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kTailBytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return 64 * 1024;
+        }
+    return kTailBytes;
 }
 
 // gt: inside the PCG loop the V-cycle skips the level-0 blocks and the tail
@@ -3869,10 +3884,6 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
         }
         const VT *tv;
         if constexpr (std::is_same<VT, float>::value) tv = A.tail_val32; else tv = A.tail_val64;
-        static const hipError_t lds_ok = hipFuncSetAttribute(
-            reinterpret_cast<const void *>(&k_vcycle_tail<VT, NR>), hipFuncAttributeMaxDynamicSharedMemorySize,
-            kTailBytes);
-        (void)lds_ok;   // where it is refused, a launch that needs it reports its own error
         const int vbase = tail_vbase(A, lt), xbase = tail_xbase<VT>(A, lt);
         k_vcycle_tail<VT, NR><<<A.ninst, 1024, (unsigned)tail_bytes<VT, NR>(A, lt), st>>>(
             gt, A.tail_tab, A.tail_idx, tv, L, lt, vbase, xbase, (const VT *)A.lev[lt].b, (VT *)A.lev[lt].x, alw(0),

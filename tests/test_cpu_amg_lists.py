@@ -1,6 +1,7 @@
 """Host-side gather lists of the multigrid set-up: what their 32-bit ends can
 hold is checked on the lists themselves (a face between two blocks is in both
-blocks' lists, so they are longer than the face matrix)."""
+blocks' lists, so they are longer than the face matrix); and the LDS limit of the
+one-workgroup tail, which every handle sets on its own device."""
 import os
 import subprocess
 
@@ -42,3 +43,21 @@ def test_lists_past_the_limit_are_refused(checker, strength, dims):
     assert "too large" in checker(strength, dims, limit=n - 1)["amg"]
     assert checker(strength, dims, element_limit=m)["hash"] == ok["hash"]
     assert "too many entries" in checker(strength, dims, element_limit=m - 1)["element"]
+
+
+def test_tail_lds_limit_is_set_for_every_handle(pkg, tmp_path):
+    exe, here = str(tmp_path / "tail_limit_check"), os.path.join(ROOT, "opm-porsol_amd")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    cmd = ["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(rocm, "include"), "-I",
+           os.path.join(here, "csrc"), "-I", os.path.join(ROOT, "include"),
+           os.path.join(ROOT, "tests", "tail_limit_check.cpp"), "-o", exe, "-L", here, "-lmhs", f"-Wl,-rpath,{here}",
+           "-L", os.path.join(rocm, "lib"), "-lamdhip64", f"-Wl,-rpath,{os.path.join(rocm, 'lib')}"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout + res.stderr
+    out = [subprocess.run([exe, *a], capture_output=True, text=True, timeout=60) for a in ([], ["refuse"])]
+    assert [o.returncode for o in out] == [0, 0], out
+    lines = [[tuple(map(int, l.split())) for l in o.stdout.splitlines()] for o in out]
+    # two precisions, one to four right-hand sides, for each of the two handles
+    assert lines[0] == [(152 * 1024, 8, 8)] * 2
+    # refused: what a launch may take without asking
+    assert [l[0] for l in lines[1]] == [64 * 1024] * 2
