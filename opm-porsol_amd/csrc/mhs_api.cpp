@@ -137,7 +137,7 @@ struct mhs_solver {
     std::vector<double> rho;            // largest eigenvalue of D^-1 A per level (empty: not estimated)
     long long rho_gen = -1;             // permeability generation the estimate was made for
     bool rho_aniso = false;             // ... and whether that solve had tensor mobilities
-    double *lz[7] = {};                 // work arrays of that estimate (in amg_bufs, from the first one on)
+    double *lz = nullptr;               // work arrays of that estimate (in amg_bufs, from the first one on)
     double *z64 = nullptr;
     float *z32 = nullptr;
 
@@ -226,7 +226,7 @@ T *dupload(mhs_solver *s, std::vector<DevBuf> &list, const std::vector<T> &v, hi
 void mhs_solver::free_amg() {
     for (auto &b : amg_bufs) (void)hipFree(b.p);
     amg_bufs.clear();
-    std::fill(lz, lz + 7, nullptr);
+    lz = nullptr;
     amg_planned = false;
     dA = DevAmg{};
     setup_gen = -1;
@@ -1067,20 +1067,19 @@ int estimate_rho(mhs_solver *s) {
     if (const int rm = ensure_matrix(s)) return rm;
     const DevAmg &A = s->dA;
     const int nl = A.nlev - 1;
-    if (!s->lz[0]) {
-        const size_t n = lanczos_rows(s->dT, A), sizes[7] = {n, n, n, n, n, lanczos_parts(s->dT, A),
-                                                             (size_t)kLzState * kMaxLevels};
+    // five vectors over the rows of all levels, the partial sums and the state: one
+    // allocation, which is there or not
+    const size_t n = lanczos_rows(s->dT, A), np = lanczos_parts(s->dT, A);
+    if (!s->lz) {
         hipError_t he = hipSuccess;
-        for (int i = 6; i >= 0 && he == hipSuccess; --i) s->lz[i] = dalloc<double>(s, s->amg_bufs, sizes[i], &he);
-        if (he != hipSuccess) {
-            s->lz[0] = nullptr;
-            return fail(s, MHS_ERR_ALLOC, std::string("smoother weights: ") + hipGetErrorString(he));
-        }
+        s->lz = dalloc<double>(s, s->amg_bufs, 5 * n + np + (size_t)kLzState * kMaxLevels, &he);
+        if (he != hipSuccess) return fail(s, MHS_ERR_ALLOC, std::string("smoother weights: ") + hipGetErrorString(he));
     }
-    HIPCHECK(launch_lanczos(s->stream, s->dT, A, s->val64, s->dinv64, s->lz[0], s->lz[1], s->lz[2], s->lz[3], s->lz[4],
-                            s->lz[5], s->lz[6]));
+    double *const w = s->lz, *const part = w + 5 * n, *const state = part + np;
+    HIPCHECK(launch_lanczos(s->stream, s->dT, A, s->val64, s->dinv64, w, w + n, w + 2 * n, w + 3 * n, w + 4 * n, part,
+                            state));
     std::vector<double> st((size_t)kLzState * kMaxLevels);
-    HIPCHECK(hipMemcpyAsync(st.data(), s->lz[6], st.size() * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+    HIPCHECK(hipMemcpyAsync(st.data(), state, st.size() * sizeof(double), hipMemcpyDeviceToHost, s->stream));
     HIPCHECK(hipStreamSynchronize(s->stream));
     std::vector<double> rho(nl, 0.0);
     for (int l = 0; l < nl; ++l) {
