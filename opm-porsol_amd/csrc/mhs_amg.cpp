@@ -1,121 +1,15 @@
 // Aggregation multigrid hierarchy (host-side set-up); see mhs_amg.h.
 #include "mhs_amg.h"
+#include "mhs_lists.h"
 
 #include <algorithm>
 #include <array>
 #include <cmath>
-#include <exception>
 #include <numeric>
-#include <thread>
 
 namespace mhs {
 
 namespace {
-
-// Host threads for the row loops below (each row's lists depend on that row
-// alone): fn(t, begin, end) on contiguous ranges of [0, n), at least `least`
-// items each.  The hierarchy of 128x128x64 cells is 100M list entries.
-constexpr int kMaxThreads = 8;
-int ranges(int n, int least) {
-    const int hw = std::max(1u, std::thread::hardware_concurrency());
-    return std::max(1, std::min({n / std::max(1, least), hw, kMaxThreads}));
-}
-template <class Fn>
-void in_ranges(int n, int nt, Fn fn) {
-    std::vector<std::exception_ptr> err(nt);
-    auto run = [&](int t) {
-        try {
-            fn(t, int((long long)n * t / nt), int((long long)n * (t + 1) / nt));
-        } catch (...) {
-            err[t] = std::current_exception();
-        }
-    };
-    std::vector<std::thread> pool;
-    pool.reserve(nt);
-    int t = 1;
-    try {
-        for (; t < nt; ++t) pool.emplace_back(run, t);
-    } catch (...) {   // no more threads to be had: the rest runs here
-    }
-    run(0);
-    for (int u = t; u < nt; ++u) run(u);
-    for (auto &th : pool) th.join();
-    for (auto &e : err)
-        if (e) std::rethrow_exception(e);
-}
-// Appends the ranges' lists in order; returns where each one starts.
-template <class I>
-std::vector<size_t> append(std::vector<I> &out, const std::vector<std::vector<I>> &parts) {
-    std::vector<size_t> at(parts.size() + 1, out.size());
-    for (size_t t = 0; t < parts.size(); ++t) at[t + 1] = at[t] + parts[t].size();
-    out.resize(at.back());
-    in_ranges(int(parts.size()), int(parts.size()), [&](int, int b, int e) {
-        for (int t = b; t < e; ++t) std::copy(parts[t].begin(), parts[t].end(), out.begin() + at[t]);
-    });
-    return at;
-}
-
-size_t total(const std::vector<std::vector<int>> &parts) {
-    size_t n = 0;
-    for (const auto &p : parts) n += p.size();
-    return n;
-}
-// What the lists of one pattern may hold: positions of its entries are 32-bit
-// signed (~pos marks a half entry), the ends of its lists 32-bit unsigned.
-bool too_long(size_t entries, size_t list, size_t max_list) {
-    return entries > std::min<size_t>(max_list, 0x7fffffff) || list > std::min(max_list, kMaxList);
-}
-
-// Rows of a CSR pattern whose entries each carry a list, built range by range:
-// row(i, R) appends the row's columns to R.col and, per entry, its sources to
-// R.src (and R.src2) and their end to R.end.  False: too long.
-struct RowPart {
-    std::vector<int> col, src, src2, len;
-    std::vector<ListEnd> end;
-};
-template <class Row>
-bool build_rows(int n, std::vector<int> &ptr, std::vector<int> &col, std::vector<ListEnd> &src_ptr,
-                std::vector<int> &src, std::vector<int> *src2, size_t max_list, Row row) {
-    const int nt = ranges(n, 2048);
-    std::vector<RowPart> P(nt);
-    in_ranges(n, nt, [&](int t, int b, int e) {
-        RowPart &R = P[t];
-        R.len.reserve(e - b);
-        for (int i = b; i < e; ++i) {
-            const size_t c0 = R.col.size();
-            row(i, R);
-            R.len.push_back(int(R.col.size() - c0));
-        }
-    });
-    std::vector<std::vector<int>> cols(nt), srcs(nt), srcs2(nt);
-    std::vector<std::vector<ListEnd>> ends(nt);
-    for (int t = 0; t < nt; ++t) {
-        cols[t].swap(P[t].col);
-        srcs[t].swap(P[t].src);
-        srcs2[t].swap(P[t].src2);
-        ends[t].swap(P[t].end);
-    }
-    if (too_long(total(cols), total(srcs), max_list)) return false;
-    ptr.assign(n + 1, 0);
-    for (int t = 0, i = 0; t < nt; ++t)
-        for (int l : P[t].len) {
-            ptr[i + 1] = ptr[i] + l;
-            ++i;
-        }
-    col.clear();
-    src.clear();
-    append(col, cols);
-    const std::vector<size_t> at = append(src, srcs);
-    for (int t = 0; t < nt; ++t)
-        for (ListEnd &e : ends[t]) e += ListEnd(at[t]);
-    src_ptr.assign(1, 0);
-    append(src_ptr, ends);
-    if (src2) {
-        src2->clear();
-        append(*src2, srcs2);
-    }
-    return true;
-}
 
 void children(AmgLevel &C, int nf) {
     const bool two = !C.agg2.empty();
@@ -143,39 +37,36 @@ void find_diagonal(AmgLevel &C) {
 }
 
 // Sparsity of P'AP and the gather lists, coarse row by coarse row: the
-// entries (agg(j), pos) of the coarse row's children are sorted locally.
+// entries (agg(j), pos) of the coarse row's children by column.
 // row_entries(i, emit) must call emit(j, pos) for every stored entry of
 // finer row i (COARSE: j is already the coarse column, the entries being
 // those of A P).  Requires children() to have run.
 template <bool COARSE = false, class RowEntries>
 bool galerkin_pattern(AmgLevel &C, size_t max_list, RowEntries row_entries) {
-    const bool ok = build_rows(C.n, C.row_ptr, C.col, C.src_ptr, C.src, nullptr, max_list, [&](int I, RowPart &R) {
-        thread_local std::vector<std::pair<int, int>> buf;
-        buf.clear();
-        for (int k = C.child_ptr[I]; k < C.child_ptr[I + 1]; ++k)
-            row_entries(C.child[k], [&](int j, int pos) {
-                const int J = COARSE ? j : C.agg[j];
-                if (J >= 0) buf.emplace_back(J, pos);
+    const bool ok = build_rows(C.n, C.row_ptr, C.col, C.src_ptr, C.src, nullptr, max_list, [&]() {
+        return [&, rows = ByColumn<int>(C.n)](int I, RowPart &R) mutable {
+            rows.start();
+            for (int k = C.child_ptr[I]; k < C.child_ptr[I + 1]; ++k)
+                row_entries(C.child[k], [&](int j, int pos) {
+                    const int J = COARSE ? j : C.agg[j];
+                    if (J >= 0) rows.put(J, pos);
+                });
+            rows.finish([&](int J, int *e, int n) {
+                // by position whatever its weight (from CSR rows they come so)
+                if constexpr (COARSE)
+                    std::sort(e, e + n, [](int x, int y) { return std::max(x, ~x) < std::max(y, ~y); });
+                R.col.push_back(J);
+                R.src.insert(R.src.end(), e, e + n);
+                R.end.push_back(ListEnd(R.src.size()));
             });
-        // by column, then by position whatever its weight
-        std::sort(buf.begin(), buf.end(), [](const std::pair<int, int> &x, const std::pair<int, int> &y) {
-            return x.first != y.first ? x.first < y.first : std::max(x.second, ~x.second) < std::max(y.second, ~y.second);
-        });
-        for (size_t k = 0; k < buf.size(); ++k) {
-            if (k == 0 || buf[k].first != buf[k - 1].first) {
-                if (k > 0) R.end.push_back(ListEnd(R.src.size()));
-                R.col.push_back(buf[k].first);
-            }
-            R.src.push_back(buf[k].second);
-        }
-        if (!buf.empty()) R.end.push_back(ListEnd(R.src.size()));
+        };
     });
     if (ok) find_diagonal(C);
     return ok;
 }
 
-// False: too long.
-bool build_ap(ApPattern &P, const Topology &T, const std::vector<int> &agg, const std::vector<int> &agg2,
+// naggs: rows of level 1.  False: too long.
+bool build_ap(ApPattern &P, const Topology &T, int naggs, const std::vector<int> &agg, const std::vector<int> &agg2,
               size_t max_list) {
     const int ns = T.nslices, nt = ranges(ns, 32);
     P.slice_ptr.assign(ns + 1, 0);
@@ -187,7 +78,7 @@ bool build_ap(ApPattern &P, const Topology &T, const std::vector<int> &agg, cons
     std::vector<int> width(ns, 0);
     in_ranges(ns, nt, [&](int t, int b, int e) {
         Part &Q = parts[t];
-        std::vector<std::pair<int, int>> buf;
+        ByColumn<int> row(naggs);
         std::vector<std::vector<Run>> runs(kSlice);
         std::vector<int> pos;
         for (int sl = b; sl < e; ++sl) {
@@ -196,21 +87,20 @@ bool build_ap(ApPattern &P, const Topology &T, const std::vector<int> &agg, cons
             for (int l = 0; l < kSlice; ++l) {
                 const int f = sl * kSlice + l;
                 const long long base = T.slice_ptr[sl] + l;
-                buf.clear();
+                row.start();
                 for (int k = 0; k < T.row_len[f]; ++k) {
                     const long long p = base + (long long)k * kSlice;
                     const int j = T.col[p], J = agg[j], J2 = agg2[j];
-                    if (J >= 0) buf.emplace_back(J, J2 >= 0 ? ~int(p) : int(p));
-                    if (J2 >= 0) buf.emplace_back(J2, ~int(p));
+                    if (J >= 0) row.put(J, J2 >= 0 ? ~int(p) : int(p));
+                    if (J2 >= 0) row.put(J2, ~int(p));
                 }
-                std::sort(buf.begin(), buf.end());
                 auto &r = runs[l];
                 r.clear();
-                for (const auto &q : buf) {
-                    if (r.empty() || r.back().J != q.first) r.push_back({q.first, 0, int(pos.size())});
-                    r.back().n++;
-                    pos.push_back(q.second);
-                }
+                row.finish([&](int J, int *e, int n) {
+                    std::sort(e, e + n);
+                    r.push_back({J, n, int(pos.size())});
+                    pos.insert(pos.end(), e, e + n);
+                });
                 w = std::max(w, r.size());
             }
             width[sl] = int(w);
@@ -257,19 +147,16 @@ bool sa_transfer(AmgLevel &F, AmgLevel &C, size_t max_list) {
     const int n = F.n;
     F.sa_out = true;
     F.p_own.assign(n, -1);
-    if (!build_rows(n, F.p_ptr, F.p_col, F.p_src_ptr, F.p_src, nullptr, max_list, [&](int i, RowPart &R) {
-        thread_local std::vector<std::pair<int, int>> buf;
-        buf.clear();
-        for (int k = F.row_ptr[i]; k < F.row_ptr[i + 1]; ++k) buf.emplace_back(C.agg[F.col[k]], k);
-        std::sort(buf.begin(), buf.end());
-        for (size_t k = 0; k < buf.size(); ++k) {
-            if (k == 0 || buf[k].first != buf[k - 1].first) {
-                if (k > 0) R.end.push_back(ListEnd(R.src.size()));
-                R.col.push_back(buf[k].first);
-            }
-            R.src.push_back(buf[k].second);
-        }
-        if (!buf.empty()) R.end.push_back(ListEnd(R.src.size()));
+    if (!build_rows(n, F.p_ptr, F.p_col, F.p_src_ptr, F.p_src, nullptr, max_list, [&]() {
+        return [&, row = ByColumn<int>(C.n)](int i, RowPart &R) mutable {
+            row.start();
+            for (int k = F.row_ptr[i]; k < F.row_ptr[i + 1]; ++k) row.put(C.agg[F.col[k]], k);
+            row.finish([&](int J, int *e, int m) {
+                R.col.push_back(J);
+                R.src.insert(R.src.end(), e, e + m);
+                R.end.push_back(ListEnd(R.src.size()));
+            });
+        };
     })) return false;
     for (int i = 0; i < n; ++i)
         for (int q = F.p_ptr[i]; q < F.p_ptr[i + 1]; ++q)
@@ -291,38 +178,39 @@ bool sa_transfer(AmgLevel &F, AmgLevel &C, size_t max_list) {
         F.p_tpos.assign(F.p_col.size(), 0);
         for (size_t e = 0; e < F.pt_map.size(); ++e) F.p_tpos[F.pt_map[e]] = int(e);
     }
-    // T = A P, then A_C = P' T: sorted triples (column, the two factors' positions)
-    using Triples = std::vector<std::array<int, 3>>;
-    auto emit = [](Triples &tb, RowPart &R) {
-        std::sort(tb.begin(), tb.end());
-        for (size_t k = 0; k < tb.size(); ++k) {
-            if (k == 0 || tb[k][0] != tb[k - 1][0]) {
-                if (k > 0) R.end.push_back(ListEnd(R.src.size()));
-                R.col.push_back(tb[k][0]);
+    // T = A P, then A_C = P' T: per column the pairs of the two factors' positions,
+    // which come in ascending order
+    using Pair = std::pair<int, int>;
+    auto emit = [](ByColumn<Pair> &row, RowPart &R) {
+        row.finish([&](int J, const Pair *e, int m) {
+            R.col.push_back(J);
+            for (int k = 0; k < m; ++k) {
+                R.src.push_back(e[k].first);
+                R.src2.push_back(e[k].second);
             }
-            R.src.push_back(tb[k][1]);
-            R.src2.push_back(tb[k][2]);
-        }
-        if (!tb.empty()) R.end.push_back(ListEnd(R.src.size()));
+            R.end.push_back(ListEnd(R.src.size()));
+        });
     };
-    if (!build_rows(n, F.t_ptr, F.t_col, F.t_pair_ptr, F.t_pa, &F.t_pb, max_list, [&](int i, RowPart &R) {
-        thread_local Triples tb;
-        tb.clear();
-        for (int k = F.row_ptr[i]; k < F.row_ptr[i + 1]; ++k) {
-            const int j = F.col[k];
-            for (int q = F.p_ptr[j]; q < F.p_ptr[j + 1]; ++q) tb.push_back({F.p_col[q], k, q});
-        }
-        emit(tb, R);
+    if (!build_rows(n, F.t_ptr, F.t_col, F.t_pair_ptr, F.t_pa, &F.t_pb, max_list, [&]() {
+        return [&, row = ByColumn<Pair>(C.n)](int i, RowPart &R) mutable {
+            row.start();
+            for (int k = F.row_ptr[i]; k < F.row_ptr[i + 1]; ++k) {
+                const int j = F.col[k];
+                for (int q = F.p_ptr[j]; q < F.p_ptr[j + 1]; ++q) row.put(F.p_col[q], {k, q});
+            }
+            emit(row, R);
+        };
     })) return false;
     C.sa_in = true;
-    if (!build_rows(C.n, C.row_ptr, C.col, C.src_ptr, C.src, &C.src2, max_list, [&](int I, RowPart &R) {
-        thread_local Triples tb;
-        tb.clear();
-        for (int e = F.pt_ptr[I]; e < F.pt_ptr[I + 1]; ++e) {
-            const int i = F.pt_col[e], q = F.pt_map[e];
-            for (int t = F.t_ptr[i]; t < F.t_ptr[i + 1]; ++t) tb.push_back({F.t_col[t], q, t});
-        }
-        emit(tb, R);
+    if (!build_rows(C.n, C.row_ptr, C.col, C.src_ptr, C.src, &C.src2, max_list, [&]() {
+        return [&, row = ByColumn<Pair>(C.n)](int I, RowPart &R) mutable {
+            row.start();
+            for (int e = F.pt_ptr[I]; e < F.pt_ptr[I + 1]; ++e) {
+                const int i = F.pt_col[e], q = F.pt_map[e];
+                for (int t = F.t_ptr[i]; t < F.t_ptr[i + 1]; ++t) row.put(F.t_col[t], {q, t});
+            }
+            emit(row, R);
+        };
     })) return false;
     find_diagonal(C);
     return true;
@@ -545,7 +433,7 @@ std::string build_amg(AmgHierarchy &H, const Topology &T, const std::vector<int>
         children(L1, T.nfp);
         // A_1 = P' (A P): each entry sums the A P slots of its row's faces
         // (about 7 per face row) instead of the face matrix's entries (11)
-        if (!build_ap(H.ap, T, L1.agg, L1.agg2, max_list)) return kTooLong;
+        if (!build_ap(H.ap, T, L1.n, L1.agg, L1.agg2, max_list)) return kTooLong;
         const ApPattern &ap = H.ap;
         const bool fits = galerkin_pattern<true>(L1, max_list, [&](int child, auto emit) {
             const bool half = child < 0;
