@@ -2,6 +2,7 @@
 #include "mhs_ebe.h"
 
 #include "mhs_kernels.h"
+#include "mhs_lists.h"
 
 #include <algorithm>
 #include <numeric>
@@ -52,54 +53,77 @@ std::string ebe_ap_lists(const EbeLayout &E, const Topology &T, const ApPattern 
                          size_t max_list) {
     const long long slots = (long long)ap.col.size();
     if (slots >= 0x7fffffffLL || E.nval >= 0x7fffffffLL) return "too many values for 32-bit lists";
-    // slot of (row f, aggregate J): the row's slots are few (about 7)
-    auto slot_of = [&](int f, int J) -> long long {
-        const int sl = f / kSlice;
-        const long long base = ap.slice_ptr[sl] + f % kSlice;
-        const int w = int((ap.slice_ptr[sl + 1] - ap.slice_ptr[sl]) / kSlice);
-        for (int e = 0; e < w; ++e) {
-            const long long q = base + (long long)e * kSlice;
-            if (ap.col[q] == J && ap.src_ptr[q + 1] > ap.src_ptr[q]) return q;
-        }
-        return -1;
+    // row by row (each row's slots depend on its own cells, in ascending order),
+    // the lists in slot order
+    const int ns = T.nslices, nt = ranges(ns, 32);
+    struct Part {
+        std::vector<int> src;
+        std::vector<ListEnd> end;
+        bool outside = false;
     };
-    ptr.assign(slots + 1, 0);
-    // two passes: counts, then the lists in slot order
-    for (int pass = 0; pass < 2; ++pass) {
-        std::vector<ListEnd> fill;
-        if (pass == 1) {
-            size_t n = 0;
-            for (long long q = 0; q < slots; ++q) n += ptr[q + 1];
-            if (n > std::min(max_list, kMaxList)) return "too many entries for 32-bit lists";
-            for (long long q = 0; q < slots; ++q) ptr[q + 1] += ptr[q];
-            src.assign(n, 0);
-            fill.assign(ptr.begin(), ptr.end() - 1);
-        }
-        for (int c = 0; c < T.nc; ++c) {
-            const int s = E.cell_seg[c], l = E.cell_local[c];
-            const int f0 = T.facepos[c], n = T.facepos[c + 1] - f0, np = n * (n + 1) / 2;
-            for (int i = 0; i < n; ++i) {
-                const int f = T.hf_dof[f0 + i];
+    std::vector<Part> parts(nt);
+    in_ranges(ns, nt, [&](int t, int b, int e) {
+        Part &Q = parts[t];
+        std::vector<std::pair<int, int>> in;   // (slot of the slice, position)
+        std::vector<int> J, end;
+        for (int sl = b; sl < e; ++sl) {
+            const long long base = ap.slice_ptr[sl];
+            const int w = int((ap.slice_ptr[sl + 1] - base) / kSlice);
+            in.clear();
+            end.assign((size_t)w * kSlice + 1, 0);
+            for (int l = 0; l < kSlice; ++l) {
+                const int f = sl * kSlice + l;
                 if (agg[f] < 0) continue;
-                for (int j = 0; j < n; ++j) {
-                    const int rj = T.hf_dof[f0 + j];
-                    const bool half = agg2[rj] >= 0;
-                    for (int J : {agg[rj], agg2[rj]}) {
-                        if (J < 0) continue;
-                        const long long q = slot_of(f, J);
-                        if (q < 0) return "a cell entry outside the A P pattern";
-                        if (pass == 0) {
-                            ++ptr[q + 1];
-                        } else {
-                            const int pq = i <= j ? pidx(i, j, n) : pidx(j, i, n);
-                            const int v = int(E.seg_val[s] + ebe_slot(l, pq, np));
-                            src[fill[q]++] = half ? ~v : v;
+                // the row's aggregates (about 7; padding slots list nothing)
+                J.clear();
+                for (int q = 0; q < w; ++q) {
+                    const long long at = base + l + (long long)q * kSlice;
+                    if (ap.src_ptr[at + 1] > ap.src_ptr[at]) J.push_back(ap.col[at]);
+                }
+                for (int r = 0; r < 2; ++r) {
+                    const int c = T.row_cell[2 * (size_t)f + r];
+                    if (c < 0) continue;
+                    const int f0 = T.facepos[c], n = T.facepos[c + 1] - f0, np = n * (n + 1) / 2;
+                    const int i = T.row_loc[2 * (size_t)f + r], s = E.cell_seg[c], loc = E.cell_local[c];
+                    for (int j = 0; j < n; ++j) {
+                        const int rj = T.hf_dof[f0 + j];
+                        const int v = int(E.seg_val[s] + ebe_slot(loc, i <= j ? pidx(i, j, n) : pidx(j, i, n), np));
+                        for (int a : {agg[rj], agg2[rj]}) {
+                            if (a < 0) continue;
+                            const auto at = std::find(J.begin(), J.end(), a);
+                            if (at == J.end()) {
+                                Q.outside = true;
+                                continue;
+                            }
+                            const int q = int(at - J.begin()) * kSlice + l;
+                            in.emplace_back(q, agg2[rj] >= 0 ? ~v : v);
+                            ++end[q + 1];
                         }
                     }
                 }
             }
+            const size_t s0 = Q.src.size();
+            for (int q = 0; q < w * kSlice; ++q) end[q + 1] += end[q];
+            Q.src.resize(s0 + in.size());
+            for (const auto &x : in) Q.src[s0 + end[x.first]++] = x.second;
+            // (each end has moved to where the next slot starts)
+            for (int q = 0; q < w * kSlice; ++q) Q.end.push_back(ListEnd(s0 + end[q]));
         }
+    });
+    std::vector<std::vector<int>> srcs(nt);
+    std::vector<std::vector<ListEnd>> ends(nt);
+    for (int t = 0; t < nt; ++t) {
+        if (parts[t].outside) return "a cell entry outside the A P pattern";
+        srcs[t].swap(parts[t].src);
+        ends[t].swap(parts[t].end);
     }
+    if (too_long(0, total(srcs), max_list)) return "too many entries for 32-bit lists";
+    src.clear();
+    const std::vector<size_t> at = append(src, srcs);
+    for (int t = 0; t < nt; ++t)
+        for (ListEnd &e : ends[t]) e += ListEnd(at[t]);
+    ptr.assign(1, 0);
+    append(ptr, ends);
     return "";
 }
 
