@@ -1,6 +1,7 @@
 """Host-side gather lists of the multigrid set-up: what their 32-bit ends can
 hold is checked on the lists themselves (a face between two blocks is in both
-blocks' lists, so they are longer than the face matrix); and the LDS limit of the
+blocks' lists, so they are longer than the face matrix); the lists are the same on one
+host thread as on several; and the LDS limit of the
 one-workgroup tail, which every handle sets on its own device."""
 import os
 import subprocess
@@ -43,6 +44,14 @@ def test_lists_past_the_limit_are_refused(checker, strength, dims):
     assert "too large" in checker(strength, dims, limit=n - 1)["amg"]
     assert checker(strength, dims, element_limit=m)["hash"] == ok["hash"]
     assert "too many entries" in checker(strength, dims, element_limit=m - 1)["element"]
+
+
+@pytest.mark.parametrize("strength", STRENGTHS)
+@pytest.mark.parametrize("dims", [(40, 36, 30), (30, 20, 25, 41, 19, 22)])
+def test_one_host_thread_and_several_build_the_same_lists(checker, strength, dims):
+    one, many = checker(strength, dims, threads=1), checker(strength, dims, threads=8)
+    assert int(one["asked"]) > 0 and int(many["asked"]) > 0   # the program's answer was the one used
+    assert one["hash"] == many["hash"]
 
 
 def test_tail_lds_limit_is_set_for_every_handle(pkg, tmp_path):
