@@ -1198,7 +1198,7 @@ int autotune(mhs_solver *s, int nrhs, bool mixed, bool amg, bool choose_ebe, dou
             s->dT.sweep_tb = best.sweep_tb;
             s->dT.sweep_xcd = best.sweep_xcd;
             float bt = 1e30f;
-            for (int rows : {0, 128, 512, 2048, 8192, 32768}) {
+            for (int rows : tail_candidates(s->dA, nrhs, mixed ? sizeof(float) : sizeof(double))) {
                 s->dT.tail_rows = rows;
                 const float ms = time_it([&]() {
                     return mixed ? launch_vcycle<float>(s->stream, s->dT, s->dA, s->ftype, nrhs, s->val32, s->dinv32, s->r32,

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <vector>
 
 namespace mhs {
 
@@ -269,6 +270,11 @@ hipError_t launch_resnorm(hipStream_t st, const DevTopo &T, int nrhs, const doub
 // LDS that the one-workgroup tail may take on the current device: kTailBytes, or
 // what a launch may take without asking where asking is refused.
 int tail_lds_limit();
+// First level of the one-workgroup tail for that many rows, nrhs right-hand sides
+// and vsize-byte values: as far as the levels fit in LDS.
+int tail_level(const DevAmg &A, int tail_rows, int nrhs, int vsize);
+// Row limits that the autotuner times, one for each first level there is to choose.
+std::vector<int> tail_candidates(const DevAmg &A, int nrhs, int vsize);
 
 // Multigrid: per-solve set-up (Galerkin products, diagonals, coarsest inverses)
 // and the preconditioned iteration pieces.

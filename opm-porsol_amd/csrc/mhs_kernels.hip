@@ -3751,17 +3751,24 @@ static void sweep0(hipStream_t st, const DevTopo &T, const VT *val0, const VT *d
 
 // LDS of a tail that starts at level lt: indices, then values, then vectors.
 static inline int tail_vbase(const DevAmg &A, int lt) { return 2 * A.tail_iend[lt]; }
-template <typename VT>
-static inline int tail_xbase(const DevAmg &A, int lt) {
-    return tail_vbase(A, lt) + A.tail_vend[lt] * (int)sizeof(VT);
+static inline int tail_xbase(const DevAmg &A, int lt, int vsize) {
+    return tail_vbase(A, lt) + A.tail_vend[lt] * vsize;
 }
-template <typename VT, int NR>
-static inline long long tail_bytes(const DevAmg &A, int lt) {
-    return tail_xbase<VT>(A, lt) + (long long)A.tail_vec[lt] * NR * (int)sizeof(VT);
+static inline long long tail_bytes(const DevAmg &A, int lt, int nrhs, int vsize) {
+    return tail_xbase(A, lt, vsize) + (long long)A.tail_vec[lt] * nrhs * vsize;
 }
-template <typename VT, int NR>
-static inline bool tail_fits(const DevAmg &A, int lt) {
-    return lt >= A.tail_first && tail_bytes<VT, NR>(A, lt) <= A.tail_lds;
+int tail_level(const DevAmg &A, int tail_rows, int nrhs, int vsize) {
+    int lt = A.nlev - 1;
+    while (lt > 1 && A.max_rows[lt - 1] <= tail_rows && lt - 1 >= A.tail_first &&
+           tail_bytes(A, lt - 1, nrhs, vsize) <= A.tail_lds)
+        --lt;
+    return lt;
+}
+std::vector<int> tail_candidates(const DevAmg &A, int nrhs, int vsize) {
+    std::vector<int> rows;
+    for (int r : {0, 128, 512, 2048, 8192, 32768})
+        if (rows.empty() || tail_level(A, r, nrhs, vsize) != tail_level(A, rows.back(), nrhs, vsize)) rows.push_back(r);
+    return rows;
 }
 // The attribute belongs to the kernels of the current device: every hierarchy
 // asks for it on its own.
@@ -3836,8 +3843,7 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
     }
     if (nu == 1) {
         // first level handled by the workgroup-per-instance tail kernel
-        int lt = L - 1;
-        while (lt > 1 && A.max_rows[lt - 1] <= T.tail_rows && tail_fits<VT, NR>(A, lt - 1)) --lt;
+        const int lt = tail_level(A, T.tail_rows, NR, sizeof(VT));
         const VT als = (VT)A.alpha_sa;
         for (int l = 1; l < lt; ++l) {
             const DevAmgLevel &F = A.lev[l];
@@ -3884,8 +3890,8 @@ static void vcycle_impl(hipStream_t st, const Gate &gt, const DevTopo &T, const 
         }
         const VT *tv;
         if constexpr (std::is_same<VT, float>::value) tv = A.tail_val32; else tv = A.tail_val64;
-        const int vbase = tail_vbase(A, lt), xbase = tail_xbase<VT>(A, lt);
-        k_vcycle_tail<VT, NR><<<A.ninst, 1024, (unsigned)tail_bytes<VT, NR>(A, lt), st>>>(
+        const int vbase = tail_vbase(A, lt), xbase = tail_xbase(A, lt, sizeof(VT));
+        k_vcycle_tail<VT, NR><<<A.ninst, 1024, (unsigned)tail_bytes(A, lt, NR, sizeof(VT)), st>>>(
             gt, A.tail_tab, A.tail_idx, tv, L, lt, vbase, xbase, (const VT *)A.lev[lt].b, (VT *)A.lev[lt].x, alw(0),
             (VT)A.alpha, lsa, als,
             A.lev[lt].agg, fuse[lt] ? (VT *)A.lev[lt - 1].x : nullptr);

@@ -11,6 +11,7 @@
 
 #include "mhs_amg.h"
 #include "mhs_ebe.h"
+#include "mhs_kernels.h"
 #include "mhs_structure.h"
 
 using namespace mhs;
@@ -73,5 +74,24 @@ int main(int argc, char **argv) {
     e = ebe_ap_lists(E, T, H.ap, H.lev[1].agg, H.lev[1].agg2, ptr, src, elimit ? elimit : kMaxList);
     mix(ptr); mix(src);
     std::printf("element %s\nelement_list %zu\nhash %llx\n", e.empty() ? "ok" : e.c_str(), src.size(), g_hash);
+    // what the autotuner would time: per right-hand sides and value size the first
+    // level of every candidate's tail
+    DevAmg A{};
+    A.nlev = H.nlev();
+    A.tail_first = H.tail.first;
+    A.tail_lds = kTailBytes;
+    for (int l = 0; l < A.nlev; ++l) {
+        A.tail_iend[l] = H.tail.iend[l];
+        A.tail_vend[l] = H.tail.vend[l];
+        A.tail_vec[l] = H.tail.vec[l];
+        for (size_t t = 0; l > 0 && t + 1 < H.lev[l].inst_ptr.size(); ++t)
+            A.max_rows[l] = std::max(A.max_rows[l], H.lev[l].inst_ptr[t + 1] - H.lev[l].inst_ptr[t]);
+    }
+    for (int vsize : {4, 8})
+        for (int nrhs : {1, 3}) {
+            std::printf("tail_%d_%d", vsize, nrhs);
+            for (int r : tail_candidates(A, nrhs, vsize)) std::printf(" %d", tail_level(A, r, nrhs, vsize));
+            std::printf(" | %d\n", tail_level(A, 32768, nrhs, vsize));
+        }
     return 0;
 }

@@ -9,6 +9,9 @@ import subprocess
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+HIP = ["-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROCM, "include")]
+HIP_LIBS = ["-L", os.path.join(ROCM, "lib"), "-lamdhip64", f"-Wl,-rpath,{os.path.join(ROCM, 'lib')}"]
 STRENGTHS = [("1", "1", "1"), ("1", "1", "0.1"), ("0.1", "0.1", "1")]   # blocks 2x2x2, 2x2x1, 1x1x2
 
 
@@ -16,9 +19,9 @@ STRENGTHS = [("1", "1", "1"), ("1", "1", "0.1"), ("0.1", "0.1", "1")]   # blocks
 def checker(pkg, tmp_path_factory):
     exe = str(tmp_path_factory.mktemp("amg") / "amg_lists_check")
     here = os.path.join(ROOT, "opm-porsol_amd")
-    cmd = ["g++", "-O1", "-std=c++17", "-Wall", "-pthread", "-I", os.path.join(here, "csrc"), "-I",
+    cmd = ["g++", "-O1", "-std=c++17", "-Wall", "-pthread", *HIP, "-I", os.path.join(here, "csrc"), "-I",
            os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "amg_lists_check.cpp"), "-o", exe, "-L", here,
-           "-lmhs", f"-Wl,-rpath,{here}"]
+           "-lmhs", f"-Wl,-rpath,{here}", *HIP_LIBS]
     res = subprocess.run(cmd, capture_output=True, text=True)
     assert res.returncode == 0, res.stdout + res.stderr
 
@@ -54,13 +57,21 @@ def test_one_host_thread_and_several_build_the_same_lists(checker, strength, dim
     assert one["hash"] == many["hash"]
 
 
+@pytest.mark.parametrize("dims", [(1, 1, 1), (9, 9, 9), (20, 20, 10), (40, 36, 30), (8, 8, 8, 26, 25, 24)])
+def test_autotuner_times_every_tail_once(checker, dims):
+    out = checker(STRENGTHS[0], dims)
+    for vsize in (4, 8):
+        for nrhs in (1, 3):
+            levels, last = out[f"tail_{vsize}_{nrhs}"].split("|")
+            levels = list(map(int, levels.split()))
+            assert levels == sorted(set(levels), reverse=True) and levels[-1] == int(last)
+
+
 def test_tail_lds_limit_is_set_for_every_handle(pkg, tmp_path):
     exe, here = str(tmp_path / "tail_limit_check"), os.path.join(ROOT, "opm-porsol_amd")
-    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
-    cmd = ["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(rocm, "include"), "-I",
-           os.path.join(here, "csrc"), "-I", os.path.join(ROOT, "include"),
+    cmd = ["g++", "-O1", "-std=c++17", *HIP, "-I", os.path.join(here, "csrc"), "-I", os.path.join(ROOT, "include"),
            os.path.join(ROOT, "tests", "tail_limit_check.cpp"), "-o", exe, "-L", here, "-lmhs", f"-Wl,-rpath,{here}",
-           "-L", os.path.join(rocm, "lib"), "-lamdhip64", f"-Wl,-rpath,{os.path.join(rocm, 'lib')}"]
+           *HIP_LIBS]
     res = subprocess.run(cmd, capture_output=True, text=True)
     assert res.returncode == 0, res.stdout + res.stderr
     out = [subprocess.run([exe, *a], capture_output=True, text=True, timeout=60) for a in ([], ["refuse"])]
