@@ -397,7 +397,7 @@ std::string build_amg(AmgHierarchy &H, const Topology &T, const std::vector<int>
     // pair's faces those of the two cells across it): linear pressures are
     // interpolated exactly from block means, so the coarse operator is not
     // too stiff across the blocks as it is with the owner's block alone
-    // (50 -> 34 iterations at 128x128x64).
+    // (51 -> 35 iterations at 128x128x64).
     {
         const std::array<int, 3> &b0 = H.blocks[0];
         AmgLevel L1;

@@ -154,8 +154,14 @@ __global__ __launch_bounds__(256) void k_finish(DevRed R, DevScal S, FinArgs A) 
 // wavefront per quantity, in the same order, so all of them find the same step.
 // One launch less, each about 4.3 us of waiting for a few dozen numbers (and the
 // gap to the next).  The reads of all workgroups grow with the square of the
-// partials: at 763 (80x80x40) a solve takes 6.74 ms with the launches and 6.57
-// without, at 3105 (128x128x64) they would read 230 MB, more than the launch costs.
+// partials: multigrid iterations with the launches / without (us, cubes of
+// 48^3 to 101^3 cells, one right-hand side and four):
+//   partials       331        745        1020       1519       2160       3049
+//   FP64, 1      120/114    165/160    197/194    261/260    344/346    452/458
+//   FP64, 4      195/176    283/274    391/379    544/539    736/761   1019/1074
+//   mixed, 1     109/104    138/134    161/157    204/202    268/272    330/341
+//   mixed, 4     169/144    233/211    275/256    380/363    513/509    653/672
+// It pays up to about 2000 whatever the precision and the right-hand sides.
 constexpr int kFuseParts = 1024;
 template <int NQ>
 __device__ __forceinline__ void inst_totals(const DevRed &R, int s, int nq, double (&tot)[NQ]) {

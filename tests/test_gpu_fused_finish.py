@@ -43,8 +43,9 @@ def test_small_instance_alone_and_beside_a_large_one(pkg, orc, solver, nrhs, pre
 @pytest.mark.parametrize("solver", [0, 1])
 @pytest.mark.parametrize("n", [55, 56, 69])
 def test_more_partials_than_one_round_of_loads(pkg, solver, precision, n):
-    """Around 512 and just below 1024 partials (rows of 1024 faces), each summed
-    eight loads at a time; a uniform medium has the closed form v = k dp / L."""
+    """Around 512 and just below 1024 partials of the assembled operator (rows of 1024
+    faces), each summed eight loads at a time; a uniform medium has the closed form
+    v = k dp / L."""
     g = pkg.grids.cartesian(n, n, n)
     nc = g.num_cells
     bt, bv = cases.xdrop_bc(g, 1.0, 0.0)
@@ -56,4 +57,25 @@ def test_more_partials_than_one_round_of_loads(pkg, solver, precision, n):
     exact[g.side == 1], exact[g.side == 0] = 1.0 / n, -1.0 / n
     v = np.asarray(s.getSolution()[2]).reshape(-1)
     # solves to 1e-12 of a system with a condition number of about n^2 < 5e3
+    assert np.max(np.abs(v - exact)[(g.side == 0) | (g.side == 1)]) < 1e-8
+
+
+@pytest.mark.parametrize("solver", [0, 1])
+@pytest.mark.parametrize("element_operator,n", [(0, 70), (0, 71), (2, 63), (2, 64), (2, 65)])
+def test_both_sides_of_the_limit_in_mixed_precision(pkg, element_operator, n, solver):
+    """Just below and above 1024 partials of each operator: one per 1024 face rows
+    (1020 and 1064), or one per 256 cells of a colour (978, 1024 and 1074)."""
+    g = pkg.grids.cartesian(n, n, n)
+    nc = g.num_cells
+    bt, bv = cases.xdrop_bc(g, 1.0, 0.0)
+    s = pkg.HybridSolver(0)
+    s.init(g, pkg.fields.diag_perm(np.ones(nc), np.ones(nc), np.ones(nc)), (0, 0, 0), bt, None)
+    tm, rm = cases.unit_fluid(nc)
+    s.solve(tm, rm, np.zeros(nc), bt, bv, residual_tolerance=1e-12, precision="mixed", linsolver_type=solver,
+            element_operator=element_operator)
+    assert s.report.element_operator == (1 if element_operator else 0)
+    exact = np.zeros(g.num_half_faces)
+    exact[g.side == 1], exact[g.side == 0] = 1.0 / n, -1.0 / n
+    v = np.asarray(s.getSolution()[2]).reshape(-1)
+    # solves to 1e-12 of a system with a condition number of about n^2 < 6e3
     assert np.max(np.abs(v - exact)[(g.side == 0) | (g.side == 1)]) < 1e-8
