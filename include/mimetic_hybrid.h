@@ -66,7 +66,9 @@ enum mhs_precision {
 };
 
 typedef struct {
-    double tol;                /* residual_tolerance (:662): ||r||/||r0|| bound */
+    double tol;                /* residual_tolerance (:662): ||r||/||r0|| bound; r0 of the start,
+                                  zero for linsolver_type 0 and the Dirichlet values for the
+                                  others (:1521-1532), whatever precond is */
     int maxit;                 /* linsolver_maxit (:666); 0 -> number of unknowns */
     int linsolver_type;        /* (:664) 0: Jacobi-PCG, standing in for SeqILU0-CG
                                   (:1387-1420); it needs more iterations than ILU0,
