@@ -893,8 +893,12 @@ int ensure_solve_buffers(mhs_solver *s, int nrhs, bool mixed) {
         if (ok()) s->dE.val32 = dalloc<float>(s, L, (size_t)s->EL.nval, &e);
         if (ok()) s->dE.R.partials = dalloc<double>(s, L, (size_t)s->EL.nslots * 16, &e);
         // padding rows are never written by the element-by-element passes:
-        // their q and multigrid residual stay zero, like their p and r
+        // their q and multigrid residual stay zero, like their p and r.  p and r
+        // too from the start: the autotuner's products on the assembled matrix
+        // take them into q before a solve has written them
         if (ok()) e = hipMemset(s->q32, 0, nv * sizeof(float));
+        if (ok()) e = hipMemset(s->p32, 0, nv * sizeof(float));
+        if (ok()) e = hipMemset(s->r32, 0, nv * sizeof(float));
         if (ok() && s->has_amg) e = hipMemset(s->dA.res0, 0, nv * sizeof(float));
     }
     if (ok()) e = hipMemset(s->R.counters, 0, sizeof(int) * T.ninst);
