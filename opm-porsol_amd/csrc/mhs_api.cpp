@@ -903,6 +903,8 @@ int ensure_solve_buffers(mhs_solver *s, int nrhs, bool mixed) {
     }
     if (ok()) e = hipMemset(s->R.counters, 0, sizeof(int) * T.ninst);
     if (ok()) e = hipMemset(s->x64, 0, nv * sizeof(double));
+    // the solver's stream does not wait for the default stream that these ran on
+    if (ok()) e = hipStreamSynchronize(nullptr);
     if (ok()) e = hipHostMalloc(reinterpret_cast<void **>(&s->h_sc), state_bytes(nsys), 0);
     if (ok()) {
         s->h_act = reinterpret_cast<int *>(reinterpret_cast<unsigned char *>(s->h_sc) +
