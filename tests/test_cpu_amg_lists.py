@@ -1,8 +1,9 @@
 """Host-side gather lists of the multigrid set-up: what their 32-bit ends can
 hold is checked on the lists themselves (a face between two blocks is in both
-blocks' lists, so they are longer than the face matrix); the lists are the same on one
-host thread as on several; and the LDS limit of the
-one-workgroup tail, which every handle sets on its own device."""
+blocks' lists, so they are longer than the face matrix), they are the same on
+one host thread as on several, and the autotuner times each tail that they
+allow once; and the LDS limit of the one-workgroup tail, which every handle
+sets on its own device."""
 import os
 import subprocess
 
@@ -16,7 +17,7 @@ STRENGTHS = [("1", "1", "1"), ("1", "1", "0.1"), ("0.1", "0.1", "1")]   # blocks
 
 
 @pytest.fixture(scope="module")
-def checker(pkg, tmp_path_factory):
+def lists(pkg, tmp_path_factory):
     exe = str(tmp_path_factory.mktemp("amg") / "amg_lists_check")
     here = os.path.join(ROOT, "opm-porsol_amd")
     cmd = ["g++", "-O1", "-std=c++17", "-Wall", "-pthread", *HIP, "-I", os.path.join(here, "csrc"), "-I",
@@ -36,30 +37,30 @@ def checker(pkg, tmp_path_factory):
 
 @pytest.mark.parametrize("strength", STRENGTHS)
 @pytest.mark.parametrize("dims", [(12, 11, 9), (8, 8, 8, 5, 4, 7)])
-def test_lists_past_the_limit_are_refused(checker, strength, dims):
-    ok = checker(strength, dims)
+def test_lists_past_the_limit_are_refused(lists, strength, dims):
+    ok = lists(strength, dims)
     assert ok["amg"] == ok["element"] == "ok"
     # longer than the face matrix that used to bound them, by less than the ends' extra bit
     assert int(ok["matrix"]) < int(ok["ap"]) <= 2 * int(ok["matrix"])
     assert int(ok["longest"]) <= 2 * int(ok["matrix"])
     n, m = int(ok["longest"]), int(ok["element_list"])
-    assert checker(strength, dims, limit=n)["hash"] == ok["hash"]
-    assert "too large" in checker(strength, dims, limit=n - 1)["amg"]
-    assert checker(strength, dims, element_limit=m)["hash"] == ok["hash"]
-    assert "too many entries" in checker(strength, dims, element_limit=m - 1)["element"]
+    assert lists(strength, dims, limit=n)["hash"] == ok["hash"]
+    assert "too large" in lists(strength, dims, limit=n - 1)["amg"]
+    assert lists(strength, dims, element_limit=m)["hash"] == ok["hash"]
+    assert "too many entries" in lists(strength, dims, element_limit=m - 1)["element"]
 
 
 @pytest.mark.parametrize("strength", STRENGTHS)
 @pytest.mark.parametrize("dims", [(40, 36, 30), (30, 20, 25, 41, 19, 22)])
-def test_one_host_thread_and_several_build_the_same_lists(checker, strength, dims):
-    one, many = checker(strength, dims, threads=1), checker(strength, dims, threads=8)
+def test_one_host_thread_and_several_build_the_same_lists(lists, strength, dims):
+    one, many = lists(strength, dims, threads=1), lists(strength, dims, threads=8)
     assert int(one["asked"]) > 0 and int(many["asked"]) > 0   # the program's answer was the one used
     assert one["hash"] == many["hash"]
 
 
 @pytest.mark.parametrize("dims", [(1, 1, 1), (9, 9, 9), (20, 20, 10), (40, 36, 30), (8, 8, 8, 26, 25, 24)])
-def test_autotuner_times_every_tail_once(checker, dims):
-    out = checker(STRENGTHS[0], dims)
+def test_autotuner_times_every_tail_once(lists, dims):
+    out = lists(STRENGTHS[0], dims)
     for vsize in (4, 8):
         for nrhs in (1, 3):
             levels, last = out[f"tail_{vsize}_{nrhs}"].split("|")
